@@ -76,6 +76,10 @@ struct LegArgs {
     void *out0, *out1;      // spectral outputs (analysis)
     long long spec_fstride; // complex elements per field in spectral arrays
     double2 *F0, *F1;       // Fourier workspace [field][im][nlat]
+    int nf;                 // fields (field-group kernels)
+    const int4 *seglist;    // field-group analysis: [nlist] (global segment or -1, order, segment of the
+                            // order, coff), entry i for XCD i mod 8
+    int nlist;
     int gx, gy, gz;         // work items form a (gx, gy, gz = nfields) box, x fastest
     int xcd;                // synthesis: 1 keeps the pair blocks of an order on one XCD
     int nm_run;             // synthesis: only orders im < nm_run (0: all)
@@ -231,6 +235,8 @@ struct shtk_plan {
     double *oz_asc = nullptr;
     int4 *oz_run = nullptr;  // analysis work runs: (order, first segment, segments, 0)
     int oz_nrun = 0, oz_run_len = 8;
+    int4 *seglist = nullptr;  // segments dealt to the XCDs by order (LegArgs.seglist), inside segm's array
+    int nlist = 0;
     size_t qc_len = 0;
     int oz_ch_total = 0;
     void *oz_ws = nullptr;
@@ -408,6 +414,9 @@ hipError_t launch_f32_anal(const OzArgs &a, hipStream_t st);
 hipError_t launch_seed(const SeedArgs &a, hipStream_t st);
 hipError_t launch_leg_synth(const LegArgs &a, int nfields, int vector, int chains, hipStream_t st);
 hipError_t launch_leg_anal(const LegArgs &a, int nfields, int vector, hipStream_t st);
+// FP64 kernels of field groups (shtk_fields.hip).
+int fields_anal_count(const LegArgs &a, int nfields);  // leading fields it takes (0: none)
+hipError_t launch_fields_anal(const LegArgs &a, int nfields, hipStream_t st);
 hipError_t launch_fft(const FftArgs &a, int nfields, int inverse, hipStream_t st);
 hipError_t launch_spec_scale(const void *in, void *out, int in_f32, int out_f32, const double *scale, int divide,
                              int lmax, int mmax, int mres, long long nelem_per_field, int nfields,

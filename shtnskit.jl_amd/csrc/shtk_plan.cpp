@@ -449,6 +449,8 @@ shtk::LegArgs base_args(const shtk_plan *p, int ltr) {
     a.segbase = p->segbase;
     a.segm = p->segm;
     a.nseg_total = p->nseg_total;
+    a.seglist = p->seglist;
+    a.nlist = p->nlist;
     a.seedq0 = p->seedq0;
     a.seedq1 = p->seedq1;
     a.seedk = p->seedk;
@@ -1031,9 +1033,18 @@ int run_to_spec(shtk_plan *p, const Job &j, const void *g0, const void *g1, void
     }
     const int pblk = j.vector ? p->vanal_pblk : 512;  // pairs per analysis work item (launch_leg_anal)
     a.apblk = pblk;
+    // scalar batches: groups of fields share the recurrence (shtk_fields.hip); the
+    // fields left over take the single-field kernel below
+    const int ngrp = j.vector ? 0 : shtk::fields_anal_count(a, nf), nrest = nf - ngrp;
+    if (ngrp > 0) {
+        HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_fields_anal(a, ngrp, st); }),
+                "Legendre analysis launch");
+        a.F0 += (size_t)ngrp * p->nm * p->d.nlat;
+        a.out0 = (char *)a.out0 + (size_t)ngrp * a.spec_fstride * (a.io_f32 ? 8 : 16);
+    }
     a.atomic = p->np > pblk;
-    if (a.atomic) {
-        const size_t bytes = (size_t)nf * a.spec_fstride * (a.io_f32 ? 8 : 16);
+    if (a.atomic && nrest > 0) {
+        const size_t bytes = (size_t)nrest * a.spec_fstride * (a.io_f32 ? 8 : 16);
         void *outs[2] = {a.out0, a.out1};
         for (int q = 0; q <= j.vector; ++q)
             HIP_TRY(shtk::launch_zero(outs[q], bytes, st), "output clear");
@@ -1059,8 +1070,8 @@ int run_to_spec(shtk_plan *p, const Job &j, const void *g0, const void *g1, void
         HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_leg_anal(a, nf, 1, st); }),
                 "Legendre analysis launch");
         HIP_TRY(side.join(), "order-0 rows join");
-    } else {
-        HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_leg_anal(a, nf, j.vector, st); }),
+    } else if (nrest > 0) {
+        HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_leg_anal(a, nrest, j.vector, st); }),
                 "Legendre analysis launch");
     }
     if (j.pole_fix && p->poles && p->d.mres == 1 && p->d.mmax >= 1)
@@ -1696,6 +1707,26 @@ static int plan_tables(shtk_plan *p) {
         }
     }
     p->nseg_total = nseg_total;
+    // segments for the field-group analysis, order im on XCD im mod 8: behind segm in
+    // one array (LegArgs.seglist)
+    const size_t segm_len = (segm.size() + 3) / 4 * 4;
+    {
+        std::vector<int> per[shtk::kXcds];
+        for (int gs = 0; gs < nseg_total; ++gs) per[segm[gs] % shtk::kXcds].push_back(gs);
+        size_t most = 0;
+        for (auto &v : per) most = std::max(most, v.size());
+        p->nlist = (int)(most * shtk::kXcds);
+        segm.resize(segm_len + 4 * (size_t)p->nlist, -1);
+        for (int x = 0; x < shtk::kXcds; ++x)
+            for (size_t k = 0; k < per[x].size(); ++k) {
+                const int gs = per[x][k], im = segm[gs];
+                int *e = &segm[segm_len + 4 * (k * shtk::kXcds + x)];
+                e[0] = gs;
+                e[1] = im;
+                e[2] = gs - segbase[im];
+                e[3] = (int)coff[im];
+            }
+    }
 
     // Sectoral seeds P_m^m(x_p) = (-1)^m sqrt(1/4pi) prod_k sqrt((2k+1)/(2k)) sin(theta)
     // (src/legendre.jl:252-271), carried as mantissa * 2^e (exact rescaling) and
@@ -1801,6 +1832,7 @@ static int plan_tables(shtk_plan *p) {
     p->hcoff = coff;
     RC_TRY(upload(&p->segbase, segbase, "plan tables"));
     RC_TRY(upload(&p->segm, segm, "plan tables"));
+    p->seglist = (int4 *)(p->segm + segm_len);
     RC_TRY(upload(&p->convscale, conv, "plan tables"));
     RC_TRY(upload(&p->tw, tw, "plan tables"));
     RC_TRY(upload(&p->chirp, chirp, "plan tables"));

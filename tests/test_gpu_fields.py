@@ -1,0 +1,69 @@
+"""Field-group Legendre kernels (batches whose fields share one recurrence)
+against the oracle, at the edges of their tiles: group remainders, orders that
+end inside a 32-degree chunk, pair counts around 64, odd latitude counts,
+orders between multiples of mres, truncation, scaled polar chains, and outputs
+handed over full of NaN.  FP64 throughout, so the bound is the FP64 path's
+(1e-12 relative L2 per field; 1e-6 where the arrays are FP32)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from _util import rel_l2, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+SHAPES = [
+    # lmax, nlat, nlon, mres, ltr, nf
+    (3, 4, 8, 1, -1, 4),
+    (31, 33, 64, 1, -1, 5),
+    (63, 64, 128, 1, -1, 8),
+    (64, 127, 130, 1, 50, 9),      # one field left over, odd nlat
+    (97, 130, 200, 3, 80, 12),
+    (130, 257, 264, 2, -1, 15),
+    (255, 259, 512, 1, 201, 10),
+    (700, 702, 1404, 9, -1, 6),    # scaled polar chains
+]
+
+
+def _worst(got, ref):
+    return max(rel_l2(got[..., k], ref[..., k]) for k in range(ref.shape[-1]))
+
+
+def _nan_spec(cfg, nf):
+    t = torch.full((nf, cfg.mmax + 1, cfg.lmax + 1), complex(float("nan"), float("nan")),
+                   dtype=torch.complex128, device="cuda:0")
+    return t.permute(2, 1, 0)
+
+
+@pytest.mark.parametrize("lmax,nlat,nlon,mres,ltr,nf", SHAPES)
+def test_batch_analysis_matches_oracle(shtk, oracle, cuda, lmax, nlat, nlon, mres, ltr, nf):
+    from shtnskit_jl_amd import _lib
+    from shtnskit_jl_amd.transforms import _ptr, _stream
+
+    cfg = shtk.create_gauss_config(lmax, nlat, nlon=nlon, mres=mres)
+    ocfg = oracle.Config(lmax, nlat, nlon=nlon, mres=mres)
+    f = np.asfortranarray(np.random.default_rng(lmax).standard_normal((nlat, nlon, nf)))
+    fd, out = to_dev(f), _nan_spec(cfg, nf)
+    print(f"analysis lmax={lmax} nlat={nlat} mres={mres} ltr={ltr} nf={nf}", flush=True)
+    _lib.check(_lib.load().shtk_analysis(ctypes.c_void_p(cfg.plan), _ptr(fd), _ptr(out), nf, _lib.SHTK_F64, ltr,
+                                         _stream(fd.device)), "analysis")
+    got, ref = to_host(out), ocfg.analysis(f, ltr=ltr)
+    assert _worst(got, ref) < TOL
+    assert np.all(got[ref == 0] == 0)
+
+
+@pytest.mark.parametrize("lmax,nlat,nlon,mres,ltr,nf", SHAPES[1:5])
+def test_batch_adjoint_synthesis_matches_oracle(shtk, oracle, cuda, lmax, nlat, nlon, mres, ltr, nf):
+    cfg = shtk.create_gauss_config(lmax, nlat, nlon=nlon, mres=mres)
+    ocfg = oracle.Config(lmax, nlat, nlon=nlon, mres=mres)
+    f = np.asfortranarray(np.random.default_rng(lmax + 1).standard_normal((nlat, nlon, nf)))
+    print(f"adjoint synthesis lmax={lmax} nlat={nlat} mres={mres} nf={nf}", flush=True)
+    assert _worst(to_host(shtk._adjoint_synthesis(cfg, to_dev(f))), ocfg.adjoint_synthesis(f)) < TOL
+    f32 = f.astype(np.float32)
+    got = to_host(shtk._adjoint_synthesis(cfg, to_dev(f32)))
+    assert got.dtype == np.complex64
+    assert _worst(got, ocfg.adjoint_synthesis(f32.astype(np.float64))) < 1e-6
