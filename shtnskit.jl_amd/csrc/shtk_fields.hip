@@ -246,6 +246,198 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// Synthesis of field groups.  One wavefront per (order, 64 latitude pairs, group
+// of NG fields) runs the order's recurrence once, from the seeds of its first
+// live segment to the last degree, and adds every degree to the NG fields' sums
+// (even and odd degrees, re and im: 4 NG accumulators per lane).  The operands of
+// 16 degrees, beta_{l+1} and c_l a_l of every field, sit in VGPRs, lane n of each
+// 16-lane row holding degree n, and reach the FMAs by DPP broadcast as in
+// k_synth_d; the next 16 degrees are loaded meanwhile.  Per degree and pair: one
+// multiply, one FMA and 2 NG FMAs.
+// NW waves per block take equal runs of the order's live segments, each from its own
+// seeds, and add their sums through LDS.
+//
+// Bound: FP64 issue (VALU 91 % of the busy cycles for 16 fields at lmax 1023, where
+// the chip runs at 2.0 GHz).  16 fields at lmax 1023: 815 us (k_synth_d) -> 435; 3
+// fields: 192 -> 105; 16 at 511: 124 -> 63; 37 at 255: 40 -> 29; 5 at 340: 30 -> 19.
+// ---------------------------------------------------------------------------
+template <int NG>
+struct SFRec {
+    double b, c;      // beta_{l+1}, c_l
+    double2 v[NG];    // a_l of the fields
+};
+
+// Degrees N .. 15 of a record group.
+template <int NG, bool FAST, int N>
+__device__ __forceinline__ void sf_steps(const SFRec<NG> &r, double x, double cm, double &prev, double &cur,
+                                         double (*acc)[NG][2]) {
+    if constexpr (N < 16) {
+        double t = x * cur;
+        const double u = FAST ? cur : cur * cm;
+#pragma unroll
+        for (int f = 0; f < NG; ++f) {
+            SHTK_FMAC_BC(acc[N & 1][f][0], r.v[f].x, u, N, "");
+            SHTK_FMAC_BC(acc[N & 1][f][1], r.v[f].y, u, N, "");
+        }
+        SHTK_FMAC_BC(t, r.b, prev, N, "-");
+        prev = cur;
+        cur = t;
+        sf_steps<NG, FAST, N + 1>(r, x, cm, prev, cur, acc);
+    }
+}
+
+template <int NG, int NW>
+__global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const LegArgs a) {
+    __shared__ double red[NW > 1 ? NW - 1 : 1][NW > 1 ? 4 * NG : 1][64];
+    // units lowest order first for every pair block and group: the long columns start first
+    const int unit = blockIdx.x, b = unit % a.gx, fg = unit / a.gx % a.gz, im = unit / (a.gx * a.gz);
+    const int m = im * a.mres, np = a.np, lmax = a.lmax, ltr = a.ltr;
+    const int lane = threadIdx.x & 63;
+    const int w = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int f0 = fg * NG, nfl = min(NG, a.nf - f0);
+    const int p = b * 64 + lane, pc = min(p, np - 1), pb1 = min(b * 64 + 64, np);
+    const int segb = as_const(a.segbase)[im];
+    const long long co = as_const(a.coff)[im] - m;
+    double acc[2][NG][2];
+#pragma unroll
+    for (int f = 0; f < NG; ++f) acc[0][f][0] = acc[0][f][1] = acc[1][f][0] = acc[1][f][1] = 0.0;
+    // first segment with a live pair of this block
+    const int nseg = ltr >= m ? (ltr - m) / DSEG + 1 : 0;
+    int s0 = nseg;
+    for (int q = 0; q < nseg; q += 64) {
+        const unsigned long long live = __ballot(q + lane < nseg && pb1 > a.pfirst[segb + min(q + lane, nseg - 1)]);
+        if (live) {
+            s0 = q + __builtin_ctzll(live);
+            break;
+        }
+    }
+    s0 = __builtin_amdgcn_readfirstlane(s0);
+    const int sa = s0 + w * (nseg - s0) / NW, sb = s0 + (w + 1) * (nseg - s0) / NW;
+    if (sa < sb) {
+        const double x = a.x[pc];
+        const size_t q = (size_t)(segb + sa) * np + pc;
+        double prev = a.seedq0[q], cur = a.seedq1[q];
+        int kk = a.seedk[q];
+        const double *qb = a.qb + co + 1, *qc = a.qcc + co;  // padded past lmax
+        const cptr<double> qcm = as_const(a.qcc) + co;
+        const double2 *av = (const double2 *)a.in0 + (size_t)f0 * a.spec_fstride + (size_t)(lmax + 1) * m;
+        const int l1 = min(m + sb * DSEG, ltr + 1);
+        SFRec<NG> n;
+        auto load = [&](int l0) {
+            // uniform bases and one 32-bit lane offset (64-bit addresses per field would
+            // take the registers of a wave)
+            const unsigned l = l0 + (lane & 15), lc = 16u * min(l, (unsigned)lmax);
+            n.b = qb[l];
+            n.c = qc[l];
+#pragma unroll
+            for (int f = 0; f < NG; ++f)
+                n.v[f] = *(const double2 *)((const char *)(av + (size_t)min(f, nfl - 1) * a.spec_fstride) + lc);
+        };
+        int l = m + sa * DSEG;
+        load(l);
+        bool slow = __any(kk > 0);
+        // the group's operands, and the loads of the next group (the last one reads clamped
+        // positions and is not used)
+        auto take = [&](SFRec<NG> &r) {
+            if (l + 16 > l1) {  // degrees past the last one contribute nothing
+                const bool in = l + (lane & 15) < l1;
+#pragma unroll
+                for (int f = 0; f < NG; ++f) {
+                    n.v[f].x = in ? n.v[f].x : 0.0;
+                    n.v[f].y = in ? n.v[f].y : 0.0;
+                }
+            }
+            r.b = n.b;
+            const double sc = a.qscale_in ? n.c : 1.0;
+#pragma unroll
+            for (int f = 0; f < NG; ++f) r.v[f] = make_double2(n.v[f].x * sc, n.v[f].y * sc);
+            load(l + 16);
+            asm volatile("s_nop 4");
+        };
+        // groups with scaled lanes first (a lane never becomes scaled again), then the rest in
+        // a loop of its own, whose registers hold one body
+        for (; l < l1 && slow; l += 16) {
+            SFRec<NG> r;
+            take(r);
+            sf_steps<NG, false, 0>(r, x, kk == 0 ? 1.0 : 0.0, prev, cur, acc);
+            // one check per 16 degrees: growth below 2^120, so what a chain misses before it
+            // counts is below 2^(100 + 120 - 512)
+            const double cl = qcm[l + 15];
+            if (kk > 0 && fmax(fabs(cur), fabs(prev)) * cl > kHi) {
+                cur *= kDown;
+                prev *= kDown;
+                kk -= 1;
+            }
+            slow = __any(kk > 0);
+            if (((l - m + 16) & (DSEG - 1)) == 0) {  // the Q form of the next segment
+                prev *= cl;
+                cur *= cl;
+            }
+        }
+        // once every lane is live each segment starts from its own seeds, loaded a segment ahead
+        size_t qn = (size_t)(segb + (l - m) / DSEG + 1) * np + pc;
+        double nq0 = 0.0, nq1 = 0.0;
+        auto load_seeds = [&] {
+            if (m + ((l - m) / DSEG + 1) * DSEG < l1) {
+                nq0 = a.seedq0[qn];
+                nq1 = a.seedq1[qn];
+                qn += np;
+            }
+        };
+        load_seeds();
+        for (; l < l1; l += 16) {
+            SFRec<NG> r;
+            take(r);
+            sf_steps<NG, true, 0>(r, x, 1.0, prev, cur, acc);
+            if (((l - m + 16) & (DSEG - 1)) == 0) {
+                prev = nq0;
+                cur = nq1;
+                l += 16;
+                load_seeds();
+                l -= 16;
+            }
+        }
+    }
+    if constexpr (NW > 1) {
+        if (w > 0)
+#pragma unroll
+            for (int f = 0; f < NG; ++f)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) red[w - 1][4 * f + k][lane] = acc[k >> 1][f][k & 1];
+        __syncthreads();
+        if (w > 0) return;
+#pragma unroll
+        for (int f = 0; f < NG; ++f)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int v = 0; v < NW - 1; ++v) acc[k >> 1][f][k & 1] += red[v][4 * f + k][lane];
+    }
+    if (p >= np) return;
+    const double sc = a.g * mfac_of(a.mfac_mode, m) * (a.wlat ? a.wlat[p] : 1.0);
+    double2 *Fo = a.F0 + ((size_t)f0 * a.nm + im) * a.nlat;
+    const int ps = a.nlat - 1 - p;
+#pragma unroll
+    for (int f = 0; f < NG; ++f) {
+        if (f >= nfl) break;
+        double2 *Ff = Fo + (size_t)f * a.nm * a.nlat;
+        Ff[p] = make_double2((acc[0][f][0] + acc[1][f][0]) * sc, (acc[0][f][1] + acc[1][f][1]) * sc);
+        if (ps != p) Ff[ps] = make_double2((acc[0][f][0] - acc[1][f][0]) * sc, (acc[0][f][1] - acc[1][f][1]) * sc);
+    }
+}
+
+template <int NG>
+void launch_synth_sf(const LegArgs &a, hipStream_t st) {
+    const long long units = (long long)a.nm * a.gx * a.gz;
+    // 2 waves per unit where one would leave the chip short of waves (4096 units, 16
+    // fields at lmax 511: 65 -> 62 us; 16384, 16 at 1023: 429 against 432; 4 waves lose
+    // the accumulator traffic through LDS: 98 us at 511)
+    const dim3 grid((unsigned)units);
+    if (units >= 8192 || a.lmax < DSEG) hipLaunchKernelGGL((k_synth_sf<NG, 1>), grid, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((k_synth_sf<NG, 2>), grid, dim3(128), 0, st, a);
+}
+
 }  // namespace
 
 // A group costs the same for 1 to 8 fields.  Against the single-field kernel, lmax
@@ -264,6 +456,26 @@ hipError_t launch_fields_anal(const LegArgs &a0, int nfields, hipStream_t st) {
     const dim3 grid((unsigned)a.nlist * a.gz);
     if (a.io_f32) hipLaunchKernelGGL(k_anal_mx<float>, grid, dim3(64), 0, st, a);
     else hipLaunchKernelGGL(k_anal_mx<double>, grid, dim3(64), 0, st, a);
+    return hipGetLastError();
+}
+
+bool fields_synth_ok(const LegArgs &a, int nfields) { return nfields >= 2 && a.seg == DSEG; }
+
+hipError_t launch_fields_synth(const LegArgs &a0, int nfields, hipStream_t st) {
+    LegArgs a = a0;
+    a.nf = nfields;
+    a.gx = (a.np + 63) / 64;
+    // equal groups of at most 8 fields
+    a.gz = (nfields + 7) / 8;
+    switch ((nfields + a.gz - 1) / a.gz) {
+        case 2: launch_synth_sf<2>(a, st); break;
+        case 3: launch_synth_sf<3>(a, st); break;
+        case 4: launch_synth_sf<4>(a, st); break;
+        case 5: launch_synth_sf<5>(a, st); break;
+        case 6: launch_synth_sf<6>(a, st); break;
+        case 7: launch_synth_sf<7>(a, st); break;
+        default: launch_synth_sf<8>(a, st); break;
+    }
     return hipGetLastError();
 }
 

@@ -416,6 +416,8 @@ hipError_t launch_leg_synth(const LegArgs &a, int nfields, int vector, int chain
 hipError_t launch_leg_anal(const LegArgs &a, int nfields, int vector, hipStream_t st);
 // FP64 kernels of field groups (shtk_fields.hip).
 int fields_anal_count(const LegArgs &a, int nfields);  // leading fields it takes (0: none)
+bool fields_synth_ok(const LegArgs &a, int nfields);
+hipError_t launch_fields_synth(const LegArgs &a, int nfields, hipStream_t st);
 hipError_t launch_fields_anal(const LegArgs &a, int nfields, hipStream_t st);
 hipError_t launch_fft(const FftArgs &a, int nfields, int inverse, hipStream_t st);
 hipError_t launch_spec_scale(const void *in, void *out, int in_f32, int out_f32, const double *scale, int divide,

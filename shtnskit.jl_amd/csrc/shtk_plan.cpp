@@ -932,6 +932,9 @@ int run_to_grid(shtk_plan *p, const Job &j, const void *s0, const void *s1, void
                           [&] { return shtk::launch_leg_synth(a, nf, 1, p->vsynth_chains, st); }),
                     "Legendre synthesis launch");
             HIP_TRY(side.join(), "order-0 rows join");
+        } else if (!j.vector && shtk::fields_synth_ok(a, nf)) {
+            HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_fields_synth(a, nf, st); }),
+                    "Legendre synthesis launch");
         } else {
             HIP_TRY(timed(p, j.leg_name, st,
                           [&] { return shtk::launch_leg_synth(a, nf, j.vector, j.vector ? p->vsynth_chains : p->synth_chains, st); }),

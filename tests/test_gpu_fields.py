@@ -67,3 +67,38 @@ def test_batch_adjoint_synthesis_matches_oracle(shtk, oracle, cuda, lmax, nlat, 
     got = to_host(shtk._adjoint_synthesis(cfg, to_dev(f32)))
     assert got.dtype == np.complex64
     assert _worst(got, ocfg.adjoint_synthesis(f32.astype(np.float64))) < 1e-6
+
+
+@pytest.mark.parametrize("lmax,nlat,nlon,mres,ltr,nf", SHAPES + [
+    (40, 41, 82, 1, 17, 2),
+    (191, 193, 384, 1, -1, 3),     # degrees fill whole segments
+    (128, 200, 258, 1, 127, 7),
+])
+def test_batch_synthesis_matches_oracle(shtk, oracle, cuda, lmax, nlat, nlon, mres, ltr, nf):
+    cfg = shtk.create_gauss_config(lmax, nlat, nlon=nlon, mres=mres)
+    ocfg = oracle.Config(lmax, nlat, nlon=nlon, mres=mres)
+    alm = oracle.random_alm(lmax, lmax, seed=lmax, power=1.0, nf=nf)
+    if 0 <= ltr < lmax:
+        alm[ltr + 1:] = np.nan  # not read
+    ref = ocfg.synthesis(np.nan_to_num(alm), ltr=ltr)
+    print(f"synthesis lmax={lmax} nlat={nlat} mres={mres} ltr={ltr} nf={nf}", flush=True)
+    assert _worst(to_host(shtk.synthesis_batch(cfg, to_dev(alm), ltr=ltr)), ref) < TOL
+
+
+@pytest.mark.parametrize("lmax,nlat,nlon,mres,ltr,nf", SHAPES[1:4])
+def test_batch_adjoint_analysis_and_conventions(shtk, oracle, cuda, lmax, nlat, nlon, mres, ltr, nf):
+    alm = oracle.random_alm(lmax, lmax, seed=lmax, power=1.0, nf=nf)
+    print(f"adjoint analysis lmax={lmax} nlat={nlat} nf={nf}", flush=True)
+    cfg, ocfg = shtk.create_gauss_config(lmax, nlat, nlon=nlon), oracle.Config(lmax, nlat, nlon=nlon)
+    assert _worst(to_host(shtk._adjoint_analysis(cfg, to_dev(alm))), ocfg.adjoint_analysis(alm)) < TOL
+    kw = dict(nlon=nlon, norm="schmidt", cs_phase=False, real_norm=True)
+    cfg, ocfg = shtk.create_gauss_config(lmax, nlat, **kw), oracle.Config(lmax, nlat, **kw)
+    ref = ocfg.synthesis(alm)
+    f = shtk.synthesis_batch(cfg, to_dev(alm))
+    assert _worst(to_host(f), ref) < TOL
+    assert _worst(to_host(shtk.analysis_batch(cfg, f)), ocfg.analysis(to_host(f))) < TOL
+    a32 = alm.astype(np.complex64)
+    f32 = to_host(shtk.synthesis_batch(cfg, to_dev(a32)))
+    assert f32.dtype == np.float32 and _worst(f32, ocfg.synthesis(a32.astype(np.complex128))) < 1e-6
+    assert _worst(to_host(shtk.synthesis_batch(cfg, to_dev(alm), real_output=False)),
+                  ocfg.synthesis(alm, real_output=False)) < TOL
