@@ -315,6 +315,12 @@ __device__ __forceinline__ FftTile fft_tiles(const FftArgs &a, int G, int nfield
     return t;
 }
 
+// Grid of field f (n elements per field).
+template <typename GT>
+__device__ __forceinline__ GT *fft_grid(const FftArgs &a, int f, size_t n) {
+    return a.grid1 && f >= a.nf0 ? (GT *)a.grid1 + (size_t)(f - a.nf0) * n : (GT *)a.grid + (size_t)f * n;
+}
+
 // Row factor of latitude lat (pair index p = min(lat, nlat - 1 - lat)).
 __device__ __forceinline__ double fft_row_scale(const FftArgs &a, int lat) {
     const int p = min(lat, a.nlat - 1 - lat);
@@ -387,7 +393,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_t(const FftArgs a, int nfiel
         __syncthreads();
         fft_lds<+1, GEN>(zs + row * RS, a, lt, tr);
         const int nrow = a.nrow;
-        GT *gf = (GT *)a.grid + (size_t)f * nrow * N + lat;
+        GT *gf = fft_grid<GT>(a, f, (size_t)nrow * N) + lat;
         if (live && lat < nrow) {
             const double sc = fft_row_scale(a, lat);
             // this lane's latitude is the real (k < G) or imaginary part of the packed row
@@ -427,7 +433,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_c(const FftArgs a, int nfiel
         __syncthreads();
         fft_lds<+1, GEN>(zs + row * RS, a, lt, tr);
         const int nrow = a.nrow;
-        GT *gf = (GT *)a.grid + 2 * ((size_t)f * nrow * N + lat);
+        GT *gf = fft_grid<GT>(a, f, 2 * (size_t)nrow * N) + 2 * lat;
         if (live && lat < nrow) {
             const double sc = fft_row_scale(a, lat);
             for (int e = tid; e < N * G; e += nt) {
@@ -459,7 +465,7 @@ __global__ __launch_bounds__(1024) void k_fft_anal_c(const FftArgs a, int nfield
         const int nrow = a.nrow;
         const bool has_row = live && lat < nrow;  // rows past nrow read as zero
         const double sc = live ? fft_row_scale(a, lat) : 0.0;
-        const GT *gf = (const GT *)a.grid + 2 * ((size_t)f * nrow * N + lat);
+        const GT *gf = fft_grid<GT>(a, f, 2 * (size_t)nrow * N) + 2 * lat;
         double2 *z = zs + k * RS;
         for (int e = tid; e < N * G; e += nt) {
             const int j = e / G;
@@ -501,7 +507,7 @@ __global__ __launch_bounds__(1024) void k_fft_anal_t(const FftArgs a, int nfield
         const double sc = live ? fft_row_scale(a, lat) : 0.0;
         const int nrow = a.nrow;
         const bool has_row = live && lat < nrow;  // rows past nrow read as zero
-        const GT *gf = (const GT *)a.grid + (size_t)f * nrow * N + lat;
+        const GT *gf = fft_grid<GT>(a, f, (size_t)nrow * N) + lat;
         double2 *z = zs + gk * RS;
         // this lane's latitude is the real (k < G) or imaginary part of the packed row
         double *zr = (double *)z + (k < G ? 0 : 1);

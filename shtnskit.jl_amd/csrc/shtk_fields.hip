@@ -86,10 +86,19 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
     // XCD, so its Fourier columns are read into one L2
     const int xcd = blockIdx.x % kXcds, fg = blockIdx.x / kXcds % a.gz;
     const cptr<int> item = as_const((const int *)a.seglist) + 4 * (size_t)(blockIdx.x / kXcds / a.gz * kXcds + xcd);
-    const int gs = item[0], im = item[1], s = item[2], coff = item[3];  // one load, short waves
-    if (gs < 0) return;
+    int gs = item[0], coff = item[3];  // one load, short waves
+    const int im = item[1], s = item[2];
+    if (gs < 0 || (a.skip_m0 && im == 0)) return;
     const int m = im * a.mres, np = a.np, nlat = a.nlat, lmax = a.lmax;
-    const int l0 = m + s * DSEG, lend = min(l0 + DSEG, lmax + 1), lstop = min(lend, a.ltr + 1);
+    const bool one = a.m0_one && im == 0;  // order 0 on the tables of order 1
+    const double *wlat = one ? a.wlat0 : a.wlat;
+    const int mt = one ? 1 : m;
+    if (one) {
+        gs = min(as_const(a.segbase)[1] + s, a.nseg_total - 1);
+        coff = (int)as_const(a.coff)[1];
+    }
+    const int l0 = mt + s * DSEG, lend = min(l0 + DSEG, lmax + 1), lstop = min(lend, a.ltr + 1);
+    if (l0 >= lend) return;  // order 1 can have one segment fewer
     const int lane = threadIdx.x;
     const int f0 = fg * MX_FIELDS, nfl = min(MX_FIELDS, a.nf - f0);
     OT *col = (OT *)a.out0 + 2 * ((size_t)f0 * a.spec_fstride + (size_t)(lmax + 1) * m);
@@ -112,7 +121,7 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
     const int pfirst = as_const(a.pfirst)[gs], pfast = as_const(a.pfast)[gs];
     const int nch = l0 < lstop ? (np - min(pfirst, np) + 63) / 64 : 0;  // 64-pair chains, ending at the equator
     const int pst = np - 64 * nch;
-    const long long co = (long long)coff - m;
+    const long long co = (long long)coff - mt;
     const double *qbv = a.qb + co + l0 + 1 + (lane & 15);  // padded past lmax
     const double b0 = qbv[0], b1 = qbv[16], b2 = qbv[32], b3 = qbv[48];
     const cptr<double> qcm = as_const(a.qcc) + co;
@@ -139,7 +148,7 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
         nq1 = a.seedq1[q];
         nk = a.seedk[q];
         nx = a.x[p];
-        nw = a.wlat ? a.wlat[p] : 1.0;
+        nw = wlat ? wlat[p] : 1.0;
         if (2 * p == nlat - 1) nw *= 0.5;  // the equator's latitude is both halves of its pair
         if (pst + 64 * ch + lane < 0) nw = 0.0;
     };
@@ -236,7 +245,7 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
     __builtin_amdgcn_wave_barrier();
     const int l = l0 + lane, i = (lane & 31) >> 1;
     if (l >= lend) return;
-    const double sc = l < lstop ? a.g * mfac_of(a.mfac_mode, m) * a.qcc[co + l] : 0.0;
+    const double sc = l < lstop ? a.g * mfac_of(a.mfac_mode, m) * (a.raw_q ? 1.0 : a.qcc[co + l]) : 0.0;
     const double *src = tile + (8 * (lane >> 5) + 4 * (lane & 1) + (i >> 2)) * 64 + (i & 3) * 16;
     for (int f = 0; f < nfl; ++f) {
         const double2 v = *(const double2 *)(src + 2 * f);
@@ -287,23 +296,36 @@ __device__ __forceinline__ void sf_steps(const SFRec<NG> &r, double x, double cm
     }
 }
 
-template <int NG, int NW>
+// The degree before (N = 0, odd) or after (N = 1, even) a segment, operands in lane N of
+// each row.
+template <int NG, int N>
+__device__ __forceinline__ void sf_edge(const double2 *eg, double (*acc)[NG][2], double u) {
+#pragma unroll
+    for (int f = 0; f < NG; ++f) {
+        SHTK_FMAC_BC(acc[1 - N][f][0], eg[f].x, u, N, "");
+        SHTK_FMAC_BC(acc[1 - N][f][1], eg[f].y, u, N, "");
+    }
+}
+
+template <int NG, int NW, bool VEC>
 __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const LegArgs a) {
     __shared__ double red[NW > 1 ? NW - 1 : 1][NW > 1 ? 4 * NG : 1][64];
     // units lowest order first for every pair block and group: the long columns start first
     const int unit = blockIdx.x, b = unit % a.gx, fg = unit / a.gx % a.gz, im = unit / (a.gx * a.gz);
+    if (a.skip_m0 && im == 0) return;
     const int m = im * a.mres, np = a.np, lmax = a.lmax, ltr = a.ltr;
     const int lane = threadIdx.x & 63;
     const int w = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int f0 = fg * NG, nfl = min(NG, a.nf - f0);
     const int p = b * 64 + lane, pc = min(p, np - 1), pb1 = min(b * 64 + 64, np);
-    const int segb = as_const(a.segbase)[im];
-    const long long co = as_const(a.coff)[im] - m;
+    const bool one = VEC && a.m0_one && im == 0;  // order 0 on the tables of order 1
+    const int mt = one ? 1 : m, segb = as_const(a.segbase)[one ? 1 : im];
+    const long long co = as_const(a.coff)[one ? 1 : im] - mt;
     double acc[2][NG][2];
 #pragma unroll
     for (int f = 0; f < NG; ++f) acc[0][f][0] = acc[0][f][1] = acc[1][f][0] = acc[1][f][1] = 0.0;
     // first segment with a live pair of this block
-    const int nseg = ltr >= m ? (ltr - m) / DSEG + 1 : 0;
+    const int nseg = ltr >= mt ? (ltr - mt) / DSEG + 1 : 0;
     int s0 = nseg;
     for (int q = 0; q < nseg; q += 64) {
         const unsigned long long live = __ballot(q + lane < nseg && pb1 > a.pfirst[segb + min(q + lane, nseg - 1)]);
@@ -322,7 +344,7 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
         const double *qb = a.qb + co + 1, *qc = a.qcc + co;  // padded past lmax
         const cptr<double> qcm = as_const(a.qcc) + co;
         const double2 *av = (const double2 *)a.in0 + (size_t)f0 * a.spec_fstride + (size_t)(lmax + 1) * m;
-        const int l1 = min(m + sb * DSEG, ltr + 1);
+        const int l1 = min(mt + sb * DSEG, ltr + 1);  // VEC: ltr is the degree after the last S, T
         SFRec<NG> n;
         auto load = [&](int l0) {
             // uniform bases and one 32-bit lane offset (64-bit addresses per field would
@@ -334,9 +356,27 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
             for (int f = 0; f < NG; ++f)
                 n.v[f] = *(const double2 *)((const char *)(av + (size_t)min(f, nfl - 1) * a.spec_fstride) + lc);
         };
-        int l = m + sa * DSEG;
+        int l = mt + sa * DSEG;
         load(l);
         bool slow = __any(kk > 0);
+        // VEC: the terms that reach past the segments (a.edge): the degree before segment
+        // s (its Q is prev there) and the degree after the one that ends (cur)
+        const double2 *ev = VEC ? a.edge + 2 * ((size_t)f0 * a.nseg_total + as_const(a.segbase)[im]) : nullptr;
+        double2 eg[VEC ? NG : 1];
+        auto load_edges = [&]([[maybe_unused]] int s) {  // lane 0 of a row: before segment s, lane 1: after segment s - 1
+            if constexpr (VEC) {
+                const unsigned o = 16u * ((lane & 15) == 0 ? 2 * min(s, nseg - 1) : max(2 * s - 1, 0));
+#pragma unroll
+                for (int f = 0; f < NG; ++f)
+                    eg[f] = *(const double2 *)((const char *)(ev + 2 * (size_t)min(f, nfl - 1) * a.nseg_total) + o);
+                asm volatile("s_nop 4");
+            }
+        };
+        if constexpr (VEC)
+            if (sa > 0) {
+                load_edges(sa);
+                sf_edge<NG, 0>(eg, acc, kk == 0 ? prev : 0.0);
+            }
         // the group's operands, and the loads of the next group (the last one reads clamped
         // positions and is not used)
         auto take = [&](SFRec<NG> &r) {
@@ -370,16 +410,21 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
                 kk -= 1;
             }
             slow = __any(kk > 0);
-            if (((l - m + 16) & (DSEG - 1)) == 0) {  // the Q form of the next segment
+            if (((l - mt + 16) & (DSEG - 1)) == 0 && l + 16 <= l1) {  // the Q form of the next segment
+                const int s = (l - mt + 16) / DSEG;
+                if constexpr (VEC) load_edges(s);
+                if constexpr (VEC) sf_edge<NG, 1>(eg, acc, kk == 0 ? cur : 0.0);
                 prev *= cl;
                 cur *= cl;
+                if constexpr (VEC)
+                    if (s < sb) sf_edge<NG, 0>(eg, acc, kk == 0 ? prev : 0.0);
             }
         }
         // once every lane is live each segment starts from its own seeds, loaded a segment ahead
-        size_t qn = (size_t)(segb + (l - m) / DSEG + 1) * np + pc;
+        size_t qn = (size_t)(segb + (l - mt) / DSEG + 1) * np + pc;
         double nq0 = 0.0, nq1 = 0.0;
         auto load_seeds = [&] {
-            if (m + ((l - m) / DSEG + 1) * DSEG < l1) {
+            if (mt + ((l - mt) / DSEG + 1) * DSEG < l1) {
                 nq0 = a.seedq0[qn];
                 nq1 = a.seedq1[qn];
                 qn += np;
@@ -390,9 +435,14 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
             SFRec<NG> r;
             take(r);
             sf_steps<NG, true, 0>(r, x, 1.0, prev, cur, acc);
-            if (((l - m + 16) & (DSEG - 1)) == 0) {
+            if (((l - mt + 16) & (DSEG - 1)) == 0 && l + 16 <= l1) {
+                const int s = (l - mt + 16) / DSEG;
+                if constexpr (VEC) load_edges(s);
+                if constexpr (VEC) sf_edge<NG, 1>(eg, acc, cur);
                 prev = nq0;
                 cur = nq1;
+                if constexpr (VEC)
+                    if (s < sb) sf_edge<NG, 0>(eg, acc, prev);
                 l += 16;
                 load_seeds();
                 l -= 16;
@@ -415,7 +465,8 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
                 for (int v = 0; v < NW - 1; ++v) acc[k >> 1][f][k & 1] += red[v][4 * f + k][lane];
     }
     if (p >= np) return;
-    const double sc = a.g * mfac_of(a.mfac_mode, m) * (a.wlat ? a.wlat[p] : 1.0);
+    const double *wlat = one ? a.wlat0 : a.wlat;
+    const double sc = a.g * mfac_of(a.mfac_mode, m) * (wlat ? wlat[p] : 1.0);
     double2 *Fo = a.F0 + ((size_t)f0 * a.nm + im) * a.nlat;
     const int ps = a.nlat - 1 - p;
 #pragma unroll
@@ -427,15 +478,137 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
     }
 }
 
-template <int NG>
+template <int NG, bool VEC>
 void launch_synth_sf(const LegArgs &a, hipStream_t st) {
-    const long long units = (long long)a.nm * a.gx * a.gz;
+    const long long units = (long long)(a.nm_run > 0 ? std::min(a.nm_run, a.nm) : a.nm) * a.gx * a.gz;
     // 2 waves per unit where one would leave the chip short of waves (4096 units, 16
     // fields at lmax 511: 65 -> 62 us; 16384, 16 at 1023: 429 against 432; 4 waves lose
     // the accumulator traffic through LDS: 98 us at 511)
     const dim3 grid((unsigned)units);
-    if (units >= 8192 || a.lmax < DSEG) hipLaunchKernelGGL((k_synth_sf<NG, 1>), grid, dim3(64), 0, st, a);
-    else hipLaunchKernelGGL((k_synth_sf<NG, 2>), grid, dim3(128), 0, st, a);
+    if (units >= 8192 || a.lmax < DSEG) hipLaunchKernelGGL((k_synth_sf<NG, 1, VEC>), grid, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((k_synth_sf<NG, 2, VEC>), grid, dim3(128), 0, st, a);
+}
+
+// ---------------------------------------------------------------------------
+// Vector synthesis as two scalar ones of degree lmax + 1: with d_l = sqrt((l^2 - m^2) /
+// (4 l^2 - 1)) the coefficients of sin(theta) V_theta and sin(theta) V_phi are
+//     (l-1) d_l S_{l-1} - (l+2) d_{l+1} S_{l+1} - i m T_l
+//     i m S_l + (l-1) d_l T_{l-1} - (l+2) d_{l+1} T_{l+1}
+// (src/legendre.jl:542-546 applied to the sums of src/kernels.jl:155-169).  Written
+// times c_l, the form k_synth_sf takes: c_l d_l = c_{l-1} and d_l^2 = beta_{l+1}, so
+// they need no root, and both degrees that one S_l reaches carry the same c_l.  The
+// two terms cancel near the poles, so they also have to come from one segment's
+// recurrence: where S_l reaches past its segment the term goes to E instead, which
+// k_synth_sf adds with that segment's own Q at the degree before or after it (with
+// the neighbour segment's Q the error of the grid was 10 to 17 % larger).
+// m0_one: dP_l/dtheta of order 0 is sqrt(l(l+1)) P_l^1, so order 0 needs no division by
+// sin(theta): its column holds sqrt(l(l+1)) S_l (and T_l) for the recurrence of order 1, and
+// its rows take their own factor (LegArgs.wlat0).  That is the differentiated recurrence of the
+// zonal kernel in one more order of the same launch, instead of a kernel on a second stream
+// (two events and two waits: 20 to 30 us of a call of 70).
+// One block per (order, field); [theta fields][phi fields], columns of lmax + 2 and
+// E[field][segment][before, after].
+// ---------------------------------------------------------------------------
+template <typename IT>
+__global__ __launch_bounds__(256) void k_vcoef(const IT *S, const IT *T, double2 *C, double2 *E, const int *segbase,
+                                               int nseg_total, const double *scale, int divide, int ll1,
+                                               const double *qb, const double *qcc, const long long *coff,
+                                               int lmax, int mres, int nm, int ltr, int m0_one, long long in_fstride,
+                                               long long out_fstride, int nf) {
+    const int im = blockIdx.x % nm, f = blockIdx.x / nm, m = im * mres;
+    const size_t col = (size_t)(lmax + 1) * m;
+    const IT *Sm = S + 2 * ((size_t)f * in_fstride + col), *Tm = T + 2 * ((size_t)f * in_fstride + col);
+    const double *sm = scale ? scale + col : nullptr;
+    const double *cq = qcc + coff[im] - m, *bq = qb + coff[im] - m;
+    double2 *Ct = C + (size_t)f * out_fstride + (size_t)(lmax + 2) * m;
+    double2 *Cp = Ct + (size_t)nf * out_fstride;
+    const int lo = max(1, m), hi = min(ltr, lmax);
+    for (int l = m + (int)threadIdx.x; l <= lmax + 1; l += 256) {
+        const int t = l - m;
+        // S_k, T_k times k's factor, zero outside [lo, hi] (clamped reads)
+        auto at = [&](int k, double fac, double2 *s, double2 *q) {
+            const bool in = k >= lo && k <= hi;
+            const int kc = min(max(k, m), lmax);
+            if (sm) fac = divide ? fac / sm[kc] : fac * sm[kc];
+            if (ll1 && in) fac /= (double)k * (k + 1);
+            *s = in ? make_double2(fac * (double)Sm[2 * kc], fac * (double)Sm[2 * kc + 1]) : make_double2(0.0, 0.0);
+            *q = in ? make_double2(fac * (double)Tm[2 * kc], fac * (double)Tm[2 * kc + 1]) : make_double2(0.0, 0.0);
+        };
+        const bool first = t % DSEG == 0, last = t % DSEG == DSEG - 1;  // in the segment
+        double2 s1, t1, s0, t0, s2, t2, q, r;
+        if (m0_one && m == 0) {
+            const int l1 = max(l, 1);
+            at(l, sqrt((double)l1 * (l1 + 1)) * qcc[coff[1] + l1 - 1], &Ct[l], &Cp[l]);
+            if (first || last) {
+                const size_t e = 2 * ((size_t)f * nseg_total + segbase[0] + t / DSEG) + (last ? 1 : 0);
+                E[e] = E[e + 2 * (size_t)nf * nseg_total] = make_double2(0.0, 0.0);
+            }
+            continue;
+        }
+        const double cl = cq[l];
+        at(first ? -1 : l - 1, (l - 1) * cq[max(l - 1, m)], &s1, &t1);
+        at(l, m * cl, &s0, &t0);
+        at(last ? -1 : l + 1, (l + 2) * bq[min(l, lmax - 1) + 2] * cq[min(l, lmax) + 1], &s2, &t2);
+        Ct[l] = make_double2(s1.x - s2.x + t0.y, s1.y - s2.y - t0.x);
+        Cp[l] = make_double2(t1.x - t2.x - s0.y, t1.y - t2.y + s0.x);
+        if (first || last) {  // S_l at degree l - 1 (before), at degree l + 1 (after)
+            at(l, first ? -(l + 1) * bq[min(l, lmax) + 1] * cl : l * cl, &q, &r);
+            const size_t e = 2 * ((size_t)f * nseg_total + segbase[im] + t / DSEG) + (last ? 1 : 0);
+            E[e] = q;
+            E[e + 2 * (size_t)nf * nseg_total] = r;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Vector analysis from two scalar ones of degree lmax + 1 with the weights w / sin(theta):
+//     S_l = [l d_{l+1} Gt_{l+1} - (l+1) d_l Gt_{l-1} - i m Gp_l] / (l(l+1))
+//     T_l = [i m Gt_l + l d_{l+1} Gp_{l+1} - (l+1) d_l Gp_{l-1}] / (l(l+1))
+// (src/kernels.jl:205-215; ll1 = 0: without the division).  H: the sums against Q_l = P_l /
+// c_l (LegArgs.raw_q), so with the identities of k_vcoef the factors are table entries:
+// d_{l+1} c_{l+1} = c_l, or 1 where l + 1 starts a segment, and d_l c_{l-1} = beta_{l+1} c_l,
+// times c_{l-1} of its own segment where l starts one.  One block per (column,
+// field); columns that are not orders and rows l < max(1, m) or l > ltr are written
+// as zero.  skip_m0: the zonal kernel writes the degrees to ltr of order 0.  m0_one: order 0
+// has S_l = c_l Gt_l sqrt(l(l+1)) / (l(l+1)), T_l the same of Gp, on order 1's tables.
+// ---------------------------------------------------------------------------
+template <typename OT>
+__global__ __launch_bounds__(256) void k_vout(const double2 *H, OT *S, OT *T, const double *scale, int divide, int ll1,
+                                              int skip_m0, int m0_one, const double *qb, const double *qcc, const long long *coff,
+                                              int lmax, int mmax, int mres, int ltr, long long h_fstride,
+                                              long long out_fstride, int nf) {
+    const int m = blockIdx.x % (mmax + 1), f = blockIdx.x / (mmax + 1), im = m / mres;
+    const bool order = im * mres == m;
+    const size_t col = (size_t)(lmax + 1) * m;
+    OT *So = S + 2 * ((size_t)f * out_fstride + col), *To = T + 2 * ((size_t)f * out_fstride + col);
+    const double2 *Ht = H + (size_t)f * h_fstride + (size_t)(lmax + 2) * m, *Hp = Ht + (size_t)nf * h_fstride;
+    const double *cq = qcc + coff[im] - im * mres, *bq = qb + coff[im] - im * mres;
+    const int lo = max(1, m), hi = min(ltr, lmax);
+    for (int l = (int)threadIdx.x + (skip_m0 && m == 0 ? hi + 1 : 0); l <= lmax; l += 256) {
+        double2 s = make_double2(0.0, 0.0), t = s;
+        if (order && l >= lo && l <= hi) {
+            const int lm = max(l - 1, m), r = l - m;
+            const double c = cq[l];
+            double k = ll1 ? 1.0 / ((double)l * (l + 1)) : 1.0;
+            if (scale) k = divide ? k / scale[col + l] : k * scale[col + l];
+            if (m0_one && m == 0) {
+                const double fac = sqrt((double)l * (l + 1)) * qcc[coff[1] + l - 1] * k;
+                const double2 t0 = Ht[l], p0 = Hp[l];
+                s = make_double2(fac * t0.x, fac * t0.y);
+                t = make_double2(fac * p0.x, fac * p0.y);
+            } else {
+                const double up = l * ((r + 1) % DSEG == 0 ? 1.0 : c) * k, mc = m * c * k;
+                const double dn = (l + 1) * bq[l + 1] * c * (r % DSEG == 0 ? cq[lm] : 1.0) * k;  // 0 for l = m
+                const double2 t2 = Ht[l + 1], t0 = Ht[l], t1 = Ht[lm], p2 = Hp[l + 1], p0 = Hp[l], p1 = Hp[lm];
+                s = make_double2(up * t2.x - dn * t1.x + mc * p0.y, up * t2.y - dn * t1.y - mc * p0.x);
+                t = make_double2(up * p2.x - dn * p1.x - mc * t0.y, up * p2.y - dn * p1.y + mc * t0.x);
+            }
+        }
+        So[2 * l] = (OT)s.x;
+        So[2 * l + 1] = (OT)s.y;
+        To[2 * l] = (OT)t.x;
+        To[2 * l + 1] = (OT)t.y;
+    }
 }
 
 }  // namespace
@@ -461,21 +634,61 @@ hipError_t launch_fields_anal(const LegArgs &a0, int nfields, hipStream_t st) {
 
 bool fields_synth_ok(const LegArgs &a, int nfields) { return nfields >= 2 && a.seg == DSEG; }
 
+template <bool VEC>
+static void launch_synth_groups(const LegArgs &a, int ng, hipStream_t st) {
+    switch (ng) {
+        case 2: launch_synth_sf<2, VEC>(a, st); break;
+        case 3: launch_synth_sf<3, VEC>(a, st); break;
+        case 4: launch_synth_sf<4, VEC>(a, st); break;
+        case 5: launch_synth_sf<5, VEC>(a, st); break;
+        case 6: launch_synth_sf<6, VEC>(a, st); break;
+        case 7: launch_synth_sf<7, VEC>(a, st); break;
+        default: launch_synth_sf<8, VEC>(a, st); break;
+    }
+}
+
 hipError_t launch_fields_synth(const LegArgs &a0, int nfields, hipStream_t st) {
     LegArgs a = a0;
     a.nf = nfields;
     a.gx = (a.np + 63) / 64;
     // equal groups of at most 8 fields
     a.gz = (nfields + 7) / 8;
-    switch ((nfields + a.gz - 1) / a.gz) {
-        case 2: launch_synth_sf<2>(a, st); break;
-        case 3: launch_synth_sf<3>(a, st); break;
-        case 4: launch_synth_sf<4>(a, st); break;
-        case 5: launch_synth_sf<5>(a, st); break;
-        case 6: launch_synth_sf<6>(a, st); break;
-        case 7: launch_synth_sf<7>(a, st); break;
-        default: launch_synth_sf<8>(a, st); break;
-    }
+    const int ng = (nfields + a.gz - 1) / a.gz;
+    if (a.edge) launch_synth_groups<true>(a, ng, st);
+    else launch_synth_groups<false>(a, ng, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_vcoef(const void *S, const void *T, void *C, void *E, int in_f32, const double *scale, int divide, int ll1,
+                        const LegArgs &v, int nf, hipStream_t st) {
+    const int lmax = v.lmax - 1, ltr = v.ltr - 1;
+    const long long in_fs = (long long)(lmax + 1) * (v.mmax + 1);
+    const int nm = v.nm_run > 0 ? std::min(v.nm_run, v.nm) : v.nm;
+    const dim3 grid((unsigned)nm * nf);
+    if (in_f32)
+        hipLaunchKernelGGL(k_vcoef<float>, grid, dim3(256), 0, st, (const float *)S, (const float *)T, (double2 *)C,
+                           (double2 *)E, v.segbase, v.nseg_total, scale, divide, ll1, v.qb, v.qcc, v.coff, lmax, v.mres,
+                           nm, ltr, v.m0_one, in_fs, v.spec_fstride, nf);
+    else
+        hipLaunchKernelGGL(k_vcoef<double>, grid, dim3(256), 0, st, (const double *)S, (const double *)T, (double2 *)C,
+                           (double2 *)E, v.segbase, v.nseg_total, scale, divide, ll1, v.qb, v.qcc, v.coff, lmax, v.mres,
+                           nm, ltr, v.m0_one, in_fs, v.spec_fstride, nf);
+    return hipGetLastError();
+}
+
+hipError_t launch_vout(const void *H, void *S, void *T, int out_f32, const double *scale, int divide, int ll1,
+                       int skip_m0, const LegArgs &v, int nf, hipStream_t st) {
+    const int lmax = v.lmax - 1, ltr = v.ltr - 1;
+    const long long out_fs = (long long)(lmax + 1) * (v.mmax + 1);
+    const dim3 grid((unsigned)(v.mmax + 1) * nf);
+    if (out_f32)
+        hipLaunchKernelGGL(k_vout<float>, grid, dim3(256), 0, st, (const double2 *)H, (float *)S, (float *)T, scale,
+                           divide, ll1, skip_m0, v.m0_one, v.qb, v.qcc, v.coff, lmax, v.mmax, v.mres, ltr, v.spec_fstride, out_fs,
+                           nf);
+    else
+        hipLaunchKernelGGL(k_vout<double>, grid, dim3(256), 0, st, (const double2 *)H, (double *)S, (double *)T, scale,
+                           divide, ll1, skip_m0, v.m0_one, v.qb, v.qcc, v.coff, lmax, v.mmax, v.mres, ltr, v.spec_fstride, out_fs,
+                           nf);
     return hipGetLastError();
 }
 

@@ -45,7 +45,7 @@ constexpr int DSEG = 64;  // segment length of the register-record Legendre kern
 // Coefficient tables, one block per stored order (offset coff[im], entries
 // l = m .. lmax+1):
 //   qc[l] = (beta_l, c_l)                  scalar and vector recurrences
-//   qd[l] = (l c_l, g_l c_{l-1})           vector: s dP_l/dtheta = l x P_l - g_l P_{l-1},
+//   qd[l] = (l c_l, g_l c_{l-1})           vector (other segment lengths than DSEG): s dP_l/dtheta = l x P_l - g_l P_{l-1},
 //                                          g_l = sqrt((2l+1)(l^2-m^2)/(2l-1))
 constexpr int OZ_TPAD = 64;  // entries past the end of the padded per-degree tables
 
@@ -80,19 +80,21 @@ struct LegArgs {
     const int4 *seglist;    // field-group analysis: [nlist] (global segment or -1, order, segment of the
                             // order, coff), entry i for XCD i mod 8
     int nlist;
+    int raw_q;              // scalar analysis: sums against Q_l, without the factor c_l
+    const double2 *edge;    // field-group synthesis of vector fields: [field][nseg_total][2] coefficients of the
+                            // degrees before and after each segment (launch_vcoef), or nullptr
     int gx, gy, gz;         // work items form a (gx, gy, gz = nfields) box, x fastest
     int xcd;                // synthesis: 1 keeps the pair blocks of an order on one XCD
     int nm_run;             // synthesis: only orders im < nm_run (0: all)
-    int skip_m0;            // vector: order 0 is computed by the zonal kernel (shtk_ml.hip)
+    int skip_m0;            // order 0 is left out (the zonal kernel of shtk_ml.hip computes it)
+    int m0_one;             // vector pair as scalar fields: order 0 runs on the tables of order 1 (launch_vcoef)
+    const double *wlat0;    // m0_one: wlat of order 0 (or nullptr)
     int qscale_in;          // scalar synthesis (64-degree segments): in0 holds canonical FP64
                             // coefficients, multiplied by c_l as they are loaded
-    int vwaves;             // vector synthesis (64-degree segments): waves per block, 1 or 4
     int s1w_units;          // scalar synthesis (64-degree segments): one wave per block when the
                             // launch has at least this many (order, pair block, field) units
     int apblk;              // analysis: latitude pairs per work item (512, or 256 for the vector
                             // analysis when it lets the kernel run 3 waves per SIMD)
-    int vdirect;            // vector synthesis (64-degree segments): in0 / in1 hold canonical FP64
-                            // S and T, the records (S, T, c_l S, c_l T) built as they are loaded
 };
 
 // Work distribution over the 8 XCDs (each with its own 4 MB L2).  The
@@ -122,6 +124,7 @@ inline unsigned grid_for_units(int xcd, int per_unit, int nunits) {
 }
 
 struct SeedArgs {
+    int lseg;           // segments cover the degrees to lseg (lmax, or lmax + 1)
     int lmax, mmax, mres, np, nm, seg;
     const double *x;
     const double2 *ab;  // P-form (a_l, b_l), same offsets as qc
@@ -162,6 +165,8 @@ struct FftArgs {
     const double2 *chirp, *bhat;
     double2 *F;               // Fourier workspace [field][im][nlat]
     void *grid;               // grid array (nrow, nlon, nfields)
+    void *grid1;              // vector pair in one launch: the grid of the fields nf0 .. (or nullptr)
+    int nf0;
     int nrow;                 // grid rows: nlat, or nlat - 1 when the last node (south pole) has no row
     int io_f32;
     int mode;          // grid row factor: 0 none, 1 1/sin(theta), 2 sin(theta) (Robert form)
@@ -176,7 +181,6 @@ struct shtk_plan {
     int np = 0, nm = 0, seg = 128, nseg_total = 0;
     int xcd_map = 0, synth_chains = 4, fft_tile = 0;  // launch-shape knobs
     int vsynth_chains = 1;
-    int vsynth_waves = 1;  // waves per vector synthesis block (SHTK_VSYNTH_WAVES: 1 or 4)
     int ssynth_1w_units = 8192;  // scalar synthesis: units from which blocks hold one wave
                                  // (SHTK_SSYNTH_1W_UNITS)
     int vanal_pblk = 256;  // pairs per vector analysis work item (SHTK_VANAL_PBLK: 256 or 512)  // latitude pairs per lane of the vector synthesis (1 or 2)
@@ -415,6 +419,12 @@ hipError_t launch_seed(const SeedArgs &a, hipStream_t st);
 hipError_t launch_leg_synth(const LegArgs &a, int nfields, int vector, int chains, hipStream_t st);
 hipError_t launch_leg_anal(const LegArgs &a, int nfields, int vector, hipStream_t st);
 // FP64 kernels of field groups (shtk_fields.hip).
+// Scalar coefficients times c_l of a vector synthesis; v: the scalar arguments (degree lmax + 1).
+hipError_t launch_vcoef(const void *S, const void *T, void *C, void *E, int in_f32, const double *scale, int divide, int ll1,
+                        const LegArgs &v, int nf, hipStream_t st);
+// S, T of a vector analysis from the scalar sums H of v (raw_q).
+hipError_t launch_vout(const void *H, void *S, void *T, int out_f32, const double *scale, int divide, int ll1,
+                       int skip_m0, const LegArgs &v, int nf, hipStream_t st);
 int fields_anal_count(const LegArgs &a, int nfields);  // leading fields it takes (0: none)
 bool fields_synth_ok(const LegArgs &a, int nfields);
 hipError_t launch_fields_synth(const LegArgs &a, int nfields, hipStream_t st);
@@ -468,9 +478,11 @@ hipError_t launch_zonal_seed(const MlArgs &a, double *out, int nseg, hipStream_t
 // poles (one block per field): synthesis rewrites them from the prologue
 // records in a.in0 times wscale (robert = 1: zeros every order's pole rows),
 // analysis adds the pole terms times wpole to the order-1 outputs in a.out0 / a.out1
-// (conv: the outputs are in the plan's convention map, or nullptr).
+// (conv: the outputs are in the plan's convention map, divided (conv_div) or multiplied
+// by it, or nullptr).
 hipError_t launch_vpole_synth(const LegArgs &a, int nfields, int robert, double wscale, hipStream_t st);
-hipError_t launch_vpole_anal(const LegArgs &a, int nfields, double wpole, const double *conv, hipStream_t st);
+hipError_t launch_vpole_anal(const LegArgs &a, int nfields, double wpole, const double *conv, int conv_div,
+                             hipStream_t st);
 // FFTs of complex grid rows: synthesis (inverse = 1) turns the bins m = 0 .. mmax
 // of F into complex rows; analysis (inverse = 0) keeps the bins m = 0 .. mmax of
 // each complex row's forward transform.

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void k_seed(const SeedArgs a) {
     const size_t sidx = (size_t)im * a.np + p;
     double cur = a.sectv[sidx], prev = 0.0;
     int k = a.sectk[sidx];
-    const int nseg = nseg_of(lmax, m, S);
+    const int nseg = nseg_of(a.lseg, m, S);
     int l = m;
     for (int s = 0; s < nseg; ++s) {
         const int gs = a.segbase[im] + s;
@@ -667,256 +667,6 @@ __global__ __launch_bounds__(256) void k_synth_v(const LegArgs a) {
     }
 }
 
-// ---------------------------------------------------------------------------
-// Vector synthesis with the per-degree operands in VGPRs (64-degree segments),
-// the treatment of k_synth_d: lane 16 r + n holds the record of degree
-// l0 + 16 g + n of record group g -- beta_{l+1}, l c_l, g_l c_{l-1} and the
-// prologue record (S', T', c_l S', c_l T') -- and every use broadcasts lane n of
-// the row (DPP row_newbcast:n) into v_fmac_f64, so the degree loop has no scalar
-// loads and no waits.  The next group's records are loaded (vector loads)
-// while the current group runs.  Per degree and chain: x Q_l, D_l = l c_l x Q_l
-// - g_l c_{l-1} Q_{l-1} (two FMAs), eight contraction FMAs and the recurrence FMA.
-// ---------------------------------------------------------------------------
-struct VRec {
-    double b, dl, dg;  // beta_{l+1}, l c_l, g_l c_{l-1}
-    double R[8];       // S'r, S'i, T'r, T'i, c S'r, c S'i, c T'r, c T'i
-};
-
-
-template <int K, int PAR, int N, bool NOP, bool FAST>
-__device__ __forceinline__ void vdstep(const VRec &r, const double *x, double *prev, double *cur, const double *cm,
-                                       double (*acc)[2][8]) {
-    double xc[K], D[K], Q[K];
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        xc[j] = x[j] * cur[j];
-        D[j] = 0.0;
-    }
-    // five wait states between a VALU write of the records (or of EXEC in a
-    // rescale) and their first DPP read
-    if (NOP) asm volatile("s_nop 4");
-#pragma unroll
-    for (int j = 0; j < K; ++j) SHTK_FMAC_BC(D[j], r.dl, xc[j], N, "");
-#pragma unroll
-    for (int j = 0; j < K; ++j) SHTK_FMAC_BC(D[j], r.dg, prev[j], N, "-");
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        Q[j] = cur[j];
-        if (!FAST) {
-            D[j] *= cm[j];
-            Q[j] *= cm[j];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        double *A = acc[j][PAR];
-        SHTK_FMAC_BC(A[0], r.R[0], D[j], N, "");
-        SHTK_FMAC_BC(A[1], r.R[1], D[j], N, "");
-        SHTK_FMAC_BC(A[2], r.R[6], Q[j], N, "");
-        SHTK_FMAC_BC(A[3], r.R[7], Q[j], N, "");
-        SHTK_FMAC_BC(A[4], r.R[4], Q[j], N, "");
-        SHTK_FMAC_BC(A[5], r.R[5], Q[j], N, "");
-        SHTK_FMAC_BC(A[6], r.R[2], D[j], N, "");
-        SHTK_FMAC_BC(A[7], r.R[3], D[j], N, "");
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) SHTK_FMAC_BC(xc[j], r.b, prev[j], N, "-");
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        prev[j] = cur[j];
-        cur[j] = xc[j];
-    }
-}
-
-// Steps N = 0 .. 15 of one record group while N < nrem; (l - m) has the parity
-// of N.  Scaled chains are checked every 8 degrees with c_l of the last degree.
-template <int K, bool FAST, int N>
-__device__ __forceinline__ bool vdgroup_from(const VRec &r, cptr<double> qcm, int l0g, int nrem, const double *x,
-                                             double *prev, double *cur, int *kk, double *cm, double (*acc)[2][8]) {
-    if constexpr (N == 16) {
-        return true;
-    } else {
-        if (N >= nrem) return false;
-        vdstep<K, N & 1, N, N == 0 || (!FAST && N == 8), FAST>(r, x, prev, cur, cm, acc);
-        if (!FAST && (N & 7) == 7) rescale<K>(prev, cur, kk, cm, qcm[l0g + N]);
-        return vdgroup_from<K, FAST, N + 1>(r, qcm, l0g, nrem, x, prev, cur, kk, cm, acc);
-    }
-}
-
-// The accumulated sums of the pair block -> Fourier columns of both components
-// (north and south rows by parity), as k_synth_v.
-template <int K, int NW = 4>
-__device__ __forceinline__ void vsynth_out(const LegArgs &a, double (*acc)[2][8], double (*red)[16][64], int w,
-                                           int lane, int pb0, int im, int f) {
-    const int m = im * a.mres, np = a.np;
-    const double mm = (double)m;
-    const double gm = a.g * mfac_of(a.mfac_mode, m);
-    const size_t fo = ((size_t)f * a.nm + im) * a.nlat;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        if constexpr (NW > 1) {
-            if (j > 0) __syncthreads();
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-#pragma unroll
-                for (int r = 0; r < 8; ++r) red[w][8 * q + r][lane] = acc[j][q][r];
-            __syncthreads();
-        }
-        const int p = pb0 + lane + 64 * j;
-        if (w == 0 && p < np) {
-            double e[8], o[8];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                if constexpr (NW > 1) {
-                    e[r] = ((red[0][r][lane] + red[1][r][lane]) + red[2][r][lane]) + red[3][r][lane];
-                    o[r] = ((red[0][8 + r][lane] + red[1][8 + r][lane]) + red[2][8 + r][lane]) + red[3][8 + r][lane];
-                } else {
-                    e[r] = acc[j][0][r];
-                    o[r] = acc[j][1][r];
-                }
-            }
-#pragma unroll
-            for (int r = 2; r < 6; ++r) {
-                e[r] *= mm;
-                o[r] *= mm;
-            }
-            const double sc = gm * (a.wlat ? a.wlat[p] : 1.0);
-            // [0..1] = A, [2..3] = m B, [4..5] = m C, [6..7] = E
-            const double tNr = e[0] + o[0] + (e[3] + o[3]), tNi = e[1] + o[1] - (e[2] + o[2]);
-            const double tSr = -e[0] + o[0] + (e[3] - o[3]), tSi = -e[1] + o[1] - (e[2] - o[2]);
-            const double pNr = -(e[5] + o[5]) + e[6] + o[6], pNi = e[4] + o[4] + e[7] + o[7];
-            const double pSr = -(e[5] - o[5]) - e[6] + o[6], pSi = (e[4] - o[4]) - e[7] + o[7];
-            a.F0[fo + p] = make_double2(tNr * sc, tNi * sc);
-            a.F1[fo + p] = make_double2(pNr * sc, pNi * sc);
-            const int ps = a.nlat - 1 - p;
-            if (ps != p) {
-                a.F0[fo + ps] = make_double2(tSr * sc, tSi * sc);
-                a.F1[fo + ps] = make_double2(pSr * sc, pSi * sc);
-            }
-        }
-    }
-}
-
-// VD: the records are built from the caller's canonical FP64 S and T as they
-// are loaded (LegArgs.vdirect); a template parameter so that neither form
-// branches around its loads (a branch would complete them at its join).
-// NW = 4: the block's 4 waves take the order's segments round-robin and add
-// their sums through LDS (units in order-major order); NW = 1: one wave runs all
-// segments of its (order, pair block, field) with no barrier, units ordered
-// lowest order first for every field (longest work first).
-template <int K, bool VD, int NW>
-__global__ __launch_bounds__(64 * NW) void k_synth_vd(const LegArgs a) {
-    __shared__ double red[NW > 1 ? 4 : 1][16][64];
-    int b, unit;
-    if (!unit_of_block(a.xcd, a.gx, a.gy * a.gz, &unit, &b)) return;
-    const int im = NW > 1 ? unit % a.gy : unit / a.gz, f = NW > 1 ? unit / a.gy : unit % a.gz;
-    if (a.skip_m0 && im == 0) return;  // written by the zonal kernel
-    const int m = im * a.mres;
-    const int lane = threadIdx.x & 63;
-    const int w = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-    const int np = a.np, lmax = a.lmax, ltr = a.ltr;
-    const int pb0 = b * 64 * K, pb1 = min(pb0 + 64 * K, np);
-    double x[K];
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        const int p = pb0 + lane + 64 * j;
-        x[j] = p < np ? a.x[p] : 0.0;
-    }
-    const long long co = as_const(a.coff)[im] - m;
-    const cptr<double> qcm = as_const(a.qcc) + co;
-    const double *qbm = a.qb + co;                              // padded past lmax + 1
-    const double2 *qdm = a.qd + co;                             // entries l = m .. lmax + 1
-    const size_t cbase = (size_t)f * a.spec_fstride + (size_t)(lmax + 1) * m;
-    const double4 *rec = (const double4 *)a.in0 + 2 * cbase;
-    // vdirect: the caller's canonical FP64 S and T, records built as they are loaded
-    const double2 *Sd = (const double2 *)a.in0 + cbase, *Td = (const double2 *)a.in1 + cbase;
-    const double *qcl = a.qcc + co;
-    double acc[K][2][8];
-#pragma unroll
-    for (int j = 0; j < K; ++j)
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int r = 0; r < 8; ++r) acc[j][q][r] = 0.0;
-    const int nseg = nseg_of(lmax, m, DSEG);
-    const int segb = as_const(a.segbase)[im];
-    // record group (segment s, group g) of this lane's degree
-    auto load_rec = [&](VRec &d, int s, int g) {
-        const int l = m + min(s, nseg - 1) * DSEG + 16 * g + (lane & 15);
-        d.b = qbm[l + 1];
-        const double2 dd = qdm[min(l, lmax + 1)];
-        d.dl = dd.x;
-        d.dg = dd.y;
-        const int lc = min(l, lmax);
-        if constexpr (VD) {
-            // raw values only: the products with c_l are formed when the group
-            // starts (a use here would wait for the loads at once)
-            const double2 sv = Sd[lc], tv = Td[lc];
-            d.R[0] = sv.x;
-            d.R[1] = sv.y;
-            d.R[2] = tv.x;
-            d.R[3] = tv.y;
-            d.R[4] = qcl[lc];
-        } else {
-            const double4 r0 = rec[2 * (size_t)lc], r1 = rec[2 * (size_t)lc + 1];
-            d.R[0] = r0.x;
-            d.R[1] = r0.y;
-            d.R[2] = r0.z;
-            d.R[3] = r0.w;
-            d.R[4] = r1.x;
-            d.R[5] = r1.y;
-            d.R[6] = r1.z;
-            d.R[7] = r1.w;
-        }
-    };
-    VRec nr;
-    if (w < nseg) load_rec(nr, w, 0);
-    for (int s = w; s < nseg; s += NW) {
-        const int l0 = m + s * DSEG;
-        if (l0 > ltr) break;
-        const int gs = segb + s;
-        const int pf = as_const(a.pfirst)[gs], pfa = as_const(a.pfast)[gs];
-        const int lstop = min(l0 + DSEG, ltr + 1);
-        if (pb1 <= pf) {
-            if (s + NW < nseg) load_rec(nr, s + NW, 0);
-            continue;
-        }
-        double prev[K], cur[K];
-        int kk[K];
-#pragma unroll
-        for (int j = 0; j < K; ++j) {
-            const int p = pb0 + lane + 64 * j;
-            const bool act = p < np;
-            const size_t q = (size_t)gs * np + (act ? p : 0);
-            prev[j] = act ? a.seedq0[q] : 0.0;
-            cur[j] = act ? a.seedq1[q] : 0.0;
-            kk[j] = act ? a.seedk[q] : 0;
-        }
-        const bool fast = pb0 >= pfa;
-        double cm[K];
-#pragma unroll
-        for (int j = 0; j < K; ++j) cm[j] = kk[j] == 0 ? 1.0 : 0.0;
-        for (int g = 0; g < 4; ++g) {
-            const int l0g = l0 + 16 * g;
-            VRec r = nr;
-            if constexpr (VD) {
-                const double c = r.R[4];
-                r.R[4] = c * r.R[0];
-                r.R[5] = c * r.R[1];
-                r.R[6] = c * r.R[2];
-                r.R[7] = c * r.R[3];
-            }
-            // the next group: this segment's next, or the first of the wave's next segment
-            if (g < 3 && l0g + 16 < lstop) load_rec(nr, s, g + 1);
-            else if (s + NW < nseg) load_rec(nr, s + NW, 0);
-            const bool full = fast ? vdgroup_from<K, true, 0>(r, qcm, l0g, lstop - l0g, x, prev, cur, kk, cm, acc)
-                                   : vdgroup_from<K, false, 0>(r, qcm, l0g, lstop - l0g, x, prev, cur, kk, cm, acc);
-            if (!full || l0g + 16 >= lstop) break;
-        }
-    }
-    vsynth_out<K, NW>(a, acc, red, w, lane, pb0, im, f);
-}
-
 // Prologue of the vector synthesis: per (order, field) and l >= m the record
 // (S', T', c_l S', c_l T') with S' = conv(l, m) S [/ l(l+1)], T' likewise.
 template <typename IT>
@@ -990,25 +740,14 @@ __global__ __launch_bounds__(256) void k_vpole_synth(const LegArgs a, int robert
         }
         return;
     }
-    // order 1: prologue records (S', T', c S', c T'), or with vdirect the caller's S and T
+    // order 1: prologue records (S', T', c S', c T')
     const size_t c1 = (size_t)f * a.spec_fstride + (size_t)(a.lmax + 1);
     const double *rec = (const double *)a.in0 + 8 * c1;
-    const double2 *Sd = (const double2 *)a.in0 + c1, *Td = (const double2 *)a.in1 + c1;
     double v[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const int lt = min(a.ltr, a.lmax);
     for (int l = 1 + (int)threadIdx.x; l <= lt; l += 256) {
         const double h = pole_h(l), hs = (l & 1) ? -h : h;
-        double r[4];
-        if (a.vdirect) {
-            const double2 sv = Sd[l], tv = Td[l];
-            r[0] = sv.x;
-            r[1] = sv.y;
-            r[2] = tv.x;
-            r[3] = tv.y;
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) r[k] = rec[8 * (size_t)l + k];
-        }
+        const double *r = rec + 8 * (size_t)l;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             v[k] = fma(h, r[k], v[k]);
@@ -1030,9 +769,11 @@ __global__ __launch_bounds__(256) void k_vpole_synth(const LegArgs a, int robert
 
 // Analysis: adds the weighted pole rows of order 1 to S_l1, T_l1 (after the
 // Legendre analysis wrote them), S += w [dP Vt - i P/s Vp], T += w [i P/s Vt + dP Vp];
-// conv (optional): the outputs are in the plan's convention, divide by it.
+// conv (optional): the outputs are in the plan's convention, divided (conv_div) or
+// multiplied by it.
 template <typename OT>
-__global__ __launch_bounds__(256) void k_vpole_anal(const LegArgs a, double wpole, const double *conv) {
+__global__ __launch_bounds__(256) void k_vpole_anal(const LegArgs a, double wpole, const double *conv,
+                                                    int conv_div) {
     const int f = blockIdx.x, nlat = a.nlat;
     const size_t fo = ((size_t)f * a.nm + 1) * nlat;
     const double2 tN = a.F0[fo], pN = a.F1[fo], tS = a.F0[fo + nlat - 1], pS = a.F1[fo + nlat - 1];
@@ -1045,7 +786,7 @@ __global__ __launch_bounds__(256) void k_vpole_anal(const LegArgs a, double wpol
         const double dN = -h, qN = -h, dS = -hs, qS = hs;  // dP/dtheta and P/sin(theta)
         double sc = gm;
         if (a.ll1_mode) sc /= (double)l * (l + 1);
-        if (conv) sc /= conv[(size_t)(a.lmax + 1) + l];
+        if (conv) sc = conv_div ? sc / conv[(size_t)(a.lmax + 1) + l] : sc * conv[(size_t)(a.lmax + 1) + l];
         const double sr = dN * tN.x + qN * pN.y + dS * tS.x + qS * pS.y;
         const double si = dN * tN.y - qN * pN.x + dS * tS.y - qS * pS.x;
         const double tr = -qN * tN.y + dN * pN.x - qS * tS.y + dS * pS.x;
@@ -1062,6 +803,8 @@ __global__ __launch_bounds__(256) void k_vpole_anal(const LegArgs a, double wpol
 // ---------------------------------------------------------------------------
 struct Item {
     int gs, pbi, im, s, m, l0, lend, lstop, pb0, pb1, pstart, f;
+    long long co;  // table entry of degree l: co + l
+    bool one;      // order 0 on the tables of order 1 (LegArgs.m0_one)
     bool fast;
 };
 
@@ -1098,7 +841,11 @@ __device__ __forceinline__ Item make_item_at(const LegArgs &a, int item, int pbl
     it.im = as_const(a.segm)[it.gs];
     it.s = it.gs - as_const(a.segbase)[it.im];
     it.m = it.im * a.mres;
-    it.l0 = it.m + it.s * a.seg;
+    it.one = a.m0_one && it.im == 0;
+    const int mt = it.one ? 1 : it.m;
+    if (it.one) it.gs = min(as_const(a.segbase)[1] + it.s, a.nseg_total - 1);
+    it.co = as_const(a.coff)[it.one ? 1 : it.im] - mt;
+    it.l0 = mt + it.s * a.seg;
     it.lend = min(it.l0 + a.seg, a.lmax + 1);
     it.lstop = min(it.lend, a.ltr + 1);
     it.pb0 = it.pbi * pblk;
@@ -1113,6 +860,7 @@ template <int K, bool FAST, typename OT>
 __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, double *red, OT *col, int lane) {
     const int np = a.np, nlat = a.nlat;
     const double2 *Fi = a.F0 + ((size_t)it.f * a.nm + it.im) * nlat;
+    const double *wlat = it.one ? a.wlat0 : a.wlat;
     double x[K], prev[K], cur[K], gpr[K], gpi[K], gmr[K], gmi[K];
     int kk[K];
 #pragma unroll
@@ -1131,7 +879,7 @@ __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, dou
             FN = Fi[p];
             const int ps = nlat - 1 - p;
             if (ps != p) FS = Fi[ps];
-            wl = a.wlat ? a.wlat[p] : 1.0;
+            wl = wlat ? wlat[p] : 1.0;
         }
         gpr[j] = wl * (FN.x + FS.x);
         gpi[j] = wl * (FN.y + FS.y);
@@ -1140,7 +888,7 @@ __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, dou
     }
     const double gm = a.g * mfac_of(a.mfac_mode, it.m);
     const int nst = it.lstop - it.l0;
-    const long long co = as_const(a.coff)[it.im] - it.m;
+    const long long co = it.co;
     const cptr<double> qcm = as_const(a.qcc) + co;
     const int o = lane & 15, qg = lane >> 4;
     // Checked path: ke = -4096 x scale count, so ldexp(cur, ke) is the lane's
@@ -1204,7 +952,7 @@ __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, dou
         sum += __shfl_xor(sum, 32);
         const int t = c0 + (o >> 1);
         if (qg == 0 && t < nst) {
-            const double v = gm * qcm[it.l0 + t] * sum;
+            const double v = gm * (a.raw_q ? 1.0 : qcm[it.l0 + t]) * sum;
             OT *dst = col + 2 * (size_t)(it.l0 + t) + (o & 1);
             if (a.atomic)
                 atomicAdd(dst, (OT)v);
@@ -1415,7 +1163,7 @@ __device__ __forceinline__ void anal_vw_run(const LegArgs &a, const Item &it, do
     const double gm = a.g * mfac_of(a.mfac_mode, it.m);
     const double mm = (double)it.m;
     const int nst = it.lstop - it.l0;
-    const long long co = as_const(a.coff)[it.im] - it.m;
+    const long long co = it.co;
     const cptr<double> qcm = as_const(a.qcc) + co;
     // per-degree records in VGPRs, broadcast by DPP (no scalar loads in the loop):
     // lane 16 r + n holds (beta_{l+1}, l c_l, g_l c_{l-1}) of degree l0 + c16 + n
@@ -1565,15 +1313,7 @@ static void launch_synth_k(LegArgs a, int nfields, int vector, hipStream_t st) {
     const dim3 grid(grid_for_units(a.xcd, a.gx, a.gy * a.gz));
     if (vector) {
         // inputs are the FP64 prologue records of k_vspec_prep
-        if (a.seg == DSEG && a.vwaves == 1) {
-            if (a.vdirect) hipLaunchKernelGGL((k_synth_vd<K, true, 1>), grid, dim3(64), 0, st, a);
-            else hipLaunchKernelGGL((k_synth_vd<K, false, 1>), grid, dim3(64), 0, st, a);
-        } else if (a.seg == DSEG && a.vdirect)
-            hipLaunchKernelGGL((k_synth_vd<K, true, 4>), grid, dim3(256), 0, st, a);
-        else if (a.seg == DSEG)
-            hipLaunchKernelGGL((k_synth_vd<K, false, 4>), grid, dim3(256), 0, st, a);
-        else
-            hipLaunchKernelGGL((k_synth_v<K>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_synth_v<K>), grid, dim3(256), 0, st, a);
     } else {
         if (a.seg == DSEG && (long long)a.gx * a.gy * a.gz >= a.s1w_units)
             hipLaunchKernelGGL((k_synth_d<K, 1>), grid, dim3(64), 0, st, a);
@@ -1680,11 +1420,12 @@ hipError_t launch_vpole_synth(const LegArgs &a, int nfields, int robert, double 
     return hipGetLastError();
 }
 
-hipError_t launch_vpole_anal(const LegArgs &a, int nfields, double wpole, const double *conv, hipStream_t st) {
+hipError_t launch_vpole_anal(const LegArgs &a, int nfields, double wpole, const double *conv, int conv_div,
+                             hipStream_t st) {
     if (a.io_f32)
-        hipLaunchKernelGGL(k_vpole_anal<float>, dim3((unsigned)nfields), dim3(256), 0, st, a, wpole, conv);
+        hipLaunchKernelGGL(k_vpole_anal<float>, dim3((unsigned)nfields), dim3(256), 0, st, a, wpole, conv, conv_div);
     else
-        hipLaunchKernelGGL(k_vpole_anal<double>, dim3((unsigned)nfields), dim3(256), 0, st, a, wpole, conv);
+        hipLaunchKernelGGL(k_vpole_anal<double>, dim3((unsigned)nfields), dim3(256), 0, st, a, wpole, conv, conv_div);
     return hipGetLastError();
 }
 

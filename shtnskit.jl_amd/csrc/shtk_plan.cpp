@@ -297,6 +297,7 @@ struct DeviceGuard {
 struct WsLayout {
     size_t f_bytes, spec_bytes, total;
     size_t zonal_off;  // vector: FP64 sums of the order-0 rewrite of the analysis
+    size_t edge_off;   // vector: coefficients past the segments (launch_vcoef)
 };
 
 WsLayout ws_layout(const shtk_plan *p, int nf, int vector) {
@@ -311,6 +312,8 @@ WsLayout ws_layout(const shtk_plan *p, int nf, int vector) {
     if (vector) L.total = std::max(L.total, 2 * L.f_bytes + 4 * L.spec_bytes);
     L.zonal_off = L.total;
     if (vector) L.total += al(sizeof(double) * 4 * (size_t)nf * ((p->np + 63) / 64) * (p->d.lmax + 1));
+    L.edge_off = L.total;
+    if (vector) L.total += al(sizeof(double2) * 4 * (size_t)nf * p->nseg_total);
     return L;
 }
 
@@ -360,7 +363,8 @@ hipError_t timed(shtk_plan *p, const char *name, hipStream_t st, F &&launch) {
 struct SideStream {
     shtk_plan *p;
     hipStream_t st, s;
-    SideStream(shtk_plan *p_, hipStream_t st_) : p(p_), st(st_), s(st_) {
+    explicit SideStream(shtk_plan *p_, hipStream_t st_, bool use = true) : p(p_), st(st_), s(st_) {
+        if (!use) return;
         if (!p->side) {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
             if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
@@ -517,6 +521,10 @@ int norm_ltr(const shtk_plan *p, int ltr, int *out) {
     return SHTK_OK;
 }
 
+// Last degree the segments cover: the vector transforms of 64-degree plans run as
+// scalar ones of degree lmax + 1.
+int seg_lmax(const shtk_plan *p) { return p->d.lmax + (p->seg == shtk::DSEG ? 1 : 0); }
+
 // Split-precision tables: quarter seeds and per-pair exponents (one kernel,
 // first use only) and the chunk offsets of every order.
 int ensure_oz_tables(shtk_plan *p, hipStream_t st) {
@@ -552,7 +560,7 @@ int ensure_oz_tables(shtk_plan *p, hipStream_t st) {
             const int s0 = r * nseg / nr, s1 = (r + 1) * nseg / nr;
             runs.push_back(make_int4(im, gs + s0, s1 - s0, 0));
         }
-        gs += nseg;
+        gs += (seg_lmax(p) - im * p->d.mres + p->seg) / p->seg;
     }
     RC_TRY(upload(&p->oz_run, runs, "split tables"));
     p->oz_nrun = (int)runs.size();
@@ -828,6 +836,91 @@ int ensure_zseed(shtk_plan *p, hipStream_t st) {
     return SHTK_OK;
 }
 
+// The vector transforms of 64-degree plans as scalar ones of degree lmax + 1 (the
+// tables and segments reach there); spectral columns of lmax + 2 entries.
+shtk::LegArgs vscalar_args(const shtk_plan *p, int ltr) {
+    shtk::LegArgs a = base_args(p, ltr + 1);
+    a.lmax = p->d.lmax + 1;
+    a.spec_fstride = (long long)(p->d.lmax + 2) * (p->d.mmax + 1);
+    return a;
+}
+
+// Order 0 of a vector transform without its own kernel (launch_vcoef): where the
+// orders include 1.
+bool m0_on_one(const shtk_plan *p, const Job &j) {
+    return p->seg == shtk::DSEG && j.pole_fix == 1 && j.ltr >= 1 && p->d.mres == 1 && p->nm >= 2;
+}
+
+// The phi transforms of a vector pair: one launch where the Fourier columns of the
+// second component follow the first's.
+hipError_t launch_fft_pair(shtk_plan *p, const Job &j, double2 *F0, double2 *F1, void *const *grids, int nf, int dtype,
+                           int inverse, hipStream_t st) {
+    shtk::FftArgs fa = fft_args(p);
+    fa.F = F0;
+    fa.grid = grids[0];
+    fa.io_f32 = dtype == SHTK_F32;
+    fa.mode = j.fft_mode;
+    const bool cplx = inverse ? j.cplx_out : j.cplx_in;
+    const bool one = j.vector && F1 == F0 + (size_t)nf * p->nm * p->d.nlat;
+    if (one) {
+        fa.grid1 = grids[1];
+        fa.nf0 = nf;
+        nf *= 2;
+    }
+    for (int q = 0; q <= (j.vector && !one); ++q) {
+        if (q == 1) {
+            fa.F = F1;
+            fa.grid = grids[1];
+        }
+        hipError_t e = timed(p, j.fft_name, st, [&] {
+            return cplx ? shtk::launch_fft_cplx(fa, nf, inverse, st) : shtk::launch_fft(fa, nf, inverse, st);
+        });
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// Legendre stage of a vector synthesis: a.in0 holds the scalar coefficients of
+// launch_vcoef (64-degree plans; theta fields, then phi fields, from a.F0 on) or
+// the records of k_vspec_prep.
+hipError_t leg_synth_vector(const shtk_plan *p, const shtk::LegArgs &a, int nf, hipStream_t st) {
+    return p->seg == shtk::DSEG ? shtk::launch_fields_synth(a, 2 * nf, st)
+                                : shtk::launch_leg_synth(a, nf, 1, p->vsynth_chains, st);
+}
+
+// Records of the orders 0 and 1 for launch_vpole_synth, into rec once the scalar
+// coefficients there are used up; a becomes the arguments it takes.
+int vpole_records(const shtk_plan *p, const Job &j, shtk::LegArgs &a, const void *S, const void *T, void *rec, int nf,
+                  int dtype, hipStream_t st) {
+    const long long fs = (long long)(p->d.lmax + 1) * (p->d.mmax + 1);
+    HIP_TRY(shtk::launch_vspec_prep(S, T, (double *)rec, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale,
+                                    j.conv_div, j.ll1_mode, p->qcc, p->coff, p->d.lmax, p->d.mres, std::min(2, p->nm),
+                                    fs, nf, st),
+            "pole records");
+    a.in0 = rec;
+    a.lmax = p->d.lmax;
+    a.ltr = j.ltr;
+    a.spec_fstride = fs;
+    return SHTK_OK;
+}
+
+// Legendre stage of a scalar analysis: groups of fields share the recurrence
+// (shtk_fields.hip), the fields left over take the single-field kernel.
+int leg_anal_scalar(shtk_plan *p, shtk::LegArgs a, int nf, const char *name, hipStream_t st) {
+    const int ngrp = shtk::fields_anal_count(a, nf), nrest = nf - ngrp;
+    if (ngrp > 0) {
+        HIP_TRY(timed(p, name, st, [&] { return shtk::launch_fields_anal(a, ngrp, st); }), "Legendre analysis launch");
+        a.F0 += (size_t)ngrp * p->nm * p->d.nlat;
+        a.out0 = (char *)a.out0 + (size_t)ngrp * a.spec_fstride * (a.io_f32 ? 8 : 16);
+    }
+    if (nrest == 0) return SHTK_OK;
+    a.atomic = p->np > 512;  // pairs per work item (launch_leg_anal)
+    if (a.atomic)
+        HIP_TRY(shtk::launch_zero(a.out0, (size_t)nrest * a.spec_fstride * (a.io_f32 ? 8 : 16), st), "output clear");
+    HIP_TRY(timed(p, name, st, [&] { return shtk::launch_leg_anal(a, nrest, 0, st); }), "Legendre analysis launch");
+    return SHTK_OK;
+}
+
 // spectral -> grid: [convert] -> Legendre synthesis -> inverse phi FFT
 // ext_ws: a caller-provided workspace of ext_bytes (nothing is allocated), or
 // nullptr for the plan's own (grown on demand).
@@ -852,7 +945,6 @@ int run_to_grid(shtk_plan *p, const Job &j, const void *s0, const void *s1, void
     a.in0 = s0;
     a.in1 = s1;
     a.io_f32 = dtype == SHTK_F32;
-    a.vwaves = p->vsynth_waves;
     if (!j.vector && j.prec == SHTK_PREC_FP64 && p->canonical && !a.io_f32 && p->seg == shtk::DSEG) {
         // scalar FP64 synthesis of canonical FP64 coefficients: the kernel applies
         // c_l (Q form) as it loads them
@@ -866,11 +958,18 @@ int run_to_grid(shtk_plan *p, const Job &j, const void *s0, const void *s1, void
                 "coefficient scaling");
         a.in0 = dst;
         a.io_f32 = 0;
-    } else if (j.vector && j.prec == SHTK_PREC_FP64 && p->canonical && !a.io_f32 && !j.ll1_mode &&
-               p->seg == shtk::DSEG) {
-        // vector FP64 synthesis of canonical FP64 S, T: the kernel builds its records
-        // (S, T, c_l S, c_l T) as it loads them
-        a.vdirect = 1;
+    } else if (j.vector && p->seg == shtk::DSEG) {
+        // vector FP64 synthesis as 2 nf scalar ones of degree lmax + 1
+        F1 = F0 + (size_t)nf * p->nm * p->d.nlat;
+        shtk::LegArgs v = vscalar_args(p, j.ltr);
+        v.m0_one = m0_on_one(p, j);
+        v.wlat0 = p->d.robert_form ? p->s : nullptr;
+        HIP_TRY(shtk::launch_vcoef(s0, s1, spec, ws + L.edge_off, a.io_f32, p->canonical ? nullptr : p->convscale, j.conv_div,
+                                   j.ll1_mode, v, nf, st),
+                "vector coefficient combination");
+        a = v;
+        a.in0 = spec;
+        a.edge = (const double2 *)(ws + L.edge_off);
     } else if (j.vector && j.prec == SHTK_PREC_FP64) {
         // vector FP64 synthesis: records (S', T', c_l S', c_l T') with the convention
         // map and the l(l+1) factor applied
@@ -911,13 +1010,14 @@ int run_to_grid(shtk_plan *p, const Job &j, const void *s0, const void *s1, void
         HIP_TRY(timed(p, "f32_synth", st, [&] { return shtk::launch_f32_synth(o, st); }),
                 "FP32 synthesis launch");
     } else {
-        // vector: the order-0 rows come from the zonal kernel, on the side stream
-        // beside the main kernel (which skips order 0); disjoint output columns
-        const bool zonal = j.vector && j.pole_fix == 1 && j.ltr >= 1;
+        // vector: without order 1 (m0_on_one) the order-0 rows come from the zonal kernel,
+        // on the side stream beside the main kernel (which skips order 0); disjoint output
+        // columns
+        const bool zonal = j.vector && j.pole_fix == 1 && j.ltr >= 1 && !a.m0_one;
         a.skip_m0 = zonal;
         if (zonal) {
             RC_TRY(ensure_zseed(p, st));
-            shtk::MlArgs z = zonal_args(p, j.ltr, a.spec_fstride);
+            shtk::MlArgs z = zonal_args(p, j.ltr, (long long)(p->d.lmax + 1) * (p->d.mmax + 1));
             z.io_f32 = dtype == SHTK_F32;
             z.conv = p->canonical ? nullptr : p->convscale;  // order 0: index l
             z.g = j.g;
@@ -928,37 +1028,29 @@ int run_to_grid(shtk_plan *p, const Job &j, const void *s0, const void *s1, void
             SideStream side(p, st);
             HIP_TRY(timed(p, "leg_synth_sphtor_m0", side.s, [&] { return shtk::launch_ml_synth(z, nf, side.s); }),
                     "order-0 rows launch");
-            HIP_TRY(timed(p, j.leg_name, st,
-                          [&] { return shtk::launch_leg_synth(a, nf, 1, p->vsynth_chains, st); }),
+            HIP_TRY(timed(p, j.leg_name, st, [&] { return leg_synth_vector(p, a, nf, st); }),
                     "Legendre synthesis launch");
             HIP_TRY(side.join(), "order-0 rows join");
         } else if (!j.vector && shtk::fields_synth_ok(a, nf)) {
             HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_fields_synth(a, nf, st); }),
                     "Legendre synthesis launch");
+        } else if (j.vector) {
+            HIP_TRY(timed(p, j.leg_name, st, [&] { return leg_synth_vector(p, a, nf, st); }),
+                    "Legendre synthesis launch");
         } else {
             HIP_TRY(timed(p, j.leg_name, st,
-                          [&] { return shtk::launch_leg_synth(a, nf, j.vector, j.vector ? p->vsynth_chains : p->synth_chains, st); }),
+                          [&] { return shtk::launch_leg_synth(a, nf, 0, p->synth_chains, st); }),
                     "Legendre synthesis launch");
         }
         const bool zero_rows = j.pole_fix == 1 && p->d.robert_form;  // Robert rows are sin(theta) V
-        if (j.pole_fix && p->poles && (zero_rows || (p->d.mres == 1 && p->d.mmax >= 1)))
+        if (j.pole_fix && p->poles && (zero_rows || (p->d.mres == 1 && p->d.mmax >= 1))) {
+            if (p->seg == shtk::DSEG) RC_TRY(vpole_records(p, j, a, s0, s1, spec, nf, dtype, st));
             HIP_TRY(shtk::launch_vpole_synth(a, nf, zero_rows, j.pole_fix == 2 ? p->hw[0] * p->scale_phi : 1.0, st),
                     "pole rows launch");
+        }
     }
     void *grids[2] = {g0, g1};
-    for (int q = 0; q <= j.vector; ++q) {
-        shtk::FftArgs fa = fft_args(p);
-        fa.F = q == 0 ? F0 : F1;
-        fa.grid = grids[q];
-        fa.io_f32 = dtype == SHTK_F32;
-        fa.mode = j.fft_mode;
-        if (j.cplx_out)
-            HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft_cplx(fa, nf, 1, st); }),
-                    "phi synthesis launch");
-        else
-            HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft(fa, nf, 1, st); }),
-                    "phi synthesis launch");
-    }
+    HIP_TRY(launch_fft_pair(p, j, F0, F1, grids, nf, dtype, 1, st), "phi synthesis launch");
     return SHTK_OK;
 }
 
@@ -972,22 +1064,12 @@ int run_to_spec(shtk_plan *p, const Job &j, const void *g0, const void *g1, void
     const WsLayout L = ws_layout(p, nf, j.vector);
     RC_TRY(ensure_ws(p, L.total));
     char *ws = (char *)p->ws;
-    double2 *F0 = (double2 *)ws, *F1 = (double2 *)(ws + L.f_bytes);
+    const bool vscalar = j.vector && p->seg == shtk::DSEG;  // as 2 nf scalar fields, one array
+    double2 *F0 = (double2 *)ws;
+    double2 *F1 = vscalar ? F0 + (size_t)nf * p->nm * p->d.nlat : (double2 *)(ws + L.f_bytes);
     char *spec = ws + (j.vector ? 2 : 1) * L.f_bytes;
-    const void *grids[2] = {g0, g1};
-    for (int q = 0; q <= j.vector; ++q) {
-        shtk::FftArgs fa = fft_args(p);
-        fa.F = q == 0 ? F0 : F1;
-        fa.grid = (void *)grids[q];
-        fa.io_f32 = dtype == SHTK_F32;
-        fa.mode = j.fft_mode;
-        if (j.cplx_in)
-            HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft_cplx(fa, nf, 0, st); }),
-                    "phi analysis launch");
-        else
-            HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft(fa, nf, 0, st); }),
-                    "phi analysis launch");
-    }
+    void *grids[2] = {(void *)g0, (void *)g1};
+    HIP_TRY(launch_fft_pair(p, j, F0, F1, grids, nf, dtype, 0, st), "phi analysis launch");
     shtk::LegArgs a = base_args(p, j.ltr);
     a.F0 = F0;
     a.F1 = F1;
@@ -1034,52 +1116,86 @@ int run_to_spec(shtk_plan *p, const Job &j, const void *g0, const void *g1, void
                     "coefficient conversion");
         return SHTK_OK;
     }
-    const int pblk = j.vector ? p->vanal_pblk : 512;  // pairs per analysis work item (launch_leg_anal)
-    a.apblk = pblk;
-    // scalar batches: groups of fields share the recurrence (shtk_fields.hip); the
-    // fields left over take the single-field kernel below
-    const int ngrp = j.vector ? 0 : shtk::fields_anal_count(a, nf), nrest = nf - ngrp;
-    if (ngrp > 0) {
-        HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_fields_anal(a, ngrp, st); }),
-                "Legendre analysis launch");
-        a.F0 += (size_t)ngrp * p->nm * p->d.nlat;
-        a.out0 = (char *)a.out0 + (size_t)ngrp * a.spec_fstride * (a.io_f32 ? 8 : 16);
-    }
-    a.atomic = p->np > pblk;
-    if (a.atomic && nrest > 0) {
-        const size_t bytes = (size_t)nrest * a.spec_fstride * (a.io_f32 ? 8 : 16);
-        void *outs[2] = {a.out0, a.out1};
-        for (int q = 0; q <= j.vector; ++q)
-            HIP_TRY(shtk::launch_zero(outs[q], bytes, st), "output clear");
-    }
-    const bool zonal = j.vector && j.pole_fix == 1 && j.ltr >= 1;
-    if (zonal) {
-        // order 0 from the zonal kernel on the side stream, beside the main kernel
-        // (which skips it); the convention map of order 0 follows with the rest
-        // (non-canonical plans)
-        a.skip_m0 = 1;
-        RC_TRY(ensure_zseed(p, st));
-        shtk::MlArgs z = zonal_args(p, j.ltr, a.spec_fstride);
-        z.io_f32 = a.io_f32;
-        z.g = j.g;
-        z.in0 = F0;
-        z.in1 = F1;
-        z.out0 = a.out0;
-        z.out1 = a.out1;
-        z.acc = (double *)(ws + L.zonal_off);
-        SideStream side(p, st);
-        HIP_TRY(timed(p, "leg_anal_sphtor_m0", side.s, [&] { return shtk::launch_ml_anal(z, nf, side.s); }),
-                "order-0 rows launch");
+    if (!j.vector) {
+        RC_TRY(leg_anal_scalar(p, a, nf, j.leg_name, st));
+    } else if (vscalar) {
+        // two scalar analyses with the weights of s V, then the combination of their sums;
+        // without order 1 (m0_on_one) order 0 comes from the zonal kernel on the side stream,
+        // beside the main kernels
+        const bool zonal = j.pole_fix == 1 && j.ltr >= 1 && !m0_on_one(p, j);
+        const double *conv = p->canonical ? nullptr : p->convscale;
+        shtk::LegArgs v = vscalar_args(p, j.ltr);
+        v.F0 = F0;
+        v.wlat = j.wlat;
+        v.g = j.g;
+        v.mfac_mode = j.mfac_mode;
+        v.out0 = spec;
+        v.raw_q = 1;
+        v.skip_m0 = zonal;
+        v.m0_one = m0_on_one(p, j);
+        v.wlat0 = p->d.robert_form ? p->winvs : p->wscaled;
+        if (zonal) RC_TRY(ensure_zseed(p, st));  // before the fork
+        SideStream side(p, st, zonal);
+        if (zonal) {
+            shtk::MlArgs z = zonal_args(p, j.ltr, a.spec_fstride);
+            z.io_f32 = dtype == SHTK_F32;
+            z.conv = conv;  // order 0: index l
+            z.g = j.g;
+            z.in0 = F0;
+            z.in1 = F1;
+            z.out0 = s0;
+            z.out1 = s1;
+            z.acc = (double *)(ws + L.zonal_off);
+            HIP_TRY(timed(p, "leg_anal_sphtor_m0", side.s, [&] { return shtk::launch_ml_anal(z, nf, side.s); }),
+                    "order-0 rows launch");
+        }
+        RC_TRY(leg_anal_scalar(p, v, 2 * nf, j.leg_name, st));
+        HIP_TRY(shtk::launch_vout(spec, s0, s1, dtype == SHTK_F32, conv, j.conv_div, j.ll1_mode, zonal, v, nf, st),
+                "vector coefficient combination");
+        HIP_TRY(side.join(), "order-0 rows join");
+        if (j.pole_fix && p->poles && p->d.mres == 1 && p->d.mmax >= 1) {
+            a.out0 = s0;
+            a.out1 = s1;
+            a.io_f32 = dtype == SHTK_F32;
+            HIP_TRY(shtk::launch_vpole_anal(a, nf, j.pole_fix == 2 ? 1.0 : p->hw[0] * p->scale_phi, conv, j.conv_div,
+                                            st),
+                    "pole rows launch");
+        }
+        return SHTK_OK;
+    } else {
+        a.apblk = p->vanal_pblk;  // pairs per analysis work item (launch_leg_anal)
+        a.atomic = p->np > a.apblk;
+        if (a.atomic) {
+            const size_t bytes = (size_t)nf * a.spec_fstride * (a.io_f32 ? 8 : 16);
+            void *outs[2] = {a.out0, a.out1};
+            for (void *o : outs) HIP_TRY(shtk::launch_zero(o, bytes, st), "output clear");
+        }
+        const bool zonal = j.pole_fix == 1 && j.ltr >= 1;
+        if (zonal) RC_TRY(ensure_zseed(p, st));  // before the fork
+        SideStream side(p, st, zonal);
+        if (zonal) {
+            // order 0 from the zonal kernel on the side stream, beside the main kernel
+            // (which skips it); the convention map of order 0 follows with the rest
+            // (non-canonical plans)
+            a.skip_m0 = 1;
+            shtk::MlArgs z = zonal_args(p, j.ltr, a.spec_fstride);
+            z.io_f32 = a.io_f32;
+            z.g = j.g;
+            z.in0 = F0;
+            z.in1 = F1;
+            z.out0 = a.out0;
+            z.out1 = a.out1;
+            z.acc = (double *)(ws + L.zonal_off);
+            HIP_TRY(timed(p, "leg_anal_sphtor_m0", side.s, [&] { return shtk::launch_ml_anal(z, nf, side.s); }),
+                    "order-0 rows launch");
+        }
         HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_leg_anal(a, nf, 1, st); }),
                 "Legendre analysis launch");
         HIP_TRY(side.join(), "order-0 rows join");
-    } else if (nrest > 0) {
-        HIP_TRY(timed(p, j.leg_name, st, [&] { return shtk::launch_leg_anal(a, nrest, j.vector, st); }),
-                "Legendre analysis launch");
+        if (j.pole_fix && p->poles && p->d.mres == 1 && p->d.mmax >= 1)
+            HIP_TRY(shtk::launch_vpole_anal(a, nf, j.pole_fix == 2 ? 1.0 : p->hw[0] * p->scale_phi, nullptr, 1, st),
+                    "pole rows launch");
     }
-    if (j.pole_fix && p->poles && p->d.mres == 1 && p->d.mmax >= 1)
-        HIP_TRY(shtk::launch_vpole_anal(a, nf, j.pole_fix == 2 ? 1.0 : p->hw[0] * p->scale_phi, nullptr, st),
-                "pole rows launch");
     if (!p->canonical) {
         void *dst[2] = {s0, s1};
         for (int q = 0; q <= j.vector; ++q)
@@ -1110,7 +1226,6 @@ int ensure_vshadow(shtk_plan *p) {
     s->synth_chains = p->synth_chains;
     s->vsynth_chains = p->vsynth_chains;
     s->vanal_pblk = p->vanal_pblk;
-    s->vsynth_waves = p->vsynth_waves;
     s->ssynth_1w_units = p->ssynth_1w_units;
     s->fft_tile = p->fft_tile;
     s->oz_run_len = p->oz_run_len;
@@ -1173,36 +1288,32 @@ int run_vsplit_to_grid(shtk_plan *p, const Job &j, const void *S, const void *T,
     // result, after the split prologues have consumed C.
     const int m_lo = std::max(16, (p->d.lmax + 1) / 32);
     const int nm_lo = std::min(p->nm, (m_lo + p->d.mres - 1) / p->d.mres);
-    HIP_TRY(shtk::launch_vspec_prep(S, T, C, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div,
-                                    0, p->qcc, p->coff, p->d.lmax, p->d.mres, nm_lo, in_fs, nf, st),
-            "coefficient scaling");
-    shtk::LegArgs a = base_args(p, j.ltr);
+    shtk::LegArgs a = p->seg == shtk::DSEG ? vscalar_args(p, j.ltr) : base_args(p, j.ltr);
+    a.nm_run = nm_lo;
+    if (p->seg == shtk::DSEG)
+        HIP_TRY(shtk::launch_vcoef(S, T, C, ws + L.edge_off, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div, 0,
+                                   a, nf, st),
+                "vector coefficient combination");
+    else
+        HIP_TRY(shtk::launch_vspec_prep(S, T, C, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div,
+                                        0, p->qcc, p->coff, p->d.lmax, p->d.mres, nm_lo, in_fs, nf, st),
+                "coefficient scaling");
     a.in0 = C;
+    if (p->seg == shtk::DSEG) a.edge = (const double2 *)(ws + L.edge_off);
     a.F0 = F0;
     a.F1 = F1;
     a.wlat = nullptr;  // sin(theta) V, as the split result
     a.g = j.g;
-    a.nm_run = nm_lo;
-    HIP_TRY(timed(p, "leg_synth_sphtor_low", st, [&] { return shtk::launch_leg_synth(a, nf, 1, p->vsynth_chains, st); }),
+    HIP_TRY(timed(p, "leg_synth_sphtor_low", st, [&] { return leg_synth_vector(p, a, nf, st); }),
             "Legendre synthesis launch");
     // grids with poles: order-1 pole rows from the limits (the phi transform divides
     // those rows by 1), Robert form: every pole row zero
-    if (p->poles && (p->d.robert_form || (p->d.mres == 1 && p->d.mmax >= 1)))
+    if (p->poles && (p->d.robert_form || (p->d.mres == 1 && p->d.mmax >= 1))) {
+        if (p->seg == shtk::DSEG) RC_TRY(vpole_records(p, j, a, S, T, C, nf, dtype, st));
         HIP_TRY(shtk::launch_vpole_synth(a, nf, p->d.robert_form, 1.0, st), "pole rows launch");
-    void *grids[2] = {Vt, Vp};
-    for (int q = 0; q < 2; ++q) {
-        shtk::FftArgs fa = fft_args(p);
-        fa.F = q == 0 ? F0 : F1;
-        fa.grid = grids[q];
-        fa.io_f32 = dtype == SHTK_F32;
-        fa.mode = j.fft_mode;
-        if (j.cplx_out)
-            HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft_cplx(fa, nf, 1, st); }),
-                    "phi synthesis launch");
-        else
-            HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft(fa, nf, 1, st); }),
-                    "phi synthesis launch");
     }
+    void *grids[2] = {Vt, Vp};
+    HIP_TRY(launch_fft_pair(p, j, F0, F1, grids, nf, dtype, 1, st), "phi synthesis launch");
     return SHTK_OK;
 }
 
@@ -1221,15 +1332,8 @@ int run_vsplit_to_spec(shtk_plan *p, const Job &j, const void *Vt, const void *V
                                                    : oz_ws_bytes(s, 2 * nf, false)));
     char *ws = (char *)p->ws;
     double2 *F0 = (double2 *)ws, *F1 = F0 + (size_t)nf * p->nm * p->d.nlat;
-    const void *grids[2] = {Vt, Vp};
-    for (int q = 0; q < 2; ++q) {
-        shtk::FftArgs fa = fft_args(p);
-        fa.F = q == 0 ? F0 : F1;
-        fa.grid = (void *)grids[q];
-        fa.io_f32 = dtype == SHTK_F32;
-        fa.mode = j.fft_mode;
-        HIP_TRY(timed(p, j.fft_name, st, [&] { return shtk::launch_fft(fa, nf, 0, st); }), "phi analysis launch");
-    }
+    void *grids[2] = {(void *)Vt, (void *)Vp};
+    HIP_TRY(launch_fft_pair(p, j, F0, F1, grids, nf, dtype, 0, st), "phi analysis launch");
     double *G = (double *)(ws + 2 * L.f_bytes);
     const long long out_fs = (long long)(p->d.lmax + 1) * (p->d.mmax + 1);
     const long long g_fs = (long long)(p->d.lmax + 2) * (p->d.mmax + 1);
@@ -1257,7 +1361,7 @@ int run_vsplit_to_spec(shtk_plan *p, const Job &j, const void *Vt, const void *V
         a.out1 = T;
         a.io_f32 = dtype == SHTK_F32;
         a.spec_fstride = out_fs;
-        HIP_TRY(shtk::launch_vpole_anal(a, nf, p->hw[0] * p->scale_phi, p->canonical ? nullptr : p->convscale, st),
+        HIP_TRY(shtk::launch_vpole_anal(a, nf, p->hw[0] * p->scale_phi, p->canonical ? nullptr : p->convscale, 1, st),
                 "pole rows launch");
     }
     return SHTK_OK;
@@ -1675,7 +1779,7 @@ static int plan_tables(shtk_plan *p) {
         const int m = im * d.mres;
         coff[im] = (long long)ab.size();
         segbase[im] = nseg_total;
-        const int nseg = (lmax - m + S) / S;
+        const int nseg = (seg_lmax(p) - m + S) / S;
         for (int q = 0; q < nseg; ++q) segm.push_back(im);
         nseg_total += nseg;
         std::vector<double> a(lmax + 2 - m + 1, 0.0), b(lmax + 2 - m + 1, 0.0);
@@ -1705,7 +1809,7 @@ static int plan_tables(shtk_plan *p) {
             const double gl = (l > 0 && l > m)
                                   ? std::sqrt((2.0 * l + 1.0) * ((double)l * l - (double)m * m) / (2.0 * l - 1.0))
                                   : 0.0;
-            qd.push_back(make_double2((double)l * c, gl * cprev));
+            if (S != shtk::DSEG) qd.push_back(make_double2((double)l * c, gl * cprev));
             gt.push_back(gl);
         }
     }
@@ -1858,6 +1962,7 @@ static int plan_tables(shtk_plan *p) {
         sa.mmax = d.mmax;
         sa.mres = d.mres;
         sa.np = np;
+        sa.lseg = seg_lmax(p);
         sa.nm = nm;
         sa.seg = S;
         sa.x = p->x;
@@ -1920,7 +2025,6 @@ int shtk_plan_create(const shtk_desc *desc, shtk_plan **out) {
     // atomically when np > 256) instead of 512 (8 chains, 256 VGPRs, 1 wave/SIMD): 2.9 -> 2.3 ms
     // for 8 fields at lmax 1023
     p->vanal_pblk = env_int("SHTK_VANAL_PBLK", 256) == 512 ? 512 : 256;
-    p->vsynth_waves = env_int("SHTK_VSYNTH_WAVES", 1) == 4 ? 4 : 1;
     // scalar FP64 synthesis blocks of one wave once a launch has 8192 units or more
     // (2 fields at lmax 1023: 126 -> 119 us; 16 fields: 943 -> 821 us; one field
     // keeps 4 waves per block, 65 against 72 us)

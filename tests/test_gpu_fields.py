@@ -102,3 +102,50 @@ def test_batch_adjoint_analysis_and_conventions(shtk, oracle, cuda, lmax, nlat, 
     assert f32.dtype == np.float32 and _worst(f32, ocfg.synthesis(a32.astype(np.complex128))) < 1e-6
     assert _worst(to_host(shtk.synthesis_batch(cfg, to_dev(alm), real_output=False)),
                   ocfg.synthesis(alm, real_output=False)) < TOL
+
+
+VECTOR_SHAPES = [
+    # lmax, nlat, nlon, mres, ltr, nf, grid
+    (1, 3, 4, 1, -1, 1, "gauss"),
+    (62, 64, 126, 1, -1, 1, "gauss"),
+    (63, 65, 128, 1, -1, 3, "gauss"),        # the combination's last degree starts a segment
+    (64, 66, 130, 1, 63, 4, "gauss"),
+    (127, 130, 256, 2, -1, 2, "gauss"),
+    (130, 261, 264, 1, 129, 5, "regular"),
+    (66, 133, 134, 1, 64, 3, "regular_poles"),
+]
+
+
+@pytest.mark.parametrize("lmax,nlat,nlon,mres,ltr,nf,grid", VECTOR_SHAPES)
+def test_vector_transforms_match_oracle(shtk, oracle, cuda, lmax, nlat, nlon, mres, ltr, nf, grid):
+    """Fresh plan per direction: the analysis of a noise grid, whose order-0 tables
+    are made in that call, and the synthesis of coefficients with NaN above ltr."""
+    def cfgs():
+        kw = dict(nlon=nlon, mres=mres)
+        if grid == "gauss":
+            return shtk.create_gauss_config(lmax, nlat, **kw)
+        return shtk.create_regular_config(lmax, nlat, include_poles=grid == "regular_poles", **kw)
+
+    ocfg = oracle.Config(lmax, nlat, nlon=nlon, mres=mres, grid=grid)
+    rng = np.random.default_rng(lmax)
+    V = [np.asfortranarray(rng.standard_normal((nlat, nlon, nf))) for _ in range(2)]
+    print(f"vector lmax={lmax} nlat={nlat} mres={mres} ltr={ltr} nf={nf} {grid}", flush=True)
+    got = shtk.analysis_sphtor_batch(cfgs(), *[to_dev(v) for v in V], ltr=ltr)
+    ref = ocfg.analysis_sphtor(*V, ltr=ltr)
+    for g, r in zip(got, ref):
+        assert _worst(to_host(g), r) < TOL
+        assert np.all(to_host(g)[r == 0] == 0)
+    ST = [oracle.random_alm(lmax, lmax, seed=s, power=1.0, nf=nf, lmin=1) for s in (1, 2)]
+    if 0 <= ltr < lmax:
+        for a in ST:
+            a[ltr + 1:] = np.nan  # not read
+    cfg = cfgs()
+    got = shtk.synthesis_sphtor_batch(cfg, *[to_dev(a) for a in ST], ltr=ltr)
+    ref = ocfg.synthesis_sphtor(*[np.nan_to_num(a) for a in ST], ltr=ltr)
+    for g, r in zip(got, ref):
+        assert _worst(to_host(g), r) < TOL
+    if ltr < 0:
+        for g, r in zip(shtk._adjoint_synthesis_sphtor(cfg, *[to_dev(v) for v in V]), ocfg.adjoint_synthesis_sphtor(*V)):
+            assert _worst(to_host(g), r) < TOL
+        for g, r in zip(shtk._adjoint_analysis_sphtor(cfg, *[to_dev(a) for a in ST]), ocfg.adjoint_analysis_sphtor(*ST)):
+            assert _worst(to_host(g), r) < TOL
