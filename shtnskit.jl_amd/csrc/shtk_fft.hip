@@ -12,10 +12,10 @@
 // order).  Two real rows travel as one complex row z = f_a + i f_b (latitudes
 // k and 2G-1-k of the tile), so a single complex FFT of length N serves both
 // rows (no separate real-FFT pass).  The rows stay resident in LDS (16 N bytes
-// each) through a Stockham autosort FFT with radix 8/4/2/3/5 passes and generic
-// passes for other small primes; lengths with larger prime factors run
-// Bluestein's chirp convolution inside the same LDS row (of the convolution
-// length).  Twiddles come from per-plan tables.  Consecutive tiles are mapped to the same XCD so
+// each) through a Stockham autosort FFT with radix 8/4/2/3/5 passes, butterflies
+// for the primes 7 to 19 and a generic pass for other small primes; lengths with
+// larger prime factors run Bluestein's chirp convolution inside the same LDS row
+// (of the convolution length).  Twiddles come from per-plan tables.  Consecutive tiles are mapped to the same XCD so
 // the L2 merges the strided longitude-major stores of neighbouring rows.
 #include <algorithm>
 
@@ -95,43 +95,81 @@ __device__ __forceinline__ void dft_small(double2 *v) {
     }
 }
 
-// One Stockham pass of radix R over the LDS row z (length N).  Every thread
-// stages all its inputs in registers before the barrier, then writes.
 // values per thread in one Stockham pass: the row length over the threads of a row
 constexpr int FFT_VPT = 8;
+
+// Kernel variants: KIND 0 has the butterflies 2, 3, 4, 5 and 8 alone, KIND 1 the primes too,
+// KIND 2 runs Bluestein's convolution (whose length has the factors 2, 3 and 5 only).  Each
+// keeps its registers free of the others' state.
+enum { FFT_DIRECT = 0, FFT_PRIMES = 1, FFT_BLUE = 2 };
 
 // LDS position of row element i: one padding slot per 16 elements, which
 // spreads the strided 16-byte accesses of the Stockham passes (stride R or
 // R Ns elements) over all LDS banks.
 __device__ __forceinline__ int zp(int i) { return i + (i >> 4); }
 
-// P2: Ns is a power of two, so the butterfly's position j splits into j / Ns and
-// j mod Ns by a shift and a mask (a division by a run-time value is a sequence
-// of some twenty instructions).
-template <int R, int SIGN, bool P2>
-__device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const double2 *tw, int tid, int nt) {
+// j / Ns and j mod Ns of a butterfly position (j < 2^13): shift and mask where Ns is a power
+// of two, else one high product (a division by a run-time value is a sequence of some twenty
+// instructions).
+template <bool P2>
+struct NsDiv {
+    int Ns, sh;
+    unsigned mg;
+    __device__ __forceinline__ explicit NsDiv(int n) : Ns(n), sh(__builtin_ctz((unsigned)n)), mg(0) {
+        if (!P2) mg = 0xFFFFFFFFu / (unsigned)n + 1u;  // 0 for Ns = 1, whose quotient is j
+    }
+    __device__ __forceinline__ int div(int j) const {
+        return P2 ? (j >> sh) : Ns == 1 ? j : (int)__umulhi((unsigned)j, mg);
+    }
+    __device__ __forceinline__ int mod(int j) const { return P2 ? (j & (Ns - 1)) : j - div(j) * Ns; }
+};
+
+// What a pass of a Bluestein transform does beside its butterflies: the first one reads the
+// row times the chirp, zero past it; the last one of the forward transform multiplies by the
+// kernel's spectrum and goes on with the first pass of the inverse transform, whose inputs are
+// the values that the thread holds (the inverse runs the radices backwards, as a forward
+// transform of the conjugate); the last one of the inverse stores the row times the chirp.
+enum { BLUE_NONE = 0, BLUE_FIRST = 1, BLUE_MID = 2, BLUE_LAST = 3 };
+
+// One Stockham pass of radix R over the LDS row z (length N).  Every thread
+// stages all its inputs in registers before the barrier, then writes.
+template <int R, int SIGN, bool P2, bool BLUE>
+__device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const double2 *tw, int tid, int nt,
+                                              const FftArgs &a, int what) {
     // nt >= N / FFT_VPT (launch_fft), so a thread has at most ceil(FFT_VPT / R) butterflies
     constexpr int MAXB = (FFT_VPT + R - 1) / R;
+    constexpr int DS = BLUE ? -1 : SIGN;
     const int nb = N / R;
     const int stride = N / (Ns * R);
-    const int sh = __builtin_ctz((unsigned)Ns);
-    auto kmod = [&](int j) { return P2 ? (j & (Ns - 1)) : j % Ns; };
-    auto kdiv = [&](int j) { return P2 ? (j >> sh) : j / Ns; };
+    const NsDiv<P2> dv(Ns);
     // base twiddle w = W^(k stride) of each butterfly (the others are its
     // powers): independent of the LDS data, so its load overlaps the barrier
     double2 w1[MAXB];
 #pragma unroll
     for (int q = 0; q < MAXB; ++q) {
         const int j = tid + q * nt;
-        w1[q] = (Ns > 1 && j < nb) ? tw[kmod(j) * stride] : make_double2(1.0, 0.0);
+        w1[q] = (Ns > 1 && j < nb) ? tw[dv.mod(j) * stride] : make_double2(1.0, 0.0);
     }
     double2 v[MAXB][R];
 #pragma unroll
     for (int q = 0; q < MAXB; ++q) {
         const int j = tid + q * nt;
         if (j < nb) {
+            if (BLUE && what == BLUE_FIRST) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[q][r] = z[zp(j + r * nb)];
+                for (int r = 0; r < R; ++r) {
+                    const int e = j + r * nb;
+                    v[q][r] = make_double2(0.0, 0.0);
+                    if (e < a.nlon) {
+                        double2 c = z[zp(e)];
+                        if (SIGN > 0) c.y = -c.y;
+                        v[q][r] = cmul(c, a.chirp[e]);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r) v[q][r] = z[zp(j + r * nb)];
+            }
         }
     }
     __syncthreads();
@@ -139,10 +177,9 @@ __device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const d
     for (int q = 0; q < MAXB; ++q) {
         const int j = tid + q * nt;
         if (j < nb) {
-            const int k = kmod(j);
             if (Ns > 1) {
                 double2 w = w1[q];
-                if (SIGN > 0) w.y = -w.y;
+                if (DS > 0) w.y = -w.y;
                 double2 wr = w;
 #pragma unroll
                 for (int r = 1; r < R; ++r) {
@@ -150,21 +187,109 @@ __device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const d
                     if (r + 1 < R) wr = cmul(wr, w);
                 }
             }
-            dft_small<R, SIGN>(v[q]);
-            const int base = kdiv(j) * Ns * R + k;
+            dft_small<R, DS>(v[q]);
+            if (BLUE && what == BLUE_MID) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) z[zp(base + r * Ns)] = v[q][r];
+                for (int r = 0; r < R; ++r) {
+                    const double2 p = cmul(v[q][r], a.bhat[j + r * nb]);
+                    v[q][r] = make_double2(p.x, -p.y);
+                }
+                dft_small<R, DS>(v[q]);
+#pragma unroll
+                for (int r = 0; r < R; ++r) z[zp(j * R + r)] = v[q][r];
+            } else if (BLUE && what == BLUE_LAST) {
+                // Ns R = N: outputs j + r nb
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int e = j + r * nb;
+                    if (e < a.nlon) {
+                        double2 c = cmul(make_double2(v[q][r].x, -v[q][r].y), a.chirp[e]);
+                        if (SIGN > 0) c.y = -c.y;
+                        z[zp(e)] = c;
+                    }
+                }
+            } else {
+                const int base = dv.div(j) * Ns * R + dv.mod(j);
+#pragma unroll
+                for (int r = 0; r < R; ++r) z[zp(base + r * Ns)] = v[q][r];
+            }
         }
     }
     __syncthreads();
 }
 
-// Generic radix-R pass (R a prime above 5): every output is the R-term sum
+// Radix-R pass, R an odd prime of 7 to 19: sums and differences of the inputs r and R - r,
+// then (R - 1)/2 sums of each with cos and sin of 2 pi r / R, which come from the twiddle table
+// (scalar loads).  An output pair is stored as soon as it is done, so a butterfly takes
+// 4 R registers.  The twiddles are table entries, not powers (no accumulated rounding).
+template <int R, int SIGN>
+__device__ __forceinline__ void stockham_prime(double2 *z, int N, int Ns, const double2 *tw, int tid, int nt) {
+    constexpr int H = (R - 1) / 2;
+    const int nb = N / R, stride = N / (Ns * R);
+    const NsDiv<false> dv(Ns);
+    typedef const __attribute__((address_space(4))) double2 *ctab;
+    const ctab tc = (ctab)tw;
+    double2 cs[H];  // (cos, SIGN sin)
+#pragma unroll
+    for (int r = 0; r < H; ++r) cs[r] = make_double2(tc[(r + 1) * nb].x, SIGN > 0 ? -tc[(r + 1) * nb].y : tc[(r + 1) * nb].y);
+    constexpr int MAXB = (FFT_VPT + R - 1) / R;  // as in stockham_pass
+    double2 v[MAXB][R];
+#pragma unroll
+    for (int q = 0; q < MAXB; ++q) {
+        const int j = tid + q * nt;
+        if (j < nb) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) v[q][r] = z[zp(j + r * nb)];
+            if (Ns > 1) {
+                const int k = dv.mod(j) * stride;
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    double2 w = tw[r * k];
+                    if (SIGN > 0) w.y = -w.y;
+                    v[q][r] = cmul(v[q][r], w);
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < MAXB; ++q) {
+        const int j = tid + q * nt;
+        if (j >= nb) continue;
+        double2 *x = v[q];
+        const int base = dv.div(j) * Ns * R + dv.mod(j);
+        double2 s0 = x[0];
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+            const double2 p = cadd(x[r], x[R - r]), m = csub(x[r], x[R - r]);
+            x[r] = p;
+            x[R - r] = m;
+            s0 = cadd(s0, p);
+        }
+        z[zp(base)] = s0;
+#pragma unroll
+        for (int o = 1; o <= H; ++o) {
+            double2 t = x[0], u = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int r = 1; r <= H; ++r) {
+                const int g = r * o % R, h = g <= H ? g : R - g;
+                const double c = cs[h - 1].x, sn = g <= H ? cs[h - 1].y : -cs[h - 1].y;
+                t = make_double2(fma(c, x[r].x, t.x), fma(c, x[r].y, t.y));
+                u = make_double2(fma(-sn, x[R - r].y, u.x), fma(sn, x[R - r].x, u.y));  // i sn (x_r - x_{R-r})
+            }
+            z[zp(base + o * Ns)] = cadd(t, u);
+            z[zp(base + (R - o) * Ns)] = csub(t, u);
+        }
+    }
+    __syncthreads();
+}
+
+// Generic radix-R pass (R a prime above 19): every output is the R-term sum
 // out(j, r) = sum_s z[j + s nb] W^(s (k + r Ns) stride), k = j mod Ns, with the
 // twiddles read from the table (exact angles, no accumulated rounding).  A
 // thread computes up to FFT_VPT outputs (nt >= N / FFT_VPT).
 template <int SIGN>
-__device__ void stockham_gen(double2 *z, int N, int Ns, int R, const double2 *tw, int tid, int nt) {
+__device__ __forceinline__ void stockham_gen(double2 *z, int N, int Ns, int R, const double2 *tw, int tid, int nt) {
     const int nb = N / R, stride = N / (Ns * R);
     double2 out[FFT_VPT];
 #pragma unroll
@@ -199,77 +324,74 @@ __device__ void stockham_gen(double2 *z, int N, int Ns, int R, const double2 *tw
     __syncthreads();
 }
 
-// All passes of a length-N transform of the LDS row z (unnormalised).  GEN =
-// false compiles the radix 2/3/4/5/8 butterflies alone (the common lengths keep
-// their registers free of the generic pass's state).
-template <int SIGN, bool GEN>
-__device__ void fft_passes(double2 *z, int N, int nrad, unsigned long long radix, const double2 *tw, int tid,
-                           int nt) {
-    int Ns = 1;
-    for (int q = 0; q < nrad; ++q) {
-        const int R = (int)((radix >> (FFT_RADIX_BITS * q)) & ((1ull << FFT_RADIX_BITS) - 1));
-        const bool p2 = (Ns & (Ns - 1)) == 0;
-        switch (R) {
-            case 8:
-                if (p2) stockham_pass<8, SIGN, true>(z, N, Ns, tw, tid, nt);
-                else stockham_pass<8, SIGN, false>(z, N, Ns, tw, tid, nt);
-                break;
-            case 4:
-                if (p2) stockham_pass<4, SIGN, true>(z, N, Ns, tw, tid, nt);
-                else stockham_pass<4, SIGN, false>(z, N, Ns, tw, tid, nt);
-                break;
-            case 2:
-                if (p2) stockham_pass<2, SIGN, true>(z, N, Ns, tw, tid, nt);
-                else stockham_pass<2, SIGN, false>(z, N, Ns, tw, tid, nt);
-                break;
-            case 3: stockham_pass<3, SIGN, false>(z, N, Ns, tw, tid, nt); break;
-            default:
-                if constexpr (GEN) {
-                    if (R != 5) {
-                        stockham_gen<SIGN>(z, N, Ns, R, tw, tid, nt);
-                        break;
-                    }
-                }
-                stockham_pass<5, SIGN, false>(z, N, Ns, tw, tid, nt);
-                break;
-        }
-        Ns *= R;
-    }
-}
-
 // Length-nlon DFT of the LDS row z (entries at zp(j), j < nlon; the row holds
-// nfft + nfft/16 + 1 slots).  Direct passes, or (GEN only) Bluestein: chirp,
-// zero-pad to nfft, cyclic convolution with the kernel spectrum (forward FFT,
-// pointwise product, inverse FFT), chirp.  The caller's barrier precedes; one
-// follows.
-template <int SIGN, bool GEN>
-__device__ void fft_lds(double2 *z, const FftArgs &a, int tid, int nt) {
-    if (!GEN || !a.blue) {
-        fft_passes<SIGN, GEN>(z, a.nlon, a.nrad, a.radix, a.tw, tid, nt);
-        return;
-    }
-    const int N = a.nlon, M = a.nfft;
-    for (int j = tid; j < M; j += nt) {
-        if (j < N) {
-            double2 c = a.chirp[j];
-            if (SIGN > 0) c.y = -c.y;
-            z[zp(j)] = cmul(z[zp(j)], c);
-        } else {
-            z[zp(j)] = make_double2(0.0, 0.0);
+// nfft + nfft/16 + 1 slots).  The caller's barrier precedes; one follows.
+//
+// Bluestein (KIND 2): chirp, cyclic convolution of length nfft with the kernel spectrum,
+// chirp, in 2 nrad - 1 passes over LDS: the products sit in the first, middle and last pass
+// (they were four passes of their own, and the middle two passes one each).  DFT of the other
+// sign: the conjugate row, whose transform is the conjugate.
+//
+// The pass loops hide the thread's index from the optimiser: the addresses of every pass
+// depend on it and the length alone, and kept over the loop they filled the registers and
+// 340 to 600 bytes of scratch per thread.  Whole calls: 16 fields at lmax 700, nlon 1402
+// (Bluestein): 895 -> 455 us; 8 at 1000, nlon 2002 = 2 * 7 * 11 * 13: 672 -> 359; 32 at
+// 303, nlon 608 = 32 * 19: 173 -> 82 (nlon 640: 75); one: 29 -> 19.
+template <int SIGN, int KIND>
+__device__ __forceinline__ void fft_lds(double2 *z, const FftArgs &a, int tid, int nt) {
+    auto rad = [&](int q) { return (int)((a.radix >> (FFT_RADIX_BITS * q)) & ((1ull << FFT_RADIX_BITS) - 1)); };
+    if constexpr (KIND == FFT_BLUE) {
+        const int M = a.nfft, np = 2 * a.nrad - 1, mid = a.nrad - 1;
+        int Ns = 1;
+        for (int q = 0; q < np; ++q) {
+            asm volatile("" : "+v"(tid));  // no pass's addresses are kept over the others
+            const int R = rad(q <= mid ? q : 2 * mid - q);
+            const int what = q == 0 ? BLUE_FIRST : q == mid ? BLUE_MID : q == np - 1 ? BLUE_LAST : BLUE_NONE;
+            switch (R) {
+                case 8: stockham_pass<8, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
+                case 4: stockham_pass<4, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
+                case 2: stockham_pass<2, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
+                case 3: stockham_pass<3, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
+                default: stockham_pass<5, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
+            }
+            Ns = q == mid ? R : Ns * R;
+        }
+    } else {
+        const int N = a.nlon;
+        int Ns = 1;
+        for (int q = 0; q < a.nrad; ++q) {
+            if (KIND != FFT_DIRECT) asm volatile("" : "+v"(tid));  // as above
+            const int R = rad(q);
+            const bool p2 = KIND == FFT_DIRECT && (Ns & (Ns - 1)) == 0;
+            switch (R) {
+                case 8:
+                    if (p2) stockham_pass<8, SIGN, true, false>(z, N, Ns, a.tw, tid, nt, a, 0);
+                    else stockham_pass<8, SIGN, false, false>(z, N, Ns, a.tw, tid, nt, a, 0);
+                    break;
+                case 4:
+                    if (p2) stockham_pass<4, SIGN, true, false>(z, N, Ns, a.tw, tid, nt, a, 0);
+                    else stockham_pass<4, SIGN, false, false>(z, N, Ns, a.tw, tid, nt, a, 0);
+                    break;
+                case 2:
+                    if (p2) stockham_pass<2, SIGN, true, false>(z, N, Ns, a.tw, tid, nt, a, 0);
+                    else stockham_pass<2, SIGN, false, false>(z, N, Ns, a.tw, tid, nt, a, 0);
+                    break;
+                case 3: stockham_pass<3, SIGN, false, false>(z, N, Ns, a.tw, tid, nt, a, 0); break;
+                case 5: stockham_pass<5, SIGN, false, false>(z, N, Ns, a.tw, tid, nt, a, 0); break;
+                default:
+                    if constexpr (KIND == FFT_PRIMES) {
+                        if (R == 7) stockham_prime<7, SIGN>(z, N, Ns, a.tw, tid, nt);
+                        else if (R == 11) stockham_prime<11, SIGN>(z, N, Ns, a.tw, tid, nt);
+                        else if (R == 13) stockham_prime<13, SIGN>(z, N, Ns, a.tw, tid, nt);
+                        else if (R == 17) stockham_prime<17, SIGN>(z, N, Ns, a.tw, tid, nt);
+                        else if (R == 19) stockham_prime<19, SIGN>(z, N, Ns, a.tw, tid, nt);
+                        else stockham_gen<SIGN>(z, N, Ns, R, a.tw, tid, nt);
+                    }
+                    break;
+            }
+            Ns *= R;
         }
     }
-    __syncthreads();
-    fft_passes<-1, GEN>(z, M, a.nrad, a.radix, a.tw, tid, nt);
-    const double2 *bh = a.bhat + (SIGN > 0 ? M : 0);
-    for (int j = tid; j < M; j += nt) z[zp(j)] = cmul(z[zp(j)], bh[j]);
-    __syncthreads();
-    fft_passes<+1, GEN>(z, M, a.nrad, a.radix, a.tw, tid, nt);
-    for (int j = tid; j < N; j += nt) {
-        double2 c = a.chirp[j];
-        if (SIGN > 0) c.y = -c.y;
-        z[zp(j)] = cmul(z[zp(j)], c);
-    }
-    __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -335,13 +457,13 @@ __device__ __forceinline__ double fft_row_scale(const FftArgs &a, int lat) {
 // rows z = f_a + i f_b of latitudes L0 + g and L0 + 2G - 1 - g at positions zp(j)
 // (row stride RS = N + N/16 + 1 complex: the rows of one longitude fall in
 // different LDS banks).
-template <int G, typename GT, bool GEN>
+template <int G, typename GT, int KIND>
 __global__ __launch_bounds__(1024) void k_fft_synth_t(const FftArgs a, int nfields) {
     extern __shared__ double2 zs[];
     constexpr int L = 2 * G;
     const int N = a.nlon, nlat = a.nlat, RS = a.nfft + (a.nfft >> 4) + 1;
-    // orders 0 .. N/2 - 1 in steps of 1 fill every bin of the row except N / 2
-    const bool full = !a.blue && a.mres == 1 && 2 * a.nm == N;
+    // orders 0, 1, .. fill every bin of the row (odd N) or all but N / 2
+    const bool full = a.mres == 1 && 2 * a.nm - 1 >= N - 1;
     const int tid = threadIdx.x, nt = blockDim.x, tr = nt / G;
     const int row = tid / tr, lt = tid % tr;
     const int k = tid % L;                // lane role within its group of 2G
@@ -356,7 +478,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_t(const FftArgs a, int nfiel
         if (full) {
             // every bin but N / 2 is written below (the previous tile's barrier
             // ordered its reads before these writes)
-            if (tid < G) zs[tid * RS + zp(N / 2)] = make_double2(0.0, 0.0);
+            if (2 * a.nm == N && tid < G) zs[tid * RS + zp(N / 2)] = make_double2(0.0, 0.0);
         } else {
             for (int q = tid; q < G * RS; q += nt) zs[q] = make_double2(0.0, 0.0);
             __syncthreads();
@@ -391,7 +513,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_t(const FftArgs a, int nfiel
             }
         }
         __syncthreads();
-        fft_lds<+1, GEN>(zs + row * RS, a, lt, tr);
+        fft_lds<+1, KIND>(zs + row * RS, a, lt, tr);
         const int nrow = a.nrow;
         GT *gf = fft_grid<GT>(a, f, (size_t)nrow * N) + lat;
         if (live && lat < nrow) {
@@ -411,7 +533,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_t(const FftArgs a, int nfiel
 // each latitude is its own complex row with the bins m = 0 .. mmax of the
 // Fourier data (no Hermitian mirror) and the grid element is the complex value.
 // Tiles of G adjacent latitudes, one LDS row each.
-template <int G, typename GT, bool GEN>
+template <int G, typename GT, int KIND>
 __global__ __launch_bounds__(1024) void k_fft_synth_c(const FftArgs a, int nfields) {
     extern __shared__ double2 zs[];
     const int N = a.nlon, nlat = a.nlat, RS = a.nfft + (a.nfft >> 4) + 1;
@@ -431,7 +553,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_c(const FftArgs a, int nfiel
             if (live) z[zp(im * a.mres)] = Ff[(size_t)im * nlat];
         }
         __syncthreads();
-        fft_lds<+1, GEN>(zs + row * RS, a, lt, tr);
+        fft_lds<+1, KIND>(zs + row * RS, a, lt, tr);
         const int nrow = a.nrow;
         GT *gf = fft_grid<GT>(a, f, 2 * (size_t)nrow * N) + 2 * lat;
         if (live && lat < nrow) {
@@ -451,7 +573,7 @@ __global__ __launch_bounds__(1024) void k_fft_synth_c(const FftArgs a, int nfiel
 // 169-207 with a complex eltype): each latitude's complex row is transformed
 // and the bins m = 0 .. mmax are kept, the columns the m-loop reads
 // (Fph[:, m+1]).  Tiles of G adjacent latitudes, one LDS row each.
-template <int G, typename GT, bool GEN>
+template <int G, typename GT, int KIND>
 __global__ __launch_bounds__(1024) void k_fft_anal_c(const FftArgs a, int nfields) {
     extern __shared__ double2 zs[];
     const int N = a.nlon, nlat = a.nlat, RS = a.nfft + (a.nfft >> 4) + 1;
@@ -474,7 +596,7 @@ __global__ __launch_bounds__(1024) void k_fft_anal_c(const FftArgs a, int nfield
                                : make_double2(0.0, 0.0);
         }
         __syncthreads();
-        fft_lds<-1, GEN>(zs + row * RS, a, lt, tr);
+        fft_lds<-1, KIND>(zs + row * RS, a, lt, tr);
         if (live) {
             double2 *Ff = a.F + (size_t)f * a.nm * nlat + lat;
             for (int e = tid; e < a.nm * G; e += nt) {
@@ -488,7 +610,7 @@ __global__ __launch_bounds__(1024) void k_fft_anal_c(const FftArgs a, int nfield
 
 // Analysis: grid rows -> Fourier data, F_a = (Z_m + conj Z_{N-m}) / 2,
 // F_b = (Z_m - conj Z_{N-m}) / (2i) of the packed row Z = f_a + i f_b.
-template <int G, typename GT, bool GEN>
+template <int G, typename GT, int KIND>
 __global__ __launch_bounds__(1024) void k_fft_anal_t(const FftArgs a, int nfields) {
     extern __shared__ double2 zs[];
     constexpr int L = 2 * G;
@@ -526,7 +648,7 @@ __global__ __launch_bounds__(1024) void k_fft_anal_t(const FftArgs a, int nfield
             }
         }
         __syncthreads();
-        fft_lds<-1, GEN>(zs + row * RS, a, lt, tr);
+        fft_lds<-1, KIND>(zs + row * RS, a, lt, tr);
         if (live) {
             double2 *Ff = a.F + (size_t)f * a.nm * nlat + lat;
             for (int e = tid; e < a.nm * L; e += nt) {
@@ -555,21 +677,20 @@ int fft_row_threads(const FftArgs &a, size_t *row_bytes) {
     return tr;
 }
 
-// The general kernels (generic prime passes, Bluestein) only where the length needs them.
-bool fft_general(const FftArgs &a) {
-    if (a.blue) return true;
+int fft_kind(const FftArgs &a) {
+    if (a.blue) return FFT_BLUE;
     for (int q = 0; q < a.nrad; ++q) {
         const int R = (int)((a.radix >> (FFT_RADIX_BITS * q)) & ((1ull << FFT_RADIX_BITS) - 1));
-        if (R != 2 && R != 3 && R != 4 && R != 5 && R != 8) return true;
+        if (R != 2 && R != 3 && R != 4 && R != 5 && R != 8) return FFT_PRIMES;
     }
-    return false;
+    return FFT_DIRECT;
 }
 
-template <int G, typename GT, bool GEN>
+template <int G, typename GT, int KIND>
 hipError_t launch_tile_g(const FftArgs &a, int nfields, int inverse, int tr, size_t row, hipStream_t st) {
     const int nt = G * tr;
     const size_t lds = row * G;
-    const void *fn = inverse ? (const void *)k_fft_synth_t<G, GT, GEN> : (const void *)k_fft_anal_t<G, GT, GEN>;
+    const void *fn = inverse ? (const void *)k_fft_synth_t<G, GT, KIND> : (const void *)k_fft_anal_t<G, GT, KIND>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
@@ -580,52 +701,64 @@ hipError_t launch_tile_g(const FftArgs &a, int nfields, int inverse, int tr, siz
     const int per_cu = (int)std::max<size_t>(1, (160 * 1024) / lds);
     int grid = std::min(256 * per_cu, (total + 7) / 8 * 8);
     grid = std::max(8, grid / 8 * 8);
-    if (inverse) hipLaunchKernelGGL((k_fft_synth_t<G, GT, GEN>), dim3(grid), dim3(nt), lds, st, a, nfields);
-    else hipLaunchKernelGGL((k_fft_anal_t<G, GT, GEN>), dim3(grid), dim3(nt), lds, st, a, nfields);
+    if (inverse) hipLaunchKernelGGL((k_fft_synth_t<G, GT, KIND>), dim3(grid), dim3(nt), lds, st, a, nfields);
+    else hipLaunchKernelGGL((k_fft_anal_t<G, GT, KIND>), dim3(grid), dim3(nt), lds, st, a, nfields);
     return hipGetLastError();
 }
 
 template <int G>
 hipError_t launch_tile(const FftArgs &a, int nfields, int inverse, int tr, size_t row, hipStream_t st) {
-    const bool gen = fft_general(a);
-    if (a.io_f32)
-        return gen ? launch_tile_g<G, float, true>(a, nfields, inverse, tr, row, st)
-                   : launch_tile_g<G, float, false>(a, nfields, inverse, tr, row, st);
-    return gen ? launch_tile_g<G, double, true>(a, nfields, inverse, tr, row, st)
-               : launch_tile_g<G, double, false>(a, nfields, inverse, tr, row, st);
+    switch (fft_kind(a)) {
+        case FFT_BLUE:
+            return a.io_f32 ? launch_tile_g<G, float, FFT_BLUE>(a, nfields, inverse, tr, row, st)
+                            : launch_tile_g<G, double, FFT_BLUE>(a, nfields, inverse, tr, row, st);
+        case FFT_PRIMES:
+            return a.io_f32 ? launch_tile_g<G, float, FFT_PRIMES>(a, nfields, inverse, tr, row, st)
+                            : launch_tile_g<G, double, FFT_PRIMES>(a, nfields, inverse, tr, row, st);
+        default:
+            return a.io_f32 ? launch_tile_g<G, float, FFT_DIRECT>(a, nfields, inverse, tr, row, st)
+                            : launch_tile_g<G, double, FFT_DIRECT>(a, nfields, inverse, tr, row, st);
+    }
 }
 
-template <int G, typename GT, bool GEN>
+template <int G, typename GT, int KIND>
 hipError_t launch_cplx_g(const FftArgs &a, int nfields, int inverse, int tr, size_t row, hipStream_t st) {
     const size_t lds = row * G;
-    const void *fn = inverse ? (const void *)k_fft_synth_c<G, GT, GEN> : (const void *)k_fft_anal_c<G, GT, GEN>;
+    const void *fn = inverse ? (const void *)k_fft_synth_c<G, GT, KIND> : (const void *)k_fft_anal_c<G, GT, KIND>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
     const int total = (a.nlat + G - 1) / G * nfields;
     const int grid = std::max(1, std::min(256 * (int)std::max<size_t>(1, (160 * 1024) / lds), total));
-    if (inverse) hipLaunchKernelGGL((k_fft_synth_c<G, GT, GEN>), dim3(grid), dim3(G * tr), lds, st, a, nfields);
-    else hipLaunchKernelGGL((k_fft_anal_c<G, GT, GEN>), dim3(grid), dim3(G * tr), lds, st, a, nfields);
+    if (inverse) hipLaunchKernelGGL((k_fft_synth_c<G, GT, KIND>), dim3(grid), dim3(G * tr), lds, st, a, nfields);
+    else hipLaunchKernelGGL((k_fft_anal_c<G, GT, KIND>), dim3(grid), dim3(G * tr), lds, st, a, nfields);
     return hipGetLastError();
 }
 
-template <typename GT, bool GEN>
+template <typename GT, int KIND>
 hipError_t launch_cplx_t(const FftArgs &a, int nfields, int inverse, hipStream_t st) {
     size_t row = 0;
     const int tr = fft_row_threads(a, &row);
     if (!tr) return hipErrorNotSupported;
-    if (4 * row <= 160 * 1024 && 4 * tr <= 1024) return launch_cplx_g<4, GT, GEN>(a, nfields, inverse, tr, row, st);
-    if (2 * row <= 160 * 1024 && 2 * tr <= 1024) return launch_cplx_g<2, GT, GEN>(a, nfields, inverse, tr, row, st);
-    return launch_cplx_g<1, GT, GEN>(a, nfields, inverse, tr, row, st);
+    if (4 * row <= 160 * 1024 && 4 * tr <= 1024) return launch_cplx_g<4, GT, KIND>(a, nfields, inverse, tr, row, st);
+    if (2 * row <= 160 * 1024 && 2 * tr <= 1024) return launch_cplx_g<2, GT, KIND>(a, nfields, inverse, tr, row, st);
+    return launch_cplx_g<1, GT, KIND>(a, nfields, inverse, tr, row, st);
 }
 }  // namespace
 
 hipError_t launch_fft_cplx(const FftArgs &a, int nfields, int inverse, hipStream_t st) {
-    const bool gen = fft_general(a);
-    if (a.io_f32)
-        return gen ? launch_cplx_t<float, true>(a, nfields, inverse, st) : launch_cplx_t<float, false>(a, nfields, inverse, st);
-    return gen ? launch_cplx_t<double, true>(a, nfields, inverse, st) : launch_cplx_t<double, false>(a, nfields, inverse, st);
+    switch (fft_kind(a)) {
+        case FFT_BLUE:
+            return a.io_f32 ? launch_cplx_t<float, FFT_BLUE>(a, nfields, inverse, st)
+                            : launch_cplx_t<double, FFT_BLUE>(a, nfields, inverse, st);
+        case FFT_PRIMES:
+            return a.io_f32 ? launch_cplx_t<float, FFT_PRIMES>(a, nfields, inverse, st)
+                            : launch_cplx_t<double, FFT_PRIMES>(a, nfields, inverse, st);
+        default:
+            return a.io_f32 ? launch_cplx_t<float, FFT_DIRECT>(a, nfields, inverse, st)
+                            : launch_cplx_t<double, FFT_DIRECT>(a, nfields, inverse, st);
+    }
 }
 
 hipError_t launch_fft(const FftArgs &a, int nfields, int inverse, hipStream_t st) {

@@ -138,14 +138,16 @@ struct SeedArgs {
 };
 
 // FFT factorisations: FFT_RADIX_BITS bits per pass, first pass in the low bits.
-// Radices 2, 3, 4, 5 and 8 have dedicated butterflies; other primes up to
-// FFT_GEN_MAX run a generic pass (R table twiddles per output).  Lengths whose
-// other prime factors would cost more take Bluestein's algorithm: a circular
-// convolution of length nfft >= 2 nlon - 1 (2^a 3^b 5^c) through two FFTs.
+// Radices 2, 3, 4, 5, 8 and the primes 7 to FFT_PRIME_MAX have butterflies; other
+// primes up to FFT_GEN_MAX run a generic pass (R table twiddles per output).
+// Lengths whose other prime factors would cost more take Bluestein's algorithm: a
+// circular convolution of length nfft >= 2 nlon - 1 (2^a 3^b 5^c) through two FFTs.
 constexpr int FFT_RADIX_BITS = 6;
 constexpr int FFT_MAX_PASSES = 10;
+constexpr int FFT_PRIME_MAX = 19;   // largest prime with a butterfly of its own
 constexpr int FFT_GEN_MAX = 61;     // largest prime of the generic pass
-constexpr int FFT_GEN_BUDGET = 48;  // largest sum of generic primes before Bluestein is used
+constexpr int FFT_GEN_BUDGET = 28;  // largest sum of generic primes before Bluestein is used
+constexpr int FFT_LONG_BUDGET = 48; // largest sum of primes above 5 of lengths too long for Bluestein
 constexpr int FFT_MAX_LEN = 8192;   // LDS FFT length limit (8 values per thread, 1024 threads)
 
 struct FftPlan {
@@ -161,7 +163,7 @@ struct FftArgs {
     unsigned long long radix; // FFT_RADIX_BITS bits per pass (of the length-nfft transform)
     const double2 *tw;        // e^{-2 pi i t / nfft}
     int nfft;                 // LDS row length: nlon, or the Bluestein convolution length
-    int blue;                 // Bluestein: chirp[nlon] = e^{-pi i t^2 / nlon}, bhat[2][nfft] = kernel spectra / nfft
+    int blue;                 // Bluestein: chirp[nlon] = e^{-pi i t^2 / nlon}, bhat[nfft] = its spectrum / nfft
     const double2 *chirp, *bhat;
     double2 *F;               // Fourier workspace [field][im][nlat]
     void *grid;               // grid array (nrow, nlon, nfields)

@@ -194,35 +194,45 @@ double coef_scale(const shtk_desc &d, int l, int m) {
     return nrm * rs * ph;
 }
 
-// Pass radices of one FFT length: 8, 4, 2, 3, 5 first, then the other primes
-// up to FFT_GEN_MAX (generic passes, whose sum is returned in *gen_sum).
-bool factor_len(int n, std::vector<int> &r, int *gen_sum) {
+// Pass radices of one FFT length: primes from 7 up to FFT_GEN_MAX, largest first
+// (the first pass needs no twiddles), then 8, 4, 2, 3, 5.  *sum: the sum of those
+// primes; *gen_sum: of the ones that run the generic pass.
+bool factor_len(int n, std::vector<int> &r, int *sum, int *gen_sum) {
     r.clear();
-    *gen_sum = 0;
+    *sum = *gen_sum = 0;
+    for (int q = shtk::FFT_GEN_MAX; q >= 7; --q) {
+        if (q % 2 == 0 || q % 3 == 0 || q % 5 == 0 || (q == 49)) continue;
+        while (n % q == 0) {
+            r.push_back(q);
+            *sum += q;
+            if (q > shtk::FFT_PRIME_MAX) *gen_sum += q;
+            n /= q;
+        }
+    }
     for (int c : {8, 4, 2, 3, 5})
         while (n % c == 0) {
             r.push_back(c);
             n /= c;
         }
-    for (int q = 7; n > 1 && q <= shtk::FFT_GEN_MAX; q += 2)
-        while (n % q == 0) {
-            r.push_back(q);
-            *gen_sum += q;
-            n /= q;
-        }
     return n == 1 && (int)r.size() <= shtk::FFT_MAX_PASSES;
 }
 
-// The longitude FFT of length n: direct mixed-radix passes when n's prime
-// factors above 5 are few and small, otherwise Bluestein's algorithm with the
-// shortest 2^a 3^b 5^c convolution length >= 2n - 1.  FFTW (the reference's
-// FFT, src/fftutils.jl:195-238) accepts every length; so does this plan up to
-// FFT_MAX_LEN (direct) and FFT_MAX_LEN / 2 (Bluestein).
+// The longitude FFT of length n: direct mixed-radix passes when its factors have
+// butterflies or one prime up to FFT_GEN_BUDGET runs the generic pass, otherwise
+// Bluestein's algorithm with the shortest 2^a 3^b 5^c convolution length >= 2n - 1.
+// A generic pass of prime R reads R values per output, so Bluestein's nine or so passes
+// of twice the length meet it between 23 and 31 (synthesis, generic against Bluestein:
+// nlon 1392 = 48 * 29, 16 fields, 434 and 441 us; 682 = 22 * 31, 24 fields, 140 and 156;
+// 2046 = 66 * 31, 8 fields, 497 and 450; 638 = 22 * 29, one field, 33 and 24).
+// FFTW (the reference's FFT, src/fftutils.jl:195-238) accepts every length; so does
+// this plan up to FFT_MAX_LEN / 2, and beyond, to FFT_MAX_LEN, where the primes above
+// 5 add up to FFT_LONG_BUDGET at most.
 shtk::FftPlan make_fft_plan(int n) {
     shtk::FftPlan f;
     if (n < 1 || n > shtk::FFT_MAX_LEN) return f;
-    int gs = 0;
-    if (factor_len(n, f.radix, &gs) && gs <= shtk::FFT_GEN_BUDGET) {
+    int sum = 0, gs = 0;
+    if (factor_len(n, f.radix, &sum, &gs) &&
+        (2 * n - 1 > shtk::FFT_MAX_LEN ? sum <= shtk::FFT_LONG_BUDGET : gs <= shtk::FFT_GEN_BUDGET)) {
         f.ok = true;
         f.nfft = n;
         return f;
@@ -231,7 +241,7 @@ shtk::FftPlan make_fft_plan(int n) {
         int t = m;
         for (int c : {2, 3, 5})
             while (t % c == 0) t /= c;
-        if (t != 1 || !factor_len(m, f.radix, &gs)) continue;
+        if (t != 1 || !factor_len(m, f.radix, &sum, &gs) || f.radix.size() < 2) continue;
         f.ok = f.blue = true;
         f.nfft = m;
         return f;
@@ -1885,7 +1895,7 @@ static int plan_tables(shtk_plan *p) {
         if (p->fft.blue) {
             // Bluestein: X_k = conj(b_k) sum_n (x_n conj(b_n)) b_{k-n}, b_n = e^{i pi n^2 / N};
             // the convolution kernel B (b_m at m and M - m) is even, so its spectrum is
-            // b_0 + 2 sum_{m>=1} b_m cos(2 pi m k / M); the inverse DFT uses conj(B).
+            // b_0 + 2 sum_{m>=1} b_m cos(2 pi m k / M); the inverse DFT conjugates the row.
             chirp.resize(N);
             std::vector<long double> br(N), bi(N);
             for (int t = 0; t < N; ++t) {
@@ -1897,7 +1907,7 @@ static int plan_tables(shtk_plan *p) {
             }
             std::vector<long double> cosM(M);
             for (int t = 0; t < M; ++t) cosM[t] = cosl(2.0L * PI_L * t / M);
-            bhat.resize(2 * (size_t)M);
+            bhat.resize(M);
             for (int k = 0; k < M; ++k) {
                 long double re = br[0], im = bi[0];
                 long long idx = 0;
@@ -1908,7 +1918,6 @@ static int plan_tables(shtk_plan *p) {
                     im += 2.0L * bi[m] * cosM[idx];
                 }
                 bhat[k] = make_double2((double)(re / M), (double)(im / M));
-                bhat[M + k] = make_double2((double)(re / M), -(double)(im / M));
             }
         }
     }
