@@ -254,7 +254,7 @@ void free_plan(shtk_plan *p) {
     if (!p) return;
     void *ptrs[] = {p->x,      p->s,      p->wscaled, p->winvs,  p->winvs2, p->invs,  p->qc,  p->ab, p->gtab,
                     p->qd,     p->coff,   p->segbase, p->seedq0, p->seedq1, p->seedk, p->pfirst,
-                    p->pfast,  p->segm,   p->convscale, p->tw, p->chirp, p->bhat, p->ws,     p->sectv, p->sectk, p->oz_q0,
+                    p->pfast,  p->segm,   p->convscale, p->tw, p->ws,     p->sectv, p->sectk, p->oz_q0,
                     p->oz_q1,  p->oz_qk,  p->oz_ep,     p->oz_chbase, p->oz_ws, p->oz_emaxl, p->oz_epl,
                     p->oz_asc, p->oz_chm, p->oz_run, p->qb, p->qcc, p->zseed};
     for (void *q : ptrs)
@@ -1763,6 +1763,38 @@ int shtk_stream_sync(void *stream) {
     return SHTK_OK;
 }
 
+struct LdCplx {
+    long double re, im;
+};
+
+// out = DFT of in[0], in[stride], .. (n = M / stride values, n's factors 2, 3 and 5) from the
+// length-M tables of cos and sin.
+static void ld_dft(const LdCplx *in, LdCplx *out, int n, int stride, const std::vector<long double> &c,
+                   const std::vector<long double> &s) {
+    if (n == 1) {
+        out[0] = in[0];
+        return;
+    }
+    const int R = n % 2 == 0 ? 2 : n % 3 == 0 ? 3 : 5, m = n / R, M = (int)c.size();
+    for (int r = 0; r < R; ++r) ld_dft(in + (size_t)r * stride, out + (size_t)r * m, m, stride * R, c, s);
+    auto mul = [&](const LdCplx &a, int t) {  // a e^{-2 pi i t / M}
+        return LdCplx{a.re * c[t] + a.im * s[t], a.im * c[t] - a.re * s[t]};
+    };
+    for (int k = 0; k < m; ++k) {
+        LdCplx v[5];
+        for (int r = 0; r < R; ++r) v[r] = mul(out[(size_t)r * m + k], r * k * stride);
+        for (int q = 0; q < R; ++q) {
+            LdCplx a = v[0];
+            for (int r = 1; r < R; ++r) {
+                const LdCplx u = mul(v[r], r * q % R * (M / R));
+                a.re += u.re;
+                a.im += u.im;
+            }
+            out[(size_t)q * m + k] = a;
+        }
+    }
+}
+
 static int plan_tables(shtk_plan *p) {
     const shtk_desc &d = p->d;
     const int np = p->np, nm = p->nm, lmax = d.lmax, S = p->seg;
@@ -1884,41 +1916,33 @@ static int plan_tables(shtk_plan *p) {
     }
     p->fft = make_fft_plan(d.nlon);
     const long double PI_L = 3.141592653589793238462643383279502884L;
-    std::vector<double2> tw, chirp, bhat;
+    std::vector<double2> tw;
     if (p->fft.ok) {
         const int M = p->fft.nfft, N = d.nlon;
-        tw.resize(M);
+        std::vector<long double> cosM(M), sinM(M);
         for (int t = 0; t < M; ++t) {
-            const long double ang = 2.0L * PI_L * t / M;
-            tw[t] = make_double2((double)cosl(ang), -(double)sinl(ang));
+            const int u = 2 * t > M ? M - t : t;
+            cosM[t] = u == t ? cosl(2.0L * PI_L * t / M) : cosM[u];
+            sinM[t] = u == t ? sinl(2.0L * PI_L * t / M) : -sinM[u];
         }
+        tw.resize(M);
+        for (int t = 0; t < M; ++t) tw[t] = make_double2((double)cosM[t], -(double)sinM[t]);
         if (p->fft.blue) {
-            // Bluestein: X_k = conj(b_k) sum_n (x_n conj(b_n)) b_{k-n}, b_n = e^{i pi n^2 / N};
-            // the convolution kernel B (b_m at m and M - m) is even, so its spectrum is
-            // b_0 + 2 sum_{m>=1} b_m cos(2 pi m k / M); the inverse DFT conjugates the row.
-            chirp.resize(N);
-            std::vector<long double> br(N), bi(N);
+            // Bluestein: X_k = conj(b_k) sum_n (x_n conj(b_n)) b_{k-n}, b_n = e^{i pi n^2 / N}; bhat is
+            // the spectrum of the convolution kernel (b_m at m and M - m), in extended precision;
+            // the inverse DFT conjugates the row.
+            std::vector<LdCplx> b(M, LdCplx{0.0L, 0.0L}), B(M);
             for (int t = 0; t < N; ++t) {
                 const long long q = ((long long)t * t) % (2LL * N);
                 const long double ang = PI_L * q / N;
-                br[t] = cosl(ang);
-                bi[t] = sinl(ang);
-                chirp[t] = make_double2((double)br[t], -(double)bi[t]);
+                LdCplx v;
+                sincosl(ang, &v.im, &v.re);
+                b[t] = v;
+                if (t > 0) b[M - t] = v;
+                tw.push_back(make_double2((double)v.re, -(double)v.im));
             }
-            std::vector<long double> cosM(M);
-            for (int t = 0; t < M; ++t) cosM[t] = cosl(2.0L * PI_L * t / M);
-            bhat.resize(M);
-            for (int k = 0; k < M; ++k) {
-                long double re = br[0], im = bi[0];
-                long long idx = 0;
-                for (int m = 1; m < N; ++m) {
-                    idx += k;
-                    if (idx >= M) idx %= M;
-                    re += 2.0L * br[m] * cosM[idx];
-                    im += 2.0L * bi[m] * cosM[idx];
-                }
-                bhat[k] = make_double2((double)(re / M), (double)(im / M));
-            }
+            ld_dft(b.data(), B.data(), M, 1, cosM, sinM);
+            for (const LdCplx &v : B) tw.push_back(make_double2((double)(v.re / M), (double)(v.im / M)));
         }
     }
 
@@ -1951,8 +1975,10 @@ static int plan_tables(shtk_plan *p) {
     p->seglist = (int4 *)(p->segm + segm_len);
     RC_TRY(upload(&p->convscale, conv, "plan tables"));
     RC_TRY(upload(&p->tw, tw, "plan tables"));
-    RC_TRY(upload(&p->chirp, chirp, "plan tables"));
-    RC_TRY(upload(&p->bhat, bhat, "plan tables"));
+    if (p->fft.blue) {  // one array
+        p->chirp = p->tw + p->fft.nfft;
+        p->bhat = p->chirp + d.nlon;
+    }
 
     // Segment seeds, computed once on the device.
     const size_t nseed = (size_t)nseg_total * np;
