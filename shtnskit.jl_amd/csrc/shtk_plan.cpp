@@ -524,6 +524,27 @@ int check_precision(const shtk_plan *p, int precision, int lmax_limit) {
     return SHTK_OK;
 }
 
+// The contraction that a call of a given precision runs: the matrix-core ones where they are
+// the faster, otherwise the FP64 field groups, whose results are within any precision's.  A
+// matrix-core contraction pads the fields to 16s and the analysis the pairs to 256s (and
+// accumulates over blocks of 512), a field group takes 1 to 8; small sizes go to its prologues.
+// Whole calls in us, FP64 against split, against FP32, nlon 2048 (lmax, fields):
+//   synthesis  511, 16: 144, 173, 149     700, 16: 304, 313, 265    800, 16: 413, 399, 357
+//              900, 12: 418, 429, 394     1023, 12: 508, 510, 467   1023, 16: 638, 592, 538
+//              1023, 10: 426, 478, 441    1023, 28: 1046, 1078, 965
+//   analysis   511, 12: 141, 151, 138     700, 12: 280, 343, 308    1023, 12: 570, 583, 529
+//              511, 16: 164, 180, 173     1023, 24: 887, 1164, 1041 1023, 32: 1138, 1305, 1190
+//              1023, 16, 1536 latitudes: 878, 1661, 1567
+int contraction_prec(const shtk_plan *p, int prec, int nf, bool synth) {
+    if (prec == SHTK_PREC_FP64 || p->seg != shtk::DSEG) return prec;
+    const int lmax = p->d.lmax, pad = (nf + 15) / 16 * 16;
+    if (synth && prec == SHTK_PREC_SPLIT) return lmax >= 800 && 4 * pad <= 5 * nf ? prec : SHTK_PREC_FP64;
+    if (synth) return lmax >= 600 && 2 * pad <= 3 * nf ? prec : SHTK_PREC_FP64;
+    const int np = p->np, npad = (np + 255) / 256 * 256;
+    if (prec == SHTK_PREC_FP32 && lmax >= 500 && pad - nf <= 5 && np <= 512 && 10 * npad <= 11 * np) return prec;
+    return SHTK_PREC_FP64;
+}
+
 int norm_ltr(const shtk_plan *p, int ltr, int *out) {
     if (ltr < 0) ltr = p->d.lmax;
     if (ltr > p->d.lmax) return fail(SHTK_EINVAL, "ltr must be <= lmax");
@@ -1257,9 +1278,11 @@ int ensure_vshadow(shtk_plan *p) {
     return SHTK_OK;
 }
 
-// Split-precision vector transforms (launch_vsplit_coef / launch_vsplit_out):
-// sin(theta) V_theta and sin(theta) V_phi are scalar syntheses of degree
-// lmax + 1, and the analysis is two scalar analyses with the weights
+// Split-precision vector transforms of plans without 64-degree segments; the others
+// run the FP64 field groups, which are faster (32 fields at lmax 511: synthesis 515
+// us against 615 split and 534 FP32, analysis 507, 556 and 514; 4 at 1023: 385, 559,
+// 505 and 394, 594, 524).  launch_vsplit_coef / launch_vsplit_out: sin(theta)
+// V_theta and sin(theta) V_phi are scalar syntheses of degree lmax + 1, and the analysis is two scalar analyses with the weights
 // w/sin(theta) followed by a three-term combination, so both directions run
 // the companion plan's split contraction on 2 nf fields whose Fourier data are
 // the contiguous [V_theta fields][V_phi fields] of the workspace.
@@ -1298,28 +1321,22 @@ int run_vsplit_to_grid(shtk_plan *p, const Job &j, const void *S, const void *T,
     // result, after the split prologues have consumed C.
     const int m_lo = std::max(16, (p->d.lmax + 1) / 32);
     const int nm_lo = std::min(p->nm, (m_lo + p->d.mres - 1) / p->d.mres);
-    shtk::LegArgs a = p->seg == shtk::DSEG ? vscalar_args(p, j.ltr) : base_args(p, j.ltr);
+    shtk::LegArgs a = base_args(p, j.ltr);
     a.nm_run = nm_lo;
-    if (p->seg == shtk::DSEG)
-        HIP_TRY(shtk::launch_vcoef(S, T, C, ws + L.edge_off, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div, 0,
-                                   a, nf, st),
-                "vector coefficient combination");
-    else
-        HIP_TRY(shtk::launch_vspec_prep(S, T, C, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div,
-                                        0, p->qcc, p->coff, p->d.lmax, p->d.mres, nm_lo, in_fs, nf, st),
-                "coefficient scaling");
+    HIP_TRY(shtk::launch_vspec_prep(S, T, C, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div, 0,
+                                    p->qcc, p->coff, p->d.lmax, p->d.mres, nm_lo, in_fs, nf, st),
+            "coefficient scaling");
     a.in0 = C;
-    if (p->seg == shtk::DSEG) a.edge = (const double2 *)(ws + L.edge_off);
     a.F0 = F0;
     a.F1 = F1;
     a.wlat = nullptr;  // sin(theta) V, as the split result
     a.g = j.g;
-    HIP_TRY(timed(p, "leg_synth_sphtor_low", st, [&] { return leg_synth_vector(p, a, nf, st); }),
+    HIP_TRY(timed(p, "leg_synth_sphtor_low", st,
+                  [&] { return shtk::launch_leg_synth(a, nf, 1, p->vsynth_chains, st); }),
             "Legendre synthesis launch");
     // grids with poles: order-1 pole rows from the limits (the phi transform divides
     // those rows by 1), Robert form: every pole row zero
     if (p->poles && (p->d.robert_form || (p->d.mres == 1 && p->d.mmax >= 1))) {
-        if (p->seg == shtk::DSEG) RC_TRY(vpole_records(p, j, a, S, T, C, nf, dtype, st));
         HIP_TRY(shtk::launch_vpole_synth(a, nf, p->d.robert_form, 1.0, st), "pole rows launch");
     }
     void *grids[2] = {Vt, Vp};
@@ -1520,9 +1537,13 @@ int batch_split(shtk_batch *b, int dir, const void *const *in, void *const *out,
 
 // One direction of a batch, eagerly (no graph).
 int batch_issue(shtk_batch *b, int dir, const void *const *in, void *const *out, int dtype, hipStream_t st) {
-    if (b->precision == SHTK_PREC_SPLIT) return batch_split(b, dir, in, out, dtype, st);
-    // FP64 and FP32: one configuration at a time, largest first (a captured graph
-    // replays the whole sequence with one launch)
+    bool split = b->precision == SHTK_PREC_SPLIT;
+    for (int gi = 0; gi < b->ngroups; ++gi)
+        split &= contraction_prec(b->plans[gi], b->precision, b->nf[gi], dir == 0) == SHTK_PREC_SPLIT;
+    if (split) return batch_split(b, dir, in, out, dtype, st);
+    // otherwise one configuration at a time, largest first (a captured graph replays the
+    // whole sequence with one launch): 10 to 16 fields at five lmax from 1023 to 63 as split
+    // groups 715 + 793 us, one by one 566 + 673
     for (int q = 0; q < b->ngroups; ++q) {
         const int gi = b->order[q];
         const int rc = dir == 0 ? shtk_synthesis_ex(b->plans[gi], in[gi], out[gi], b->nf[gi], dtype, 1, -1,
@@ -1540,10 +1561,14 @@ int batch_prepare(shtk_batch *b, int dtype, hipStream_t st) {
         shtk_plan *p = b->plans[gi];
         std::lock_guard<std::recursive_mutex> lk(p->mu);
         RC_TRY(ensure_ws(p, ws_layout(p, b->nf[gi], 0).total));
-        if (b->precision == SHTK_PREC_SPLIT) {
+        const int prec = b->precision;
+        if (contraction_prec(p, prec, b->nf[gi], true) == SHTK_PREC_FP64 &&
+            contraction_prec(p, prec, b->nf[gi], false) == SHTK_PREC_FP64)
+            continue;
+        if (prec == SHTK_PREC_SPLIT) {
             RC_TRY(ensure_oz_tables(p, st));
             RC_TRY(ensure_oz_ws(p, oz_ws_bytes(p, b->nf[gi], !p->canonical || dtype != SHTK_F64)));
-        } else if (b->precision == SHTK_PREC_FP32) {
+        } else if (prec == SHTK_PREC_FP32) {
             RC_TRY(ensure_oz_tables(p, st));
             RC_TRY(ensure_oz_ws(p, f32_ws_bytes(p, b->nf[gi], !p->canonical || dtype != SHTK_F64)));
         }
@@ -2191,7 +2216,7 @@ int shtk_synthesis_ex(shtk_plan *p, const void *alm, void *f, int nfields, int d
     // of the inverse FFT folded in g; complex output (src/core_transforms.jl:294-344):
     // the bins m >= 0 alone, f = ifft(phi_inv_scale * F)
     Job j{0, 0, nullptr, p->inv_scale / p->d.nlon, 0, 0, 0, ltr, "leg_synth", "fft_synth"};
-    j.prec = precision;
+    j.prec = contraction_prec(p, precision, nfields, true);
     j.cplx_out = real_output != 1;
     return run_to_grid(p, j, alm, nullptr, f, nullptr, nfields, dtype, stream);
 }
@@ -2202,7 +2227,7 @@ int shtk_analysis_ex(shtk_plan *p, const void *f, void *alm, int nfields, int dt
     RC_TRY(check_precision(p, precision, 4095));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     Job j{0, 1, p->wscaled, 1.0, 0, 0, 0, ltr, "leg_anal", "fft_anal"};
-    j.prec = precision;
+    j.prec = contraction_prec(p, precision, nfields, false);
     return run_to_spec(p, j, f, nullptr, alm, nullptr, nfields, dtype, stream);
 }
 
@@ -2212,7 +2237,7 @@ int shtk_analysis_cplx(shtk_plan *p, const void *f, void *alm, int nfields, int 
     RC_TRY(check_precision(p, precision, 4095));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     Job j{0, 1, p->wscaled, 1.0, 0, 0, 0, ltr, "leg_anal", "fft_anal"};
-    j.prec = precision;
+    j.prec = contraction_prec(p, precision, nfields, false);
     j.cplx_in = 1;
     return run_to_spec(p, j, f, nullptr, alm, nullptr, nfields, dtype, stream);
 }
@@ -2282,6 +2307,8 @@ int shtk_synthesis_sphtor_ex(shtk_plan *p, const void *S, const void *T, void *V
     if (precision == SHTK_PREC_FP64)
         return shtk_synthesis_sphtor(p, S, T, Vt, Vp, nfields, dtype, real_output, ltr, stream);
     RC_TRY(check_precision(p, precision, 4094));
+    if (p && p->seg == shtk::DSEG)
+        return shtk_synthesis_sphtor(p, S, T, Vt, Vp, nfields, dtype, real_output, ltr, stream);
     RC_TRY(check_common(p, nfields, dtype, {S, T, Vt, Vp}));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     // the contraction gives sin(theta) V; the phi FFT divides by sin(theta) unless Robert form
@@ -2296,6 +2323,7 @@ int shtk_analysis_sphtor_ex(shtk_plan *p, const void *Vt, const void *Vp, void *
                             int ltr, int precision, void *stream) {
     if (precision == SHTK_PREC_FP64) return shtk_analysis_sphtor(p, Vt, Vp, S, T, nfields, dtype, ltr, stream);
     RC_TRY(check_precision(p, precision, 4094));
+    if (p && p->seg == shtk::DSEG) return shtk_analysis_sphtor(p, Vt, Vp, S, T, nfields, dtype, ltr, stream);
     RC_TRY(check_common(p, nfields, dtype, {S, T, Vt, Vp}));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     if (p->pole_weights && p->d.robert_form && p->d.mres == 1 && p->d.mmax >= 1 && ltr >= 1)
