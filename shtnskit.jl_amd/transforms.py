@@ -71,13 +71,21 @@ def _adapt(x, adapt: bool, op: str):
 
 def _colmajor(t: torch.Tensor) -> torch.Tensor:
     """Same logical tensor with Julia column-major memory (first index fastest)."""
-    perm = list(range(t.dim() - 1, -1, -1))
-    return t.permute(*perm).contiguous().permute(*perm)
+    want = 1
+    for n, s in zip(t.shape, t.stride()):
+        if n != 1 and s != want:
+            perm = list(range(t.dim() - 1, -1, -1))
+            return t.permute(*perm).contiguous().permute(*perm)
+        want *= n
+    return t
 
 
 def _empty_colmajor(shape, dtype, device) -> torch.Tensor:
-    perm = list(range(len(shape) - 1, -1, -1))
-    return torch.empty([shape[p] for p in perm], dtype=dtype, device=device).permute(*perm)
+    strides, n = [], 1
+    for k in shape:
+        strides.append(n)
+        n *= max(k, 1)
+    return torch.empty_strided(shape, strides, dtype=dtype, device=device)
 
 
 def _real_dtype(t: torch.Tensor) -> torch.dtype:
@@ -97,7 +105,7 @@ def _cplx(rdt: torch.dtype) -> torch.dtype:
 
 
 def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))  # no Stream object per call
 
 
 def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
