@@ -480,7 +480,7 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
 
 template <int NG, bool VEC>
 void launch_synth_sf(const LegArgs &a, hipStream_t st) {
-    const long long units = (long long)a.nm * a.gx * a.gz;
+    const long long units = (long long)(a.nm_run > 0 ? std::min(a.nm_run, a.nm) : a.nm) * a.gx * a.gz;
     // 2 waves per unit where one would leave the chip short of waves (4096 units, 16
     // fields at lmax 511: 65 -> 62 us; 16384, 16 at 1023: 429 against 432; 4 waves lose
     // the accumulator traffic through LDS: 98 us at 511)
@@ -664,15 +664,16 @@ hipError_t launch_vcoef(const void *S, const void *T, void *C, void *E, int in_f
                         const LegArgs &v, int nf, hipStream_t st) {
     const int lmax = v.lmax - 1, ltr = v.ltr - 1;
     const long long in_fs = (long long)(lmax + 1) * (v.mmax + 1);
-    const dim3 grid((unsigned)v.nm * nf);
+    const int nm = v.nm_run > 0 ? std::min(v.nm_run, v.nm) : v.nm;
+    const dim3 grid((unsigned)nm * nf);
     if (in_f32)
         hipLaunchKernelGGL(k_vcoef<float>, grid, dim3(256), 0, st, (const float *)S, (const float *)T, (double2 *)C,
                            (double2 *)E, v.segbase, v.nseg_total, scale, divide, ll1, v.qb, v.qcc, v.coff, lmax, v.mres,
-                           v.nm, ltr, v.m0_one, in_fs, v.spec_fstride, nf);
+                           nm, ltr, v.m0_one, in_fs, v.spec_fstride, nf);
     else
         hipLaunchKernelGGL(k_vcoef<double>, grid, dim3(256), 0, st, (const double *)S, (const double *)T, (double2 *)C,
                            (double2 *)E, v.segbase, v.nseg_total, scale, divide, ll1, v.qb, v.qcc, v.coff, lmax, v.mres,
-                           v.nm, ltr, v.m0_one, in_fs, v.spec_fstride, nf);
+                           nm, ltr, v.m0_one, in_fs, v.spec_fstride, nf);
     return hipGetLastError();
 }
 

@@ -535,13 +535,22 @@ int check_precision(const shtk_plan *p, int precision, int lmax_limit) {
 //   analysis   511, 12: 141, 151, 138     700, 12: 280, 343, 308    1023, 12: 570, 583, 529
 //              511, 16: 164, 180, 173     1023, 24: 887, 1164, 1041 1023, 32: 1138, 1305, 1190
 //              1023, 16, 1536 latitudes: 878, 1661, 1567
-int contraction_prec(const shtk_plan *p, int prec, int nf, bool synth) {
+// FP64 arrays in FP32 precision keep the FP32 kernels: a caller that compares runs in that
+// precision gets the values it always got, which the FP64 groups match to 2e-7 only.
+int contraction_prec(const shtk_plan *p, int prec, int nf, int dtype, bool synth) {
     if (prec == SHTK_PREC_FP64 || p->seg != shtk::DSEG) return prec;
+    if (prec == SHTK_PREC_FP32 && dtype == SHTK_F64) return prec;
     const int lmax = p->d.lmax, pad = (nf + 15) / 16 * 16;
     if (synth && prec == SHTK_PREC_SPLIT) return lmax >= 800 && 4 * pad <= 5 * nf ? prec : SHTK_PREC_FP64;
     if (synth) return lmax >= 600 && 2 * pad <= 3 * nf ? prec : SHTK_PREC_FP64;
     const int np = p->np, npad = (np + 255) / 256 * 256;
     if (prec == SHTK_PREC_FP32 && lmax >= 500 && pad - nf <= 5 && np <= 512 && 10 * npad <= 11 * np) return prec;
+    return SHTK_PREC_FP64;
+}
+
+// The same for the vector pair, whose field groups are always the faster.
+int vector_prec(const shtk_plan *p, int prec, int dtype) {
+    if (p->seg != shtk::DSEG || (prec == SHTK_PREC_FP32 && dtype == SHTK_F64)) return prec;
     return SHTK_PREC_FP64;
 }
 
@@ -1278,11 +1287,12 @@ int ensure_vshadow(shtk_plan *p) {
     return SHTK_OK;
 }
 
-// Split-precision vector transforms of plans without 64-degree segments; the others
-// run the FP64 field groups, which are faster (32 fields at lmax 511: synthesis 515
-// us against 615 split and 534 FP32, analysis 507, 556 and 514; 4 at 1023: 385, 559,
-// 505 and 394, 594, 524).  launch_vsplit_coef / launch_vsplit_out: sin(theta)
-// V_theta and sin(theta) V_phi are scalar syntheses of degree lmax + 1, and the analysis is two scalar analyses with the weights
+// Matrix-core vector transforms: of FP64 arrays in FP32 precision, and of plans without
+// 64-degree segments; the others run the FP64 field groups, which are faster (32
+// fields at lmax 511: synthesis 515 us against 615 split and 534 FP32, analysis 507,
+// 556 and 514; 4 at 1023: 385, 559, 505 and 394, 594, 524).
+// launch_vsplit_coef / launch_vsplit_out: sin(theta) V_theta and sin(theta) V_phi
+// are scalar syntheses of degree lmax + 1, and the analysis is two scalar analyses with the weights
 // w/sin(theta) followed by a three-term combination, so both directions run
 // the companion plan's split contraction on 2 nf fields whose Fourier data are
 // the contiguous [V_theta fields][V_phi fields] of the workspace.
@@ -1321,22 +1331,28 @@ int run_vsplit_to_grid(shtk_plan *p, const Job &j, const void *S, const void *T,
     // result, after the split prologues have consumed C.
     const int m_lo = std::max(16, (p->d.lmax + 1) / 32);
     const int nm_lo = std::min(p->nm, (m_lo + p->d.mres - 1) / p->d.mres);
-    shtk::LegArgs a = base_args(p, j.ltr);
+    shtk::LegArgs a = p->seg == shtk::DSEG ? vscalar_args(p, j.ltr) : base_args(p, j.ltr);
     a.nm_run = nm_lo;
-    HIP_TRY(shtk::launch_vspec_prep(S, T, C, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div, 0,
-                                    p->qcc, p->coff, p->d.lmax, p->d.mres, nm_lo, in_fs, nf, st),
-            "coefficient scaling");
+    if (p->seg == shtk::DSEG)
+        HIP_TRY(shtk::launch_vcoef(S, T, C, ws + L.edge_off, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale,
+                                   j.conv_div, 0, a, nf, st),
+                "vector coefficient combination");
+    else
+        HIP_TRY(shtk::launch_vspec_prep(S, T, C, dtype == SHTK_F32, p->canonical ? nullptr : p->convscale, j.conv_div,
+                                        0, p->qcc, p->coff, p->d.lmax, p->d.mres, nm_lo, in_fs, nf, st),
+                "coefficient scaling");
     a.in0 = C;
+    if (p->seg == shtk::DSEG) a.edge = (const double2 *)(ws + L.edge_off);
     a.F0 = F0;
     a.F1 = F1;
     a.wlat = nullptr;  // sin(theta) V, as the split result
     a.g = j.g;
-    HIP_TRY(timed(p, "leg_synth_sphtor_low", st,
-                  [&] { return shtk::launch_leg_synth(a, nf, 1, p->vsynth_chains, st); }),
+    HIP_TRY(timed(p, "leg_synth_sphtor_low", st, [&] { return leg_synth_vector(p, a, nf, st); }),
             "Legendre synthesis launch");
     // grids with poles: order-1 pole rows from the limits (the phi transform divides
     // those rows by 1), Robert form: every pole row zero
     if (p->poles && (p->d.robert_form || (p->d.mres == 1 && p->d.mmax >= 1))) {
+        if (p->seg == shtk::DSEG) RC_TRY(vpole_records(p, j, a, S, T, C, nf, dtype, st));
         HIP_TRY(shtk::launch_vpole_synth(a, nf, p->d.robert_form, 1.0, st), "pole rows launch");
     }
     void *grids[2] = {Vt, Vp};
@@ -1539,7 +1555,7 @@ int batch_split(shtk_batch *b, int dir, const void *const *in, void *const *out,
 int batch_issue(shtk_batch *b, int dir, const void *const *in, void *const *out, int dtype, hipStream_t st) {
     bool split = b->precision == SHTK_PREC_SPLIT;
     for (int gi = 0; gi < b->ngroups; ++gi)
-        split &= contraction_prec(b->plans[gi], b->precision, b->nf[gi], dir == 0) == SHTK_PREC_SPLIT;
+        split &= contraction_prec(b->plans[gi], b->precision, b->nf[gi], dtype, dir == 0) == SHTK_PREC_SPLIT;
     if (split) return batch_split(b, dir, in, out, dtype, st);
     // otherwise one configuration at a time, largest first (a captured graph replays the
     // whole sequence with one launch): 10 to 16 fields at five lmax from 1023 to 63 as split
@@ -1562,8 +1578,8 @@ int batch_prepare(shtk_batch *b, int dtype, hipStream_t st) {
         std::lock_guard<std::recursive_mutex> lk(p->mu);
         RC_TRY(ensure_ws(p, ws_layout(p, b->nf[gi], 0).total));
         const int prec = b->precision;
-        if (contraction_prec(p, prec, b->nf[gi], true) == SHTK_PREC_FP64 &&
-            contraction_prec(p, prec, b->nf[gi], false) == SHTK_PREC_FP64)
+        if (contraction_prec(p, prec, b->nf[gi], dtype, true) == SHTK_PREC_FP64 &&
+            contraction_prec(p, prec, b->nf[gi], dtype, false) == SHTK_PREC_FP64)
             continue;
         if (prec == SHTK_PREC_SPLIT) {
             RC_TRY(ensure_oz_tables(p, st));
@@ -2216,7 +2232,7 @@ int shtk_synthesis_ex(shtk_plan *p, const void *alm, void *f, int nfields, int d
     // of the inverse FFT folded in g; complex output (src/core_transforms.jl:294-344):
     // the bins m >= 0 alone, f = ifft(phi_inv_scale * F)
     Job j{0, 0, nullptr, p->inv_scale / p->d.nlon, 0, 0, 0, ltr, "leg_synth", "fft_synth"};
-    j.prec = contraction_prec(p, precision, nfields, true);
+    j.prec = contraction_prec(p, precision, nfields, dtype, true);
     j.cplx_out = real_output != 1;
     return run_to_grid(p, j, alm, nullptr, f, nullptr, nfields, dtype, stream);
 }
@@ -2227,7 +2243,7 @@ int shtk_analysis_ex(shtk_plan *p, const void *f, void *alm, int nfields, int dt
     RC_TRY(check_precision(p, precision, 4095));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     Job j{0, 1, p->wscaled, 1.0, 0, 0, 0, ltr, "leg_anal", "fft_anal"};
-    j.prec = contraction_prec(p, precision, nfields, false);
+    j.prec = contraction_prec(p, precision, nfields, dtype, false);
     return run_to_spec(p, j, f, nullptr, alm, nullptr, nfields, dtype, stream);
 }
 
@@ -2237,7 +2253,7 @@ int shtk_analysis_cplx(shtk_plan *p, const void *f, void *alm, int nfields, int 
     RC_TRY(check_precision(p, precision, 4095));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     Job j{0, 1, p->wscaled, 1.0, 0, 0, 0, ltr, "leg_anal", "fft_anal"};
-    j.prec = contraction_prec(p, precision, nfields, false);
+    j.prec = contraction_prec(p, precision, nfields, dtype, false);
     j.cplx_in = 1;
     return run_to_spec(p, j, f, nullptr, alm, nullptr, nfields, dtype, stream);
 }
@@ -2307,7 +2323,7 @@ int shtk_synthesis_sphtor_ex(shtk_plan *p, const void *S, const void *T, void *V
     if (precision == SHTK_PREC_FP64)
         return shtk_synthesis_sphtor(p, S, T, Vt, Vp, nfields, dtype, real_output, ltr, stream);
     RC_TRY(check_precision(p, precision, 4094));
-    if (p && p->seg == shtk::DSEG)
+    if (p && vector_prec(p, precision, dtype) == SHTK_PREC_FP64)
         return shtk_synthesis_sphtor(p, S, T, Vt, Vp, nfields, dtype, real_output, ltr, stream);
     RC_TRY(check_common(p, nfields, dtype, {S, T, Vt, Vp}));
     RC_TRY(norm_ltr(p, ltr, &ltr));
@@ -2323,7 +2339,8 @@ int shtk_analysis_sphtor_ex(shtk_plan *p, const void *Vt, const void *Vp, void *
                             int ltr, int precision, void *stream) {
     if (precision == SHTK_PREC_FP64) return shtk_analysis_sphtor(p, Vt, Vp, S, T, nfields, dtype, ltr, stream);
     RC_TRY(check_precision(p, precision, 4094));
-    if (p && p->seg == shtk::DSEG) return shtk_analysis_sphtor(p, Vt, Vp, S, T, nfields, dtype, ltr, stream);
+    if (p && vector_prec(p, precision, dtype) == SHTK_PREC_FP64)
+        return shtk_analysis_sphtor(p, Vt, Vp, S, T, nfields, dtype, ltr, stream);
     RC_TRY(check_common(p, nfields, dtype, {S, T, Vt, Vp}));
     RC_TRY(norm_ltr(p, ltr, &ltr));
     if (p->pole_weights && p->d.robert_form && p->d.mres == 1 && p->d.mmax >= 1 && ltr >= 1)
