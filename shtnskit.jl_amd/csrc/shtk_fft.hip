@@ -67,6 +67,37 @@ __device__ __forceinline__ void dft_small(double2 *v) {
         v[6] = csub(e[2], o2);
         v[3] = cadd(e[3], o3);
         v[7] = csub(e[3], o3);
+    } else if constexpr (R == 16) {
+        // 4 x 4: columns r, r + 4, .. then W16^(rk), then rows
+        constexpr double c1 = 0.92387953251128675613, s1 = 0.38268343236508977173, h = 0.70710678118654752440;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            double2 t[4] = {v[r], v[r + 4], v[r + 8], v[r + 12]};
+            dft_small<4, SIGN>(t);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[r + 4 * k] = t[k];
+        }
+        // v[r + 4 k] times W16^(r k)
+        v[5] = cmul(v[5], make_double2(c1, SIGN * s1));
+        v[6] = cmul(v[6], make_double2(h, SIGN * h));
+        v[7] = cmul(v[7], make_double2(s1, SIGN * c1));
+        v[9] = cmul(v[9], make_double2(h, SIGN * h));
+        v[10] = mul_si<SIGN>(v[10]);
+        v[11] = cmul(v[11], make_double2(-h, SIGN * h));
+        v[13] = cmul(v[13], make_double2(s1, SIGN * c1));
+        v[14] = cmul(v[14], make_double2(-h, SIGN * h));
+        v[15] = cmul(v[15], make_double2(-c1, -SIGN * s1));
+        // output k + 4 q of row k
+        double2 o[16];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            double2 t[4] = {v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+            dft_small<4, SIGN>(t);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[k + 4 * q] = t[q];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = o[r];
     } else if constexpr (R == 3) {
         constexpr double c1 = -0.5, s1 = 0.86602540378443864676;
         const double2 a = v[0], b = v[1], c = v[2];
@@ -132,7 +163,10 @@ struct NsDiv {
 enum { BLUE_NONE = 0, BLUE_FIRST = 1, BLUE_MID = 2, BLUE_LAST = 3 };
 
 // One Stockham pass of radix R over the LDS row z (length N).  Every thread
-// stages all its inputs in registers before the barrier, then writes.
+// stages all its inputs in registers before the barrier, then writes.  Radix 16 leaves half
+// the threads of a row without a butterfly and saves a pass in three or four: no gain for
+// direct lengths (16 fields at nlon 2048: synthesis 174 to 179 us with either, analysis 206
+// and 221), but Bluestein's, which are bound by the passes, take powers of two in 5, not 7.
 template <int R, int SIGN, bool P2, bool BLUE>
 __device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const double2 *tw, int tid, int nt,
                                               const FftArgs &a, int what) {
@@ -144,11 +178,15 @@ __device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const d
     const NsDiv<P2> dv(Ns);
     // base twiddle w = W^(k stride) of each butterfly (the others are its
     // powers): independent of the LDS data, so its load overlaps the barrier
-    double2 w1[MAXB];
+    double2 w1[MAXB], w4 = make_double2(1.0, 0.0), w8 = w4;
 #pragma unroll
     for (int q = 0; q < MAXB; ++q) {
         const int j = tid + q * nt;
         w1[q] = (Ns > 1 && j < nb) ? tw[dv.mod(j) * stride] : make_double2(1.0, 0.0);
+        if (R == 16 && Ns > 1 && j < nb) {  // radix 16: the powers 4 and 8 too (shorter products)
+            w4 = tw[4 * dv.mod(j) * stride];
+            w8 = tw[8 * dv.mod(j) * stride];
+        }
     }
     double2 v[MAXB][R];
 #pragma unroll
@@ -180,11 +218,28 @@ __device__ __forceinline__ void stockham_pass(double2 *z, int N, int Ns, const d
             if (Ns > 1) {
                 double2 w = w1[q];
                 if (DS > 0) w.y = -w.y;
-                double2 wr = w;
+                if constexpr (R == 16) {
+                    if (DS > 0) {
+                        w4.y = -w4.y;
+                        w8.y = -w8.y;
+                    }
+                    const double2 w2 = cmul(w, w), w3 = cmul(w2, w);
+                    const double2 wl[3] = {w, w2, w3}, wh[3] = {w4, w8, cmul(w8, w4)};
 #pragma unroll
-                for (int r = 1; r < R; ++r) {
-                    v[q][r] = cmul(v[q][r], wr);
-                    if (r + 1 < R) wr = cmul(wr, w);
+                    for (int r = 1; r < 4; ++r) v[q][r] = cmul(v[q][r], wl[r - 1]);
+#pragma unroll
+                    for (int g = 1; g < 4; ++g) {
+                        v[q][4 * g] = cmul(v[q][4 * g], wh[g - 1]);
+#pragma unroll
+                        for (int r = 1; r < 4; ++r) v[q][4 * g + r] = cmul(v[q][4 * g + r], cmul(wh[g - 1], wl[r - 1]));
+                    }
+                } else {
+                    double2 wr = w;
+#pragma unroll
+                    for (int r = 1; r < R; ++r) {
+                        v[q][r] = cmul(v[q][r], wr);
+                        if (r + 1 < R) wr = cmul(wr, w);
+                    }
                 }
             }
             dft_small<R, DS>(v[q]);
@@ -335,7 +390,7 @@ __device__ __forceinline__ void stockham_gen(double2 *z, int N, int Ns, int R, c
 // The pass loops hide the thread's index from the optimiser: the addresses of every pass
 // depend on it and the length alone, and kept over the loop they filled the registers and
 // 340 to 600 bytes of scratch per thread.  Whole calls: 16 fields at lmax 700, nlon 1402
-// (Bluestein): 895 -> 455 us; 8 at 1000, nlon 2002 = 2 * 7 * 11 * 13: 672 -> 359; 32 at
+// (Bluestein): 895 -> 421 us; 8 at 1000, nlon 2002 = 2 * 7 * 11 * 13: 672 -> 359; 32 at
 // 303, nlon 608 = 32 * 19: 173 -> 82 (nlon 640: 75); one: 29 -> 19.
 template <int SIGN, int KIND>
 __device__ __forceinline__ void fft_lds(double2 *z, const FftArgs &a, int tid, int nt) {
@@ -348,6 +403,7 @@ __device__ __forceinline__ void fft_lds(double2 *z, const FftArgs &a, int tid, i
             const int R = rad(q <= mid ? q : 2 * mid - q);
             const int what = q == 0 ? BLUE_FIRST : q == mid ? BLUE_MID : q == np - 1 ? BLUE_LAST : BLUE_NONE;
             switch (R) {
+                case 16: stockham_pass<16, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
                 case 8: stockham_pass<8, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
                 case 4: stockham_pass<4, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;
                 case 2: stockham_pass<2, SIGN, false, true>(z, M, Ns, a.tw, tid, nt, a, what); break;

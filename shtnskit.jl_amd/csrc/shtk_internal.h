@@ -138,7 +138,7 @@ struct SeedArgs {
 };
 
 // FFT factorisations: FFT_RADIX_BITS bits per pass, first pass in the low bits.
-// Radices 2, 3, 4, 5, 8 and the primes 7 to FFT_PRIME_MAX have butterflies; other
+// Radices 2, 3, 4, 5, 8, 16 and the primes 7 to FFT_PRIME_MAX have butterflies; other
 // primes up to FFT_GEN_MAX run a generic pass (R table twiddles per output).
 // Lengths whose other prime factors would cost more take Bluestein's algorithm: a
 // circular convolution of length nfft >= 2 nlon - 1 (2^a 3^b 5^c) through two FFTs.

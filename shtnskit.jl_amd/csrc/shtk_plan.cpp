@@ -195,9 +195,9 @@ double coef_scale(const shtk_desc &d, int l, int m) {
 }
 
 // Pass radices of one FFT length: primes from 7 up to FFT_GEN_MAX, largest first
-// (the first pass needs no twiddles), then 8, 4, 2, 3, 5.  *sum: the sum of those
-// primes; *gen_sum: of the ones that run the generic pass.
-bool factor_len(int n, std::vector<int> &r, int *sum, int *gen_sum) {
+// (the first pass needs no twiddles), then 16 (r16: convolution lengths), 8, 4, 2, 3,
+// 5.  *sum: the sum of those primes; *gen_sum: of the ones that run the generic pass.
+bool factor_len(int n, std::vector<int> &r, bool r16, int *sum, int *gen_sum) {
     r.clear();
     *sum = *gen_sum = 0;
     for (int q = shtk::FFT_GEN_MAX; q >= 7; --q) {
@@ -209,6 +209,15 @@ bool factor_len(int n, std::vector<int> &r, int *sum, int *gen_sum) {
             n /= q;
         }
     }
+    // as few passes for the power of two as radix 16 allows, with as few of radix 16 as that
+    // takes (2048: 16, 16, 8)
+    int a = 0;
+    while (n % (2 << a) == 0) ++a;
+    if (r16)
+        for (int y = a - 3 * ((a + 3) / 4); y > 0; --y) {
+            r.push_back(16);
+            n /= 16;
+        }
     for (int c : {8, 4, 2, 3, 5})
         while (n % c == 0) {
             r.push_back(c);
@@ -219,7 +228,9 @@ bool factor_len(int n, std::vector<int> &r, int *sum, int *gen_sum) {
 
 // The longitude FFT of length n: direct mixed-radix passes when its factors have
 // butterflies or one prime up to FFT_GEN_BUDGET runs the generic pass, otherwise
-// Bluestein's algorithm with the shortest 2^a 3^b 5^c convolution length >= 2n - 1.
+// Bluestein's algorithm with the 2^a 3^b 5^c convolution length >= 2n - 1 whose LDS
+// traffic, length times passes, is least (nlon 607, 32 fields: 1215 in 11 passes 176 us,
+// 2048 in 5 140; 1402, 16 fields: 2880 in 9 455 us, 4096 in 5 421).
 // A generic pass of prime R reads R values per output, so Bluestein's nine or so passes
 // of twice the length meet it between 23 and 31 (synthesis, generic against Bluestein:
 // nlon 1392 = 48 * 29, 16 fields, 434 and 441 us; 682 = 22 * 31, 24 fields, 140 and 156;
@@ -231,21 +242,27 @@ shtk::FftPlan make_fft_plan(int n) {
     shtk::FftPlan f;
     if (n < 1 || n > shtk::FFT_MAX_LEN) return f;
     int sum = 0, gs = 0;
-    if (factor_len(n, f.radix, &sum, &gs) &&
+    if (factor_len(n, f.radix, false, &sum, &gs) &&
         (2 * n - 1 > shtk::FFT_MAX_LEN ? sum <= shtk::FFT_LONG_BUDGET : gs <= shtk::FFT_GEN_BUDGET)) {
         f.ok = true;
         f.nfft = n;
         return f;
     }
-    for (int m = 2 * n - 1; m <= shtk::FFT_MAX_LEN; ++m) {
+    long long best = 0;
+    for (int m = 2 * n - 1; m <= std::min(shtk::FFT_MAX_LEN, 4 * n); ++m) {
         int t = m;
         for (int c : {2, 3, 5})
             while (t % c == 0) t /= c;
-        if (t != 1 || !factor_len(m, f.radix, &sum, &gs) || f.radix.size() < 2) continue;
+        std::vector<int> r;
+        if (t != 1 || !factor_len(m, r, true, &sum, &gs) || r.size() < 2) continue;
+        const long long cost = (long long)m * (2 * (int)r.size() - 1);
+        if (f.blue && cost >= best) continue;
+        best = cost;
         f.ok = f.blue = true;
         f.nfft = m;
-        return f;
+        f.radix = r;
     }
+    if (f.ok) return f;
     f.radix.clear();
     return f;
 }

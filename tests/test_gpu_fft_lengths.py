@@ -18,7 +18,7 @@ TOL = 1e-12
 
 # nlon: kind
 LENGTHS = [7, 49, 56, 11, 13, 143, 17, 221, 19, 361, 608, 1001, 23, 46, 667, 61, 67, 134, 131, 499, 1018, 2039, 4093,
-           8190]
+           8190, 16, 48, 128, 256, 2048, 4096, 8192]
 
 
 @pytest.mark.parametrize("nlon", LENGTHS)
