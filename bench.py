@@ -8,9 +8,9 @@ orthonormal + Condon-Shortley, input alm complex Gaussian (seed 2) scaled by
 `value` is round trips per second.
 
 Second measured line (`split_batched`): the same grid, a batch of 16 fields
-(seed 2, same spectrum), synthesis_batch then analysis_batch with the
-split-precision contraction on the int8 matrix cores; its value is field round
-trips per second of the whole batch, with the per-field relative L2 error
+(seed 2, same spectrum), synthesis_batch then analysis_batch in split precision
+(the int8 matrix cores, or the FP64 field groups where these are the faster);
+its value is field round trips per second of the whole batch, with the per-field relative L2 error
 against the FP64 path.
 
 Inputs are resident in HBM before every timed region.  `value` comes from K
@@ -306,7 +306,7 @@ def measure_uneven(torch, np, shtk, dev, steps):
             "fp32_path_value": round(1000.0 * 64 / fp32_ms, 2),
             "max_field_rel_l2_vs_fp64_path": err, "fp32_max_field_rel_l2_vs_fp64_path": err32,
             "autotuned": tune,
-            "launches": "one hipGraph per direction; Legendre stages as persistent kernels over all groups"}
+            "launches": "one hipGraph per direction; one configuration after the other"}
 
 
 def sphtor_spectrum(np, lmax, nfields, seed):
@@ -514,6 +514,13 @@ def main() -> int:
             sroof = roofline_entry(dom, sk_us[dom], ops, PEAK_INT8_TOPS, "TOP/s", "mfma",
                                    f"{ops:.4e} int8 ops = 21 slice products x 2 x (nlat/2)(lmax+1)(lmax+2)/2 "
                                    f"x 2 x {nf} fields")
+        elif dom.startswith("leg"):  # FP64 field groups; no committed traffic figure for a batch
+            # a recurrence step (4 flops) serves up to 8 fields, the contraction is 4 per field
+            fl = 4.0 * n_triples(LMAX, NLAT) * (nf + (nf + 7) // 8)
+            sroof = roofline_entry(dom, sk_us[dom], fl, PEAK_FP64_TFLOPS, "TFLOP/s", "mfma",
+                                   f"{fl:.4e} flop = 4 x (nlat/2) x (lmax+1)(lmax+2)/2 x ({nf} fields + "
+                                   f"{(nf + 7) // 8} recurrences) (FP64)")
+            sroof["traffic"] = None
         else:
             by = fft_bytes(NLAT, NLON, LMAX, nf)
             sroof = roofline_entry(dom, sk_us[dom], by * 1e3, PEAK_HBM_GBS, "GB/s", "hbm", f"{by:.4e} bytes")
@@ -526,7 +533,7 @@ def main() -> int:
             "ms_per_batch_round_trip": round(ms_batch, 5),
             "ms_per_batch_with_kernel_events": round(s_ev / ssteps, 5),
             "speedup_vs_plain": round((1000.0 * nf / ms_batch) / res["value"], 3),
-            "dtype": "int8 MFMA slices of FP64 Legendre values, FP64 tables and cross-slice sums",
+            "dtype": "split precision: int8 MFMA slices of FP64 Legendre values with FP64 sums (oz_*), FP64 field groups (leg_*)",
             "max_field_rel_l2_vs_fp64_path": err_fp64,
             "max_field_rel_l2_round_trip": err_in,
             "config": {"workload": "batched split-precision scalar round trip (synthesis_batch+analysis_batch)",

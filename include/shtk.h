@@ -51,7 +51,10 @@ enum shtk_phi_scale { SHTK_PHI_DFT = 0, SHTK_PHI_QUAD = 1 };
 enum shtk_grid { SHTK_GRID_GAUSS = 0, SHTK_GRID_REGULAR = 1, SHTK_GRID_REGULAR_POLES = 2, SHTK_GRID_DRISCOLL_HEALY = 3 };
 enum shtk_dtype { SHTK_F64 = 0, SHTK_F32 = 1 };
 
-/* Contraction precision of the batched entry points (*_ex).
+/* Contraction precision of the batched entry points (*_ex).  Where the FP64 field
+ * groups are faster than a matrix-core contraction they run in its place, with
+ * results at least as close (never for FP64 arrays in SHTK_PREC_FP32, whose values
+ * stay those of the FP32 contraction).
  * SHTK_PREC_FP64: the FP64 recurrence-and-contraction kernels (the plain path).
  * SHTK_PREC_SPLIT: FP64 Legendre values and tables, contraction as an Ozaki
  *   split on int8 matrix cores (6 slices, exact int32 accumulation, FP64
@@ -243,9 +246,10 @@ int shtk_adjoint_analysis_sphtor_cplx(shtk_plan *plan, const void *Sb, const voi
  * Uneven batches: ngroups configurations (descs[g], nfields[g] fields each)
  * transformed together, e.g. many fields of different lmax.  The reference
  * handles such a set as one transform per field, or one batch call per
- * configuration (src/batch_transforms.jl:312-655); here every stage is one
- * launch for all groups: with SHTK_PREC_SPLIT the Legendre contractions run as
- * persistent kernels over a work queue ordered largest-first.  Arrays are
+ * configuration (src/batch_transforms.jl:312-655); here one object holds them and
+ * one graph launch can run them, one group after the other, largest first (groups
+ * that all stay on the split contraction share one launch per stage, its Legendre
+ * kernels persistent over a work queue).  Arrays are
  * passed per group (alm[g] of shape (lmax+1, mmax+1, nfields[g]), f[g] of
  * shape (nlat, nlon, nfields[g])); ngroups <= 8. */
 typedef struct shtk_batch shtk_batch;

@@ -3,11 +3,11 @@ transformed together through one batch object of libshtk_mi355x.so.
 
 The reference handles such a set one configuration (or one field) at a time,
 ``analysis_batch``/``synthesis_batch`` per configuration
-(src/batch_transforms.jl:312-655).  Here every stage is one launch for all
-configurations; with ``precision="split"`` the Legendre contractions run as
-persistent work-queue kernels on the int8 matrix cores, and with
-``graph=True`` each call's launch sequence is captured once in a hipGraph and
-replayed with a single launch (the stream must not be the default stream).
+(src/batch_transforms.jl:312-655).  Here one object runs them largest first;
+configurations that all stay on the split contraction share one launch per stage
+(persistent work-queue kernels).  With ``graph=True`` each call's launch sequence
+is captured once in a hipGraph and replayed with a single launch (the stream must
+not be the default stream).
 """
 from __future__ import annotations
 

@@ -158,7 +158,8 @@ _PRECISIONS = {"fp64": _lib.SHTK_PREC_FP64, "split": _lib.SHTK_PREC_SPLIT, "fp32
 def _precision(op, prec) -> int:
     """Contraction precision keyword of the batch transforms: "fp64" (the plain
     FP64 kernels), "split" (Ozaki split on int8 matrix cores, FP64-grade) or
-    "fp32" (FP32 matrix cores, FP32-grade; FP64 Legendre values)."""
+    "fp32" (FP32 matrix cores, FP32-grade; FP64 Legendre values).  The library takes
+    the FP64 kernels for the other two where they are faster (shtk.h)."""
     try:
         return _PRECISIONS[str(prec).lstrip(":").lower()]
     except KeyError:
@@ -236,14 +237,14 @@ def synthesis_cplx(cfg, alm):
 
 def synthesis_batch(*args, **kw):
     """``synthesis_batch(cfg, alm (lmax+1, mmax+1, nf); real_output=True, precision="fp64")``
-    -> (nlat, nlon, nf).  ``precision="split"`` runs the shared-recurrence Ozaki
-    contraction on the int8 matrix cores (FP64-grade results)."""
+    -> (nlat, nlon, nf).  ``precision="split"`` allows the shared-recurrence
+    Ozaki contraction on the int8 matrix cores (FP64-grade results)."""
     return _synthesis(args, dict(kw), True, "synthesis_batch")
 
 
 def analysis_batch(*args, **kw):
     """``analysis_batch(cfg, fields (nlat, nlon, nf); precision="fp64")`` -> (lmax+1, mmax+1, nf).
-    ``precision="split"`` contracts on the int8 matrix cores (FP64-grade results)."""
+    ``precision="split"`` allows the int8 matrix cores (FP64-grade results)."""
     return _analysis(args, dict(kw), True, "analysis_batch")
 
 
@@ -324,8 +325,8 @@ def analysis_sphtor(*args, **kw):
 
 def synthesis_sphtor_batch(*args, **kw):
     """``synthesis_sphtor_batch(cfg, Slm, Tlm (lmax+1, mmax+1, nf); real_output=True, precision="fp64")``
-    -> (Vt, Vp) each (nlat, nlon, nf).  ``precision="split"`` runs the contraction
-    on the int8 matrix cores (FP64-grade results)."""
+    -> (Vt, Vp) each (nlat, nlon, nf).  ``precision="split"`` allows FP64-grade
+    contractions (64-degree plans run the FP64 field groups)."""
     return _synthesis_sphtor(args, dict(kw), True, "synthesis_sphtor_batch")
 
 
