@@ -60,7 +60,6 @@ struct LegArgs {
     const double *gtab;   // g_l = sqrt((2l+1)(l^2-m^2)/(2l-1))
     const long long *coff;
     const int *segbase;   // [nm] first global segment index of each order
-    const int *segm;      // [nseg_total] order index im of each global segment
     int nseg_total;
     const double *seedq0; // [nseg_total][np] Q_{l0-1}
     const double *seedq1; // [nseg_total][np] Q_{l0}
@@ -80,6 +79,10 @@ struct LegArgs {
     const int4 *seglist;    // field-group analysis: [nlist] (global segment or -1, order, segment of the
                             // order, coff), entry i for XCD i mod 8
     int nlist;
+    const int4 *segitem;    // analysis work items: (global segment, order, segment of the order, 0), the
+                            // segments that hold degrees to the plan's lmax first, in order, then the
+                            // ones that hold the degree lmax + 1 alone
+    int nitem;              // items of this launch: those of scalar transforms, or nseg_total
     int raw_q;              // scalar analysis: sums against Q_l, without the factor c_l
     const double2 *edge;    // field-group synthesis of vector fields: [field][nseg_total][2] coefficients of the
                             // degrees before and after each segment (launch_vcoef), or nullptr
@@ -211,7 +214,7 @@ struct shtk_plan {
     long long *coff = nullptr;
     int *segbase = nullptr;
     double *seedq0 = nullptr, *seedq1 = nullptr;
-    int *seedk = nullptr, *pfirst = nullptr, *pfast = nullptr, *segm = nullptr;
+    int *seedk = nullptr, *pfirst = nullptr, *pfast = nullptr;
     double *convscale = nullptr;  // [(lmax+1)*(mmax+1)] configured -> canonical multiplier (non-canonical only)
     double2 *tw = nullptr;     // e^{-2 pi i t / nfft}, t < nfft
     double2 *chirp = nullptr;  // Bluestein chirp and kernel spectra (see FftArgs)
@@ -241,7 +244,9 @@ struct shtk_plan {
     double *oz_asc = nullptr;
     int4 *oz_run = nullptr;  // analysis work runs: (order, first segment, segments, 0)
     int oz_nrun = 0, oz_run_len = 8;
-    int4 *seglist = nullptr;  // segments dealt to the XCDs by order (LegArgs.seglist), inside segm's array
+    int4 *segitem = nullptr;  // analysis work items (LegArgs.segitem), nitem of them for scalar transforms
+    int nitem = 0;
+    int4 *seglist = nullptr;  // segments dealt to the XCDs by order (LegArgs.seglist), behind segitem in its array
     int nlist = 0;
     size_t qc_len = 0;
     int oz_ch_total = 0;
@@ -314,7 +319,7 @@ struct OzArgs {
     const int *epl;         // |P_l| < 2^epl over all pairs, per order
     const double *qb, *qcc; // beta_l and c_l of qc (padded by OZ_TPAD)
     const double *seedq0, *seedq1;
-    const int *seedk, *segbase, *segm, *pfirst;
+    const int *seedk, *segbase, *pfirst;
     int seg, nseg_total, nks;
     int nh, npb;            // analysis pair blocks: nh halves of 256 pairs each, npb blocks
     const double *wlat;

@@ -799,7 +799,10 @@ __global__ __launch_bounds__(256) void k_vpole_anal(const LegArgs a, double wpol
 }
 
 // ---------------------------------------------------------------------------
-// Analysis work items: (global segment, pair block of 512, field).
+// Analysis work items: (entry of segitem, pair block of 512, field).  The segments of scalar
+// transforms are counted without the ones that hold the degree lmax + 1 alone: with these
+// among them the four-wave blocks straddle the orders where lmax + 1 is a multiple of 64
+// (3 fields at lmax 511: 40.0 us without, 43.9 with; one at 1023: 77.4 and 80.2).
 // ---------------------------------------------------------------------------
 struct Item {
     int gs, pbi, im, s, m, l0, lend, lstop, pb0, pb1, pstart, f;
@@ -834,14 +837,17 @@ __device__ void zero_fill(const LegArgs &a, const Item &it, OT *col, bool all_de
 constexpr int ANW_WAVES = 4;
 constexpr int ANW_RS = 65;  // LDS row stride (doubles) of the reduction tile
 
+// VEC: a component of a vector analysis (raw_q, m0_one); scalar launches carry none of it.
+template <bool VEC>
 __device__ __forceinline__ Item make_item_at(const LegArgs &a, int item, int pblk) {
     Item it;
-    it.gs = item % a.gx;
+    const cptr<int> e = as_const((const int *)a.segitem) + 4 * (size_t)(item % a.gx);
+    it.gs = e[0];
     it.pbi = (item / a.gx) % a.gy;
-    it.im = as_const(a.segm)[it.gs];
-    it.s = it.gs - as_const(a.segbase)[it.im];
+    it.im = e[1];
+    it.s = e[2];
     it.m = it.im * a.mres;
-    it.one = a.m0_one && it.im == 0;
+    it.one = VEC && a.m0_one && it.im == 0;
     const int mt = it.one ? 1 : it.m;
     if (it.one) it.gs = min(as_const(a.segbase)[1] + it.s, a.nseg_total - 1);
     it.co = as_const(a.coff)[it.one ? 1 : it.im] - mt;
@@ -856,11 +862,11 @@ __device__ __forceinline__ Item make_item_at(const LegArgs &a, int item, int pbl
     return it;
 }
 
-template <int K, bool FAST, typename OT>
+template <int K, bool FAST, bool VEC, typename OT>
 __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, double *red, OT *col, int lane) {
     const int np = a.np, nlat = a.nlat;
     const double2 *Fi = a.F0 + ((size_t)it.f * a.nm + it.im) * nlat;
-    const double *wlat = it.one ? a.wlat0 : a.wlat;
+    const double *wlat = VEC && it.one ? a.wlat0 : a.wlat;
     double x[K], prev[K], cur[K], gpr[K], gpi[K], gmr[K], gmi[K];
     int kk[K];
 #pragma unroll
@@ -952,7 +958,7 @@ __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, dou
         sum += __shfl_xor(sum, 32);
         const int t = c0 + (o >> 1);
         if (qg == 0 && t < nst) {
-            const double v = gm * (a.raw_q ? 1.0 : qcm[it.l0 + t]) * sum;
+            const double v = gm * (VEC ? 1.0 : qcm[it.l0 + t]) * sum;
             OT *dst = col + 2 * (size_t)(it.l0 + t) + (o & 1);
             if (a.atomic)
                 atomicAdd(dst, (OT)v);
@@ -962,21 +968,21 @@ __device__ __forceinline__ void anal_w_run(const LegArgs &a, const Item &it, dou
     }
 }
 
-template <int K, typename OT>
+template <int K, bool VEC, typename OT>
 __device__ __forceinline__ void anal_w_dispatch(const LegArgs &a, const Item &it, double *red, OT *col, int lane) {
     if (it.fast)
-        anal_w_run<K, true>(a, it, red, col, lane);
+        anal_w_run<K, true, VEC>(a, it, red, col, lane);
     else
-        anal_w_run<K, false>(a, it, red, col, lane);
+        anal_w_run<K, false, VEC>(a, it, red, col, lane);
 }
 
-template <typename OT>
+template <typename OT, bool VEC>
 __global__ __launch_bounds__(64 * ANW_WAVES) void k_anal_w(const LegArgs a) {
     __shared__ double red_all[ANW_WAVES][16 * ANW_RS + SEG_MAX + 8];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int item = blockIdx.x * ANW_WAVES + w;
     if (item >= a.gx * a.gy * a.gz) return;
-    const Item it = make_item_at(a, item, 512);
+    const Item it = make_item_at<VEC>(a, item, 512);
     OT *col = (OT *)a.out0 + 2 * ((size_t)it.f * a.spec_fstride + (size_t)(a.lmax + 1) * it.m);
     const bool dead = it.lstop <= it.l0 || it.pstart >= it.pb1;
     zero_fill(a, it, col, dead, lane);
@@ -984,14 +990,14 @@ __global__ __launch_bounds__(64 * ANW_WAVES) void k_anal_w(const LegArgs a) {
     double *red = red_all[w];
     const int keff = (it.pb1 - it.pstart + 63) / 64;
     switch (keff) {
-        case 1: anal_w_dispatch<1>(a, it, red, col, lane); break;
-        case 2: anal_w_dispatch<2>(a, it, red, col, lane); break;
-        case 3: anal_w_dispatch<3>(a, it, red, col, lane); break;
-        case 4: anal_w_dispatch<4>(a, it, red, col, lane); break;
-        case 5: anal_w_dispatch<5>(a, it, red, col, lane); break;
-        case 6: anal_w_dispatch<6>(a, it, red, col, lane); break;
-        case 7: anal_w_dispatch<7>(a, it, red, col, lane); break;
-        default: anal_w_dispatch<8>(a, it, red, col, lane); break;
+        case 1: anal_w_dispatch<1, VEC>(a, it, red, col, lane); break;
+        case 2: anal_w_dispatch<2, VEC>(a, it, red, col, lane); break;
+        case 3: anal_w_dispatch<3, VEC>(a, it, red, col, lane); break;
+        case 4: anal_w_dispatch<4, VEC>(a, it, red, col, lane); break;
+        case 5: anal_w_dispatch<5, VEC>(a, it, red, col, lane); break;
+        case 6: anal_w_dispatch<6, VEC>(a, it, red, col, lane); break;
+        case 7: anal_w_dispatch<7, VEC>(a, it, red, col, lane); break;
+        default: anal_w_dispatch<8, VEC>(a, it, red, col, lane); break;
     }
 }
 
@@ -1202,7 +1208,7 @@ __global__ __launch_bounds__(64 * AVW_WAVES, KMAX <= 4 ? 3 : 1) void k_anal_vw(c
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int item = blockIdx.x * AVW_WAVES + w;
     if (item >= a.gx * a.gy * a.gz) return;
-    const Item it = make_item_at(a, item, a.apblk);
+    const Item it = make_item_at<false>(a, item, a.apblk);
     const size_t co = 2 * ((size_t)it.f * a.spec_fstride + (size_t)(a.lmax + 1) * it.m);
     OT *cs = (OT *)a.out0 + co;
     OT *ct = (OT *)a.out1 + co;
@@ -1343,7 +1349,7 @@ hipError_t launch_leg_anal(const LegArgs &a0, int nfields, int vector, hipStream
     LegArgs a = a0;
     if (!vector || a.apblk != 256) a.apblk = 512;  // pairs per work item
     const int pblk = a.apblk;
-    a.gx = a.nseg_total;
+    a.gx = a.nitem;
     a.gy = (a.np + pblk - 1) / pblk;
     a.gz = nfields;
     const dim3 grid((unsigned)a.gx * a.gy * nfields);
@@ -1363,9 +1369,11 @@ hipError_t launch_leg_anal(const LegArgs &a0, int nfields, int vector, hipStream
     } else {
         const dim3 gw((unsigned)(((long long)a.gx * a.gy * nfields + ANW_WAVES - 1) / ANW_WAVES));
         if (a.io_f32)
-            hipLaunchKernelGGL(k_anal_w<float>, gw, dim3(64 * ANW_WAVES), 0, st, a);
+            hipLaunchKernelGGL((k_anal_w<float, false>), gw, dim3(64 * ANW_WAVES), 0, st, a);
+        else if (a.raw_q)
+            hipLaunchKernelGGL((k_anal_w<double, true>), gw, dim3(64 * ANW_WAVES), 0, st, a);
         else
-            hipLaunchKernelGGL(k_anal_w<double>, gw, dim3(64 * ANW_WAVES), 0, st, a);
+            hipLaunchKernelGGL((k_anal_w<double, false>), gw, dim3(64 * ANW_WAVES), 0, st, a);
     }
     return hipGetLastError();
 }

@@ -271,7 +271,7 @@ void free_plan(shtk_plan *p) {
     if (!p) return;
     void *ptrs[] = {p->x,      p->s,      p->wscaled, p->winvs,  p->winvs2, p->invs,  p->qc,  p->ab, p->gtab,
                     p->qd,     p->coff,   p->segbase, p->seedq0, p->seedq1, p->seedk, p->pfirst,
-                    p->pfast,  p->segm,   p->convscale, p->tw, p->ws,     p->sectv, p->sectk, p->oz_q0,
+                    p->pfast,  p->segitem, p->convscale, p->tw, p->ws,     p->sectv, p->sectk, p->oz_q0,
                     p->oz_q1,  p->oz_qk,  p->oz_ep,     p->oz_chbase, p->oz_ws, p->oz_emaxl, p->oz_epl,
                     p->oz_asc, p->oz_chm, p->oz_run, p->qb, p->qcc, p->zseed};
     for (void *q : ptrs)
@@ -478,10 +478,11 @@ shtk::LegArgs base_args(const shtk_plan *p, int ltr) {
     a.gtab = p->gtab;
     a.coff = p->coff;
     a.segbase = p->segbase;
-    a.segm = p->segm;
     a.nseg_total = p->nseg_total;
     a.seglist = p->seglist;
     a.nlist = p->nlist;
+    a.segitem = p->segitem;
+    a.nitem = p->nitem;
     a.seedq0 = p->seedq0;
     a.seedq1 = p->seedq1;
     a.seedk = p->seedk;
@@ -751,7 +752,6 @@ shtk::OzArgs oz_anal_args(const shtk_plan *p, double2 *F0, double *acc, int nf, 
     o.seedq1 = p->seedq1;
     o.seedk = p->seedk;
     o.segbase = p->segbase;
-    o.segm = p->segm;
     o.pfirst = p->pfirst;
     o.seg = p->seg;
     o.nseg_total = p->nseg_total;
@@ -817,7 +817,6 @@ shtk::OzArgs f32_anal_args(const shtk_plan *p, double2 *F0, double *acc, int nf,
     o.seedq1 = p->seedq1;
     o.seedk = p->seedk;
     o.segbase = p->segbase;
-    o.segm = p->segm;
     o.pfirst = p->pfirst;
     o.seg = p->seg;
     o.nseg_total = p->nseg_total;
@@ -898,6 +897,7 @@ int ensure_zseed(shtk_plan *p, hipStream_t st) {
 shtk::LegArgs vscalar_args(const shtk_plan *p, int ltr) {
     shtk::LegArgs a = base_args(p, ltr + 1);
     a.lmax = p->d.lmax + 1;
+    a.nitem = p->nseg_total;
     a.spec_fstride = (long long)(p->d.lmax + 2) * (p->d.mmax + 1);
     return a;
 }
@@ -1914,24 +1914,27 @@ static int plan_tables(shtk_plan *p) {
         }
     }
     p->nseg_total = nseg_total;
-    // segments for the field-group analysis, order im on XCD im mod 8: behind segm in
-    // one array (LegArgs.seglist)
-    const size_t segm_len = (segm.size() + 3) / 4 * 4;
+    // analysis work items (LegArgs.segitem), then the segments for the field-group analysis,
+    // order im on XCD im mod 8 (LegArgs.seglist), in one array
+    std::vector<int4> items;
+    for (int extra = 0; extra < 2; ++extra) {
+        for (int gs = 0; gs < nseg_total; ++gs) {
+            const int im = segm[gs], s = gs - segbase[im];
+            if ((im * d.mres + s * S > lmax) == (extra == 1)) items.push_back(make_int4(gs, im, s, 0));
+        }
+        if (extra == 0) p->nitem = (int)items.size();
+    }
     {
         std::vector<int> per[shtk::kXcds];
         for (int gs = 0; gs < nseg_total; ++gs) per[segm[gs] % shtk::kXcds].push_back(gs);
         size_t most = 0;
         for (auto &v : per) most = std::max(most, v.size());
         p->nlist = (int)(most * shtk::kXcds);
-        segm.resize(segm_len + 4 * (size_t)p->nlist, -1);
+        items.resize(nseg_total + (size_t)p->nlist, make_int4(-1, -1, -1, -1));
         for (int x = 0; x < shtk::kXcds; ++x)
             for (size_t k = 0; k < per[x].size(); ++k) {
                 const int gs = per[x][k], im = segm[gs];
-                int *e = &segm[segm_len + 4 * (k * shtk::kXcds + x)];
-                e[0] = gs;
-                e[1] = im;
-                e[2] = gs - segbase[im];
-                e[3] = (int)coff[im];
+                items[nseg_total + k * shtk::kXcds + x] = make_int4(gs, im, gs - segbase[im], (int)coff[im]);
             }
     }
 
@@ -2029,8 +2032,8 @@ static int plan_tables(shtk_plan *p) {
     RC_TRY(upload(&p->coff, coff, "plan tables"));
     p->hcoff = coff;
     RC_TRY(upload(&p->segbase, segbase, "plan tables"));
-    RC_TRY(upload(&p->segm, segm, "plan tables"));
-    p->seglist = (int4 *)(p->segm + segm_len);
+    RC_TRY(upload(&p->segitem, items, "plan tables"));
+    p->seglist = p->segitem + nseg_total;
     RC_TRY(upload(&p->convscale, conv, "plan tables"));
     RC_TRY(upload(&p->tw, tw, "plan tables"));
     if (p->fft.blue) {  // one array
