@@ -615,12 +615,16 @@ __global__ __launch_bounds__(256) void k_vout(const double2 *H, OT *S, OT *T, co
 
 // A group costs the same for 1 to 8 fields.  Against the single-field kernel, lmax
 // 1023: 4 fields 228 (one group) against 256 us, 3 fields 228 against 192; so fewer
-// than 4 fields go to the single-field kernel, beside other groups fewer than 3 (whole
-// calls of 11 and 12 fields at 1023: 533 and 532 us, at 511: 141 and 125).
+// than 4 fields go to the single-field kernel.  Beside other groups that is a launch of
+// its own, which one field is worth from lmax 400 and two from 600 (whole calls, single
+// kernel against a group more: 9 fields at 127 22.7 and 15.2 us, at 255 36.6 and 31.0, at
+// 511 92.5 and 99.0; 10 at 511 103.8 and 96.4, at 700 310 and 317, at 1023 464 and 510; 11
+// at 1023 541 and 528).
 int fields_anal_count(const LegArgs &a, int nfields) {
     if (a.seg != DSEG) return 0;
     const int rest = nfields % MX_FIELDS;
-    return rest < (nfields > MX_FIELDS ? 3 : 4) ? nfields - rest : nfields;
+    const bool single = nfields < MX_FIELDS ? rest < 4 : rest < 3 && a.lmax >= 200 * (rest + 1);
+    return single ? nfields - rest : nfields;
 }
 
 hipError_t launch_fields_anal(const LegArgs &a0, int nfields, hipStream_t st) {
@@ -652,8 +656,15 @@ hipError_t launch_fields_synth(const LegArgs &a0, int nfields, hipStream_t st) {
     LegArgs a = a0;
     a.nf = nfields;
     a.gx = (a.np + 63) / 64;
-    // equal groups of at most 8 fields
-    a.gz = (nfields + 7) / 8;
+    // equal groups of at most 8 fields, 4 or 2 where these would leave fewer than 1024 units
+    // (a short launch takes as long as one unit, whose time goes with the fields: whole calls
+    // in groups of 8, 4 and 2, 8 fields at lmax 127 14.6, 13.3 and 13.3 us, at 255 24.2, 21.3
+    // and 21.1; 16 at 191 25.4, 22.3 and 23.8; 32 at 127 19.3, 16.1 and 18.5; from 1024 units
+    // of 8 on 8 at 511 60.5, 60.5 and 67.2, 32 at 340 193, 194 and 205)
+    const int nm = a.nm_run > 0 ? std::min(a.nm_run, a.nm) : a.nm;
+    int most = 8;
+    while (most > 2 && (long long)nm * a.gx * ((nfields + most - 1) / most) < 1024) most /= 2;
+    a.gz = (nfields + most - 1) / most;
     const int ng = (nfields + a.gz - 1) / a.gz;
     if (a.edge) launch_synth_groups<true>(a, ng, st);
     else launch_synth_groups<false>(a, ng, st);
