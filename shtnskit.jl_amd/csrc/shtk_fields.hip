@@ -271,10 +271,10 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
 // the chip runs at 2.0 GHz).  16 fields at lmax 1023: 815 us (k_synth_d) -> 435; 3
 // fields: 192 -> 105; 16 at 511: 124 -> 63; 37 at 255: 40 -> 29; 5 at 340: 30 -> 19.
 // ---------------------------------------------------------------------------
-template <int NG>
+template <int NG, typename CT = double2>
 struct SFRec {
     double b, c;      // beta_{l+1}, c_l
-    double2 v[NG];    // a_l of the fields
+    CT v[NG];         // a_l of the fields
 };
 
 // Degrees N .. 15 of a record group.
@@ -307,7 +307,8 @@ __device__ __forceinline__ void sf_edge(const double2 *eg, double (*acc)[NG][2],
     }
 }
 
-template <int NG, int NW, bool VEC>
+// CT: the type of the coefficients (float2: scalar transforms of FP32 arrays).
+template <int NG, int NW, bool VEC, typename CT>
 __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const LegArgs a) {
     __shared__ double red[NW > 1 ? NW - 1 : 1][NW > 1 ? 4 * NG : 1][64];
     // units lowest order first for every pair block and group: the long columns start first
@@ -343,18 +344,18 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
         int kk = a.seedk[q];
         const double *qb = a.qb + co + 1, *qc = a.qcc + co;  // padded past lmax
         const cptr<double> qcm = as_const(a.qcc) + co;
-        const double2 *av = (const double2 *)a.in0 + (size_t)f0 * a.spec_fstride + (size_t)(lmax + 1) * m;
+        const CT *av = (const CT *)a.in0 + (size_t)f0 * a.spec_fstride + (size_t)(lmax + 1) * m;
         const int l1 = min(mt + sb * DSEG, ltr + 1);  // VEC: ltr is the degree after the last S, T
-        SFRec<NG> n;
+        SFRec<NG, CT> n;
         auto load = [&](int l0) {
             // uniform bases and one 32-bit lane offset (64-bit addresses per field would
             // take the registers of a wave)
-            const unsigned l = l0 + (lane & 15), lc = 16u * min(l, (unsigned)lmax);
+            const unsigned l = l0 + (lane & 15), lc = (unsigned)sizeof(CT) * min(l, (unsigned)lmax);
             n.b = qb[l];
             n.c = qc[l];
 #pragma unroll
             for (int f = 0; f < NG; ++f)
-                n.v[f] = *(const double2 *)((const char *)(av + (size_t)min(f, nfl - 1) * a.spec_fstride) + lc);
+                n.v[f] = *(const CT *)((const char *)(av + (size_t)min(f, nfl - 1) * a.spec_fstride) + lc);
         };
         int l = mt + sa * DSEG;
         load(l);
@@ -384,14 +385,14 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
                 const bool in = l + (lane & 15) < l1;
 #pragma unroll
                 for (int f = 0; f < NG; ++f) {
-                    n.v[f].x = in ? n.v[f].x : 0.0;
-                    n.v[f].y = in ? n.v[f].y : 0.0;
+                    n.v[f].x = in ? n.v[f].x : 0;
+                    n.v[f].y = in ? n.v[f].y : 0;
                 }
             }
             r.b = n.b;
             const double sc = a.qscale_in ? n.c : 1.0;
 #pragma unroll
-            for (int f = 0; f < NG; ++f) r.v[f] = make_double2(n.v[f].x * sc, n.v[f].y * sc);
+            for (int f = 0; f < NG; ++f) r.v[f] = make_double2((double)n.v[f].x * sc, (double)n.v[f].y * sc);
             load(l + 16);
             asm volatile("s_nop 4");
         };
@@ -478,15 +479,15 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
     }
 }
 
-template <int NG, bool VEC>
+template <int NG, bool VEC, typename CT>
 void launch_synth_sf(const LegArgs &a, hipStream_t st) {
     const long long units = (long long)(a.nm_run > 0 ? std::min(a.nm_run, a.nm) : a.nm) * a.gx * a.gz;
     // 2 waves per unit where one would leave the chip short of waves (4096 units, 16
     // fields at lmax 511: 65 -> 62 us; 16384, 16 at 1023: 429 against 432; 4 waves lose
     // the accumulator traffic through LDS: 98 us at 511)
     const dim3 grid((unsigned)units);
-    if (units >= 8192 || a.lmax < DSEG) hipLaunchKernelGGL((k_synth_sf<NG, 1, VEC>), grid, dim3(64), 0, st, a);
-    else hipLaunchKernelGGL((k_synth_sf<NG, 2, VEC>), grid, dim3(128), 0, st, a);
+    if (units >= 8192 || a.lmax < DSEG) hipLaunchKernelGGL((k_synth_sf<NG, 1, VEC, CT>), grid, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((k_synth_sf<NG, 2, VEC, CT>), grid, dim3(128), 0, st, a);
 }
 
 // ---------------------------------------------------------------------------
@@ -639,16 +640,16 @@ hipError_t launch_fields_anal(const LegArgs &a0, int nfields, hipStream_t st) {
 
 bool fields_synth_ok(const LegArgs &a, int nfields) { return nfields >= 2 && a.seg == DSEG; }
 
-template <bool VEC>
+template <bool VEC, typename CT>
 static void launch_synth_groups(const LegArgs &a, int ng, hipStream_t st) {
     switch (ng) {
-        case 2: launch_synth_sf<2, VEC>(a, st); break;
-        case 3: launch_synth_sf<3, VEC>(a, st); break;
-        case 4: launch_synth_sf<4, VEC>(a, st); break;
-        case 5: launch_synth_sf<5, VEC>(a, st); break;
-        case 6: launch_synth_sf<6, VEC>(a, st); break;
-        case 7: launch_synth_sf<7, VEC>(a, st); break;
-        default: launch_synth_sf<8, VEC>(a, st); break;
+        case 2: launch_synth_sf<2, VEC, CT>(a, st); break;
+        case 3: launch_synth_sf<3, VEC, CT>(a, st); break;
+        case 4: launch_synth_sf<4, VEC, CT>(a, st); break;
+        case 5: launch_synth_sf<5, VEC, CT>(a, st); break;
+        case 6: launch_synth_sf<6, VEC, CT>(a, st); break;
+        case 7: launch_synth_sf<7, VEC, CT>(a, st); break;
+        default: launch_synth_sf<8, VEC, CT>(a, st); break;
     }
 }
 
@@ -666,8 +667,9 @@ hipError_t launch_fields_synth(const LegArgs &a0, int nfields, hipStream_t st) {
     while (most > 2 && (long long)nm * a.gx * ((nfields + most - 1) / most) < 1024) most /= 2;
     a.gz = (nfields + most - 1) / most;
     const int ng = (nfields + a.gz - 1) / a.gz;
-    if (a.edge) launch_synth_groups<true>(a, ng, st);
-    else launch_synth_groups<false>(a, ng, st);
+    if (a.edge) launch_synth_groups<true, double2>(a, ng, st);
+    else if (a.io_f32) launch_synth_groups<false, float2>(a, ng, st);
+    else launch_synth_groups<false, double2>(a, ng, st);
     return hipGetLastError();
 }
 

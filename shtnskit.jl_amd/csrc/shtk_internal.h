@@ -92,8 +92,8 @@ struct LegArgs {
     int skip_m0;            // order 0 is left out (the zonal kernel of shtk_ml.hip computes it)
     int m0_one;             // vector pair as scalar fields: order 0 runs on the tables of order 1 (launch_vcoef)
     const double *wlat0;    // m0_one: wlat of order 0 (or nullptr)
-    int qscale_in;          // scalar synthesis (64-degree segments): in0 holds canonical FP64
-                            // coefficients, multiplied by c_l as they are loaded
+    int qscale_in;          // scalar synthesis (64-degree segments): in0 holds canonical coefficients,
+                            // multiplied by c_l as they are loaded (io_f32: field groups alone)
     int s1w_units;          // scalar synthesis (64-degree segments): one wave per block when the
                             // launch has at least this many (order, pair block, field) units
     int apblk;              // analysis: latitude pairs per work item (512, or 256 for the vector

@@ -542,28 +542,30 @@ int check_precision(const shtk_plan *p, int precision, int lmax_limit) {
     return SHTK_OK;
 }
 
-// The contraction that a call of a given precision runs: the matrix-core ones where they are
-// the faster, otherwise the FP64 field groups, whose results are within any precision's.  A
-// matrix-core contraction pads the fields to 16s and the analysis the pairs to 256s (and
-// accumulates over blocks of 512), a field group takes 1 to 8; small sizes go to its prologues.
-// Whole calls in us, FP64 against split, against FP32, nlon 2048 (lmax, fields):
-//   synthesis  511, 16: 144, 173, 149     700, 16: 304, 313, 265    800, 16: 413, 399, 357
-//              900, 12: 418, 429, 394     1023, 12: 508, 510, 467   1023, 16: 638, 592, 538
-//              1023, 10: 426, 478, 441    1023, 28: 1046, 1078, 965
-//   analysis   511, 12: 141, 151, 138     700, 12: 280, 343, 308    1023, 12: 570, 583, 529
-//              511, 16: 164, 180, 173     1023, 24: 887, 1164, 1041 1023, 32: 1138, 1305, 1190
-//              1023, 16, 1536 latitudes: 878, 1661, 1567
+// The contraction that a call of a given precision runs: a matrix-core synthesis where it is
+// the faster, otherwise the FP64 field groups, whose results are within any precision's.
+// Per degree and latitude pair a group of n fields costs n + 1 FP64 steps, a matrix-core
+// contraction the same for 1 to 16 fields, and the split one a prologue per order that only
+// many degrees and pairs pay for.  Whole calls in us, FP64 and then the other contraction:
+//   synthesis, FP32 arrays in FP32 precision, nlat = lmax + 1 (lmax, fields):
+//     127, 16: 12.7, 16.6     511, 16: 93, 107     700, 16: 228, 230     800, 32: 653, 651
+//     1023, 13: 452, 452      1023, 16: 519, 487   1023, 24: 775, 870    1023, 32: 1020, 960
+//   split synthesis of FP64 arrays, 16 fields (lmax, nlat):
+//     511, 512: 97, 129       1023, 1024: 567, 593    1023, 1536: 803, 810
+//     1200, 1700: 1347, 1348  1023, 2048: 1109, 1059  1535, 1536: 1667, 1602   2047, 2048: 3688, 3172
+//     1023, 2048 with 14 and 15 fields: 959, 967 and 1056, 1001
+//   analysis, FP32 arrays in FP32 precision:
+//     511, 12: 101, 125       1023, 12: 538, 593   1023, 16: 606, 698    2047, 16: 3529, 4883
+// The lines hold all orders; with a quarter of them (mmax) at lmax 1023 the FP32 synthesis is
+// already the faster at 12 fields (223, 211).
 // FP64 arrays in FP32 precision keep the FP32 kernels: a caller that compares runs in that
 // precision gets the values it always got, which the FP64 groups match to 2e-7 only.
 int contraction_prec(const shtk_plan *p, int prec, int nf, int dtype, bool synth) {
     if (prec == SHTK_PREC_FP64 || p->seg != shtk::DSEG) return prec;
     if (prec == SHTK_PREC_FP32 && dtype == SHTK_F64) return prec;
-    const int lmax = p->d.lmax, pad = (nf + 15) / 16 * 16;
-    if (synth && prec == SHTK_PREC_SPLIT) return lmax >= 800 && 4 * pad <= 5 * nf ? prec : SHTK_PREC_FP64;
-    if (synth) return lmax >= 600 && 2 * pad <= 3 * nf ? prec : SHTK_PREC_FP64;
-    const int np = p->np, npad = (np + 255) / 256 * 256;
-    if (prec == SHTK_PREC_FP32 && lmax >= 500 && pad - nf <= 5 && np <= 512 && 10 * npad <= 11 * np) return prec;
-    return SHTK_PREC_FP64;
+    const int steps = nf + (nf + 7) / 8, blocks = (nf + 15) / 16;
+    const bool large = prec == SHTK_PREC_SPLIT ? (long long)p->d.lmax * p->np >= 1000000 : p->d.lmax >= 900;
+    return synth && large && steps >= 17 * blocks ? prec : SHTK_PREC_FP64;
 }
 
 // The same for the vector pair, whose field groups are always the faster.
@@ -1012,9 +1014,11 @@ int run_to_grid(shtk_plan *p, const Job &j, const void *s0, const void *s1, void
     a.in0 = s0;
     a.in1 = s1;
     a.io_f32 = dtype == SHTK_F32;
-    if (!j.vector && j.prec == SHTK_PREC_FP64 && p->canonical && !a.io_f32 && p->seg == shtk::DSEG) {
-        // scalar FP64 synthesis of canonical FP64 coefficients: the kernel applies
-        // c_l (Q form) as it loads them
+    if (!j.vector && j.prec == SHTK_PREC_FP64 && p->canonical && p->seg == shtk::DSEG &&
+        (!a.io_f32 || shtk::fields_synth_ok(a, nf))) {
+        // scalar FP64 synthesis of canonical coefficients: the kernel applies c_l (Q form) as it
+        // loads them; FP32 ones in the field groups alone (a pass of their own before these cost
+        // 3 of 16 us of a call at lmax 63)
         a.qscale_in = 1;
     } else if (!j.vector && j.prec == SHTK_PREC_FP64) {
         // scalar FP64 synthesis: coefficients times c_l (Q form), converted to the
