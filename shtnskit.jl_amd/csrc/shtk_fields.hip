@@ -187,7 +187,7 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
         for (int h = 0; h < 2; ++h) {
             const double bl = h ? b2 : b0, bh = h ? b3 : b1;
             if (h == 1 && l0 + MX_DEG >= lstop) break;
-            asm volatile("s_nop 4");
+            dpp_wait(bl, bh);
             if (slow) {
                 const double cm = kk == 0 ? 1.0 : 0.0;
                 mx_steps<false, 0>(bl, bh, x, cm, prev, cur, tile + lane);
@@ -370,7 +370,12 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
 #pragma unroll
                 for (int f = 0; f < NG; ++f)
                     eg[f] = *(const double2 *)((const char *)(ev + 2 * (size_t)min(f, nfl - 1) * a.nseg_total) + o);
-                asm volatile("s_nop 4");
+#pragma unroll
+                for (int f = 0; f < NG; ++f) {
+                    dpp_written(eg[f].x);
+                    dpp_written(eg[f].y);
+                }
+                dpp_wait();
             }
         };
         if constexpr (VEC)
@@ -394,7 +399,12 @@ __global__ __launch_bounds__(64 * NW, NG <= 4 ? 4 : 3) void k_synth_sf(const Leg
 #pragma unroll
             for (int f = 0; f < NG; ++f) r.v[f] = make_double2((double)n.v[f].x * sc, (double)n.v[f].y * sc);
             load(l + 16);
-            asm volatile("s_nop 4");
+#pragma unroll
+            for (int f = 0; f < NG; ++f) {
+                dpp_written(r.v[f].x);
+                dpp_written(r.v[f].y);
+            }
+            dpp_wait(r.b);
         };
         // groups with scaled lanes first (a lane never becomes scaled again), then the rest in
         // a loop of its own, whose registers hold one body

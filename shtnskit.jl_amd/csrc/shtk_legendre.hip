@@ -1028,7 +1028,7 @@ __device__ __forceinline__ void avw_step(const AVRec &r, const double *x, double
         xc[j] = x[j] * cur[j];
         D[j] = 0.0;
     }
-    if (NOP) asm volatile("s_nop 4");
+    if (NOP) dpp_wait(r.b, r.dl, r.dg);
 #pragma unroll
     for (int j = 0; j < K; ++j) SHTK_FMAC_BC(D[j], r.dl, xc[j], N, "");
 #pragma unroll

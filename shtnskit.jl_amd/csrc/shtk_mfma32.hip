@@ -358,7 +358,7 @@ __device__ __forceinline__ void anal_f32_body(const OzArgs &a, const double *__r
             // inside the padded tables, a chunk that does not exist never uses them)
             const OzRec rec = nrec;
             load_rec(nrec, min(t0 + 32 < nst ? lc + 32 : m + (s0 + sr + 1) * a.seg, a.lmax));
-            asm volatile("s_nop 4");  // wait states before DPP reads the refilled records
+            dpp_wait(rec.a[0], rec.a[1], rec.b[0], rec.b[1]);
             f32_digit_steps<0, RSF>(rec, x, prev, cur, kk, lv46, Alds, wpos);
             __syncthreads();
             // rows: the 16 degrees of parity wp; K: the 256 pairs of half kh

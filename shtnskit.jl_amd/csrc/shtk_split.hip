@@ -758,7 +758,7 @@ __device__ __forceinline__ void anal_oz_body(const OzArgs &a, const double *__re
             // (clamped to lmax: reads stay inside the order's padded tables; a chunk
             // that does not exist never uses them)
             load_rec(nrec, min(t0 + 32 < nst ? lc + 32 : m + (s0 + sr + 1) * a.seg, a.lmax));
-            asm volatile("s_nop 4");  // wait states before DPP reads the refilled records
+            dpp_wait(rec.a[0], rec.a[1], rec.b[0], rec.b[1]);
             unsigned uh_even = 0, w1 = 0, w1h = 0, b2 = 0, b2h = 0;
             oz_digit_steps<0, NH>(rec, x, prev, cur, kk, live, aul, auh, sel1, sel2, uh_even, w1, w1h, b2, b2h);
             __syncthreads();
