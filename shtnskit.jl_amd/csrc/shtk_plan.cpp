@@ -772,10 +772,12 @@ shtk::OzArgs oz_anal_args(const shtk_plan *p, double2 *F0, double *acc, int nf, 
     return o;
 }
 
-// Bytes of split workspace for nf fields in both directions (analysis adds an
-// FP64 canonical accumulator when the output is not canonical FP64).
+// Bytes of split workspace for nf fields in the directions that run the split contraction
+// (contraction_prec): syntheses alone on 64-degree plans, both on the others, whose analysis
+// adds an FP64 canonical accumulator when the output is not canonical FP64.
 size_t oz_ws_bytes(const shtk_plan *p, int nf, bool with_acc) {
     const int nfg = (nf + shtk::OZ_FIELDS - 1) / shtk::OZ_FIELDS;
+    if (p->seg == shtk::DSEG) return oz_ws_layout(p, nfg, false).total;
     const size_t acc = with_acc ? (size_t)nf * (p->d.lmax + 1) * (p->d.mmax + 1) * 16 : 0;
     return std::max(oz_ws_layout(p, nfg, false).total, oz_ws_layout(p, nfg, true).total + acc);
 }
@@ -1608,17 +1610,14 @@ int batch_prepare(shtk_batch *b, int dtype, hipStream_t st) {
         shtk_plan *p = b->plans[gi];
         std::lock_guard<std::recursive_mutex> lk(p->mu);
         RC_TRY(ensure_ws(p, ws_layout(p, b->nf[gi], 0).total));
-        const int prec = b->precision;
-        if (contraction_prec(p, prec, b->nf[gi], dtype, true) == SHTK_PREC_FP64 &&
-            contraction_prec(p, prec, b->nf[gi], dtype, false) == SHTK_PREC_FP64)
-            continue;
-        if (prec == SHTK_PREC_SPLIT) {
-            RC_TRY(ensure_oz_tables(p, st));
-            RC_TRY(ensure_oz_ws(p, oz_ws_bytes(p, b->nf[gi], !p->canonical || dtype != SHTK_F64)));
-        } else if (prec == SHTK_PREC_FP32) {
-            RC_TRY(ensure_oz_tables(p, st));
-            RC_TRY(ensure_oz_ws(p, f32_ws_bytes(p, b->nf[gi], !p->canonical || dtype != SHTK_F64)));
-        }
+        const int ps = contraction_prec(p, b->precision, b->nf[gi], dtype, true);
+        const int pa = contraction_prec(p, b->precision, b->nf[gi], dtype, false);
+        if (ps == SHTK_PREC_FP64 && pa == SHTK_PREC_FP64) continue;
+        RC_TRY(ensure_oz_tables(p, st));
+        const bool with_acc = !p->canonical || dtype != SHTK_F64;
+        if (ps == SHTK_PREC_SPLIT || pa == SHTK_PREC_SPLIT)
+            RC_TRY(ensure_oz_ws(p, oz_ws_bytes(p, b->nf[gi], with_acc)));
+        if (pa == SHTK_PREC_FP32) RC_TRY(ensure_oz_ws(p, f32_ws_bytes(p, b->nf[gi], with_acc)));
     }
     return SHTK_OK;
 }
