@@ -268,7 +268,8 @@ int shtk_batch_synthesis(shtk_batch *batch, const void *const *alm, void *const 
 int shtk_batch_analysis(shtk_batch *batch, const void *const *f, void *const *alm, int dtype, void *stream);
 /* Autotuner: times round trips (synthesis into f, analysis back into alm, which
  * therefore ends up holding its own projection) for every candidate launch
- * shape and keeps the fastest; reports it if the pointers are not NULL. */
+ * shape and keeps the fastest; reports it if the pointers are not NULL.  Candidates are the
+ * grids of the persistent kernels that run; a direction without one reports 0. */
 int shtk_batch_autotune(shtk_batch *batch, void *const *alm, void *const *f, int dtype, int reps, void *stream,
                         int *best_synth_blocks, int *best_anal_blocks, double *best_ms);
 

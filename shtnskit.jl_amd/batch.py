@@ -112,7 +112,8 @@ class UnevenBatch:
 
     def autotune(self, alms: Sequence[torch.Tensor], fields: Sequence[torch.Tensor], reps: int = 3) -> dict:
         """Times every candidate launch shape on these arrays (round trips that
-        overwrite them) and keeps the fastest; returns the choice."""
+        overwrite them) and keeps the fastest; returns the choice (0 blocks for a
+        direction that does not run its persistent kernel)."""
         alms = self._arrays(alms, "spec", "autotune")
         fields = self._arrays(fields, "grid", "autotune")
         if (alms[0].dtype == torch.complex64) != (fields[0].dtype == torch.float32):

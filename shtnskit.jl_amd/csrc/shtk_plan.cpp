@@ -1584,12 +1584,16 @@ int batch_split(shtk_batch *b, int dir, const void *const *in, void *const *out,
     return SHTK_OK;
 }
 
+// Whether a direction of a batch runs the grouped split kernels: every group stays split.
+bool batch_is_split(const shtk_batch *b, int dir, int dtype) {
+    for (int gi = 0; gi < b->ngroups; ++gi)
+        if (contraction_prec(b->plans[gi], b->precision, b->nf[gi], dtype, dir == 0) != SHTK_PREC_SPLIT) return false;
+    return true;
+}
+
 // One direction of a batch, eagerly (no graph).
 int batch_issue(shtk_batch *b, int dir, const void *const *in, void *const *out, int dtype, hipStream_t st) {
-    bool split = b->precision == SHTK_PREC_SPLIT;
-    for (int gi = 0; gi < b->ngroups; ++gi)
-        split &= contraction_prec(b->plans[gi], b->precision, b->nf[gi], dtype, dir == 0) == SHTK_PREC_SPLIT;
-    if (split) return batch_split(b, dir, in, out, dtype, st);
+    if (batch_is_split(b, dir, dtype)) return batch_split(b, dir, in, out, dtype, st);
     // otherwise one configuration at a time, largest first (a captured graph replays the
     // whole sequence with one launch): 10 to 16 fields at five lmax from 1023 to 63 as split
     // groups 715 + 793 us, one by one 566 + 673
@@ -1782,16 +1786,20 @@ int shtk_batch_autotune(shtk_batch *b, void *const *alm, void *const *f, int dty
     hipStream_t st = (hipStream_t)stream;
     const int graph_was = b->use_graph;
     RC_TRY(shtk_batch_set_graph(b, 0));
-    // candidate grids of the two persistent kernels: 1..4 blocks per CU each
-    std::vector<int> blocks = {0};
-    if (b->precision == SHTK_PREC_SPLIT) blocks = {b->cus, 2 * b->cus, 3 * b->cus, 4 * b->cus};
+    // candidate grids of the two persistent kernels, 1 to 4 blocks per CU; a direction that does
+    // not run its kernel has no grid to choose (0)
+    std::vector<int> blocks[2];
+    for (int dir = 0; dir < 2; ++dir) {
+        if (batch_is_split(b, dir, dtype)) blocks[dir] = {b->cus, 2 * b->cus, 3 * b->cus, 4 * b->cus};
+        else blocks[dir] = {0};
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIP_TRY(hipEventCreate(&e0), "autotune events");
     HIP_TRY(hipEventCreate(&e1), "autotune events");
     double best = 1e300;
     int bb = 0, bp = 0;
-    for (int nb : blocks)
-        for (int fp : blocks) {
+    for (int nb : blocks[0])
+        for (int fp : blocks[1]) {
             RC_TRY(shtk_batch_set_tiles(b, nb, fp));
             // one untimed round trip, then reps timed ones
             RC_TRY(shtk_batch_synthesis(b, (const void *const *)alm, f, dtype, st));
