@@ -105,7 +105,9 @@ def _cplx(rdt: torch.dtype) -> torch.dtype:
 
 
 def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))  # no Stream object per call
+    # the raw handle makes no Stream object per call; torch documents the object alone
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return ctypes.c_void_p(raw(device.index) if raw else torch.cuda.current_stream(device).cuda_stream)
 
 
 def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
