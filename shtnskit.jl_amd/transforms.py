@@ -71,6 +71,8 @@ def _adapt(x, adapt: bool, op: str):
 
 def _colmajor(t: torch.Tensor) -> torch.Tensor:
     """Same logical tensor with Julia column-major memory (first index fastest)."""
+    if t.is_conj() or t.is_neg():  # lazy views: the memory holds other values than the tensor
+        t = t.resolve_conj().resolve_neg()
     want = 1
     for n, s in zip(t.shape, t.stride()):
         if n != 1 and s != want:
