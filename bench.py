@@ -11,7 +11,7 @@ Second measured line (`split_batched`): the same grid, a batch of 16 fields
 (seed 2, same spectrum), synthesis_batch then analysis_batch in split precision
 (the int8 matrix cores, or the FP64 field groups where these are the faster);
 its value is field round trips per second of the whole batch, with the per-field relative L2 error
-against the FP64 path.
+against the FP64 path where another contraction ran (`contraction` names it).
 
 Inputs are resident in HBM before every timed region.  `value` comes from K
 steps with no instrumentation; per-kernel durations come from a second pass of
@@ -39,6 +39,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-spli
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import statistics
@@ -221,10 +222,16 @@ def plain_roofline(kernels_us):
     return roofline_entry(dom, us, by * 1e3, PEAK_HBM_GBS, "GB/s", "hbm", f"{by:.4e} bytes")
 
 
-def measure_uneven(torch, np, shtk, dev, steps):
+def contraction_of(names):
+    """The Legendre contractions among the names of kernel events."""
+    kinds = {"oz": "int8 split", "f32": "FP32 matrix cores", "leg": "FP64"}
+    return sorted({kinds[n.split("_")[0]] for n in names if n.split("_")[0] in kinds})
+
+
+def measure_uneven(torch, np, shtk, _lib, dev, steps):
     """64 fields with lmax drawn uniformly from {63, 127, 255, 511, 1023} (seed 3),
-    nlat = lmax + 1, nlon = 2 nlat, (l+1)^-1 spectra: one split-precision batch
-    object, launch sequence captured in a hipGraph, launch shapes autotuned.
+    nlat = lmax + 1, nlon = 2 nlat, (l+1)^-1 spectra: one batch object that allows split
+    precision, launch sequence captured in a hipGraph, launch shapes autotuned.
     Value: field round trips per second of the whole batch."""
     rng = np.random.Generator(np.random.PCG64(3))
     draws = rng.choice([63, 127, 255, 511, 1023], size=64)
@@ -246,6 +253,17 @@ def measure_uneven(torch, np, shtk, dev, steps):
     cfgs2 = [shtk.create_gauss_config(L, L + 1, nlon=2 * L + 2) for L, _ in groups]
     b = shtk.UnevenBatch(cfgs2, nfs, precision="split")
     tune = b.autotune([a.clone() for a in alms], [f.clone() for f in ref_f], reps=2)
+    # the contractions that run: a direction with persistent kernels is split, the others by
+    # the events of each group's plan
+    plans = []
+    for i in range(len(groups)):
+        p = ctypes.c_void_p()
+        _lib.check(_lib.load().shtk_batch_plan(ctypes.c_void_p(b._b), i, ctypes.byref(p)), "batch_plan")
+        _lib.profile_enable(p.value, True)
+        plans.append(p.value)
+    b.analysis(b.synthesis(alms))
+    names = {n for p in plans for n in _lib.profile_read(p)}
+    ran = contraction_of(names | ({"oz"} if tune["synth_blocks"] or tune["anal_blocks"] else set()))
     b.close()
     cfgs3 = [shtk.create_gauss_config(L, L + 1, nlon=2 * L + 2) for L, _ in groups]
     g = shtk.UnevenBatch(cfgs3, nfs, precision="split", graph=True)
@@ -304,7 +322,8 @@ def measure_uneven(torch, np, shtk, dev, steps):
             "ms_per_batch_round_trip": round(ms, 4), "fp64_path_ms_per_batch_round_trip": round(fp64_ms, 4),
             "fp32_path_ms_per_batch_round_trip": round(fp32_ms, 4),
             "fp32_path_value": round(1000.0 * 64 / fp32_ms, 2),
-            "max_field_rel_l2_vs_fp64_path": err, "fp32_max_field_rel_l2_vs_fp64_path": err32,
+            "contraction": ran, "max_field_rel_l2_vs_fp64_path": err if ran != ["FP64"] else None,
+            "fp32_max_field_rel_l2_vs_fp64_path": err32,
             "autotuned": tune,
             "launches": "one hipGraph per direction; one configuration after the other"}
 
@@ -352,7 +371,8 @@ def measure_sphtor(torch, np, shtk, _lib, dev, steps, stream):
             "steps": steps, "ms_per_batch_round_trip": round(ms_split, 4),
             "fp64_path_value": round(1000.0 * nf / ms_plain, 2),
             "fp64_path_ms_per_batch_round_trip": round(ms_plain, 4),
-            "speedup_split_vs_fp64": round(ms_plain / ms_split, 3),
+            "contraction": {"split": contraction_of(k_split), "fp64": contraction_of(k_plain)},
+            "speedup_split_vs_fp64": round(ms_plain / ms_split, 3) if set(k_split) != set(k_plain) else None,
             "max_field_rel_l2_round_trip": {"split": err_split, "fp64": err_plain},
             "config": {"workload": "vector (sphtor) batch round trip, synthesis_sphtor_batch+analysis_sphtor_batch",
                        "lmax": lmax, "nlat": nlat, "nlon": nlon, "fields": nf,
@@ -533,8 +553,10 @@ def main() -> int:
             "ms_per_batch_round_trip": round(ms_batch, 5),
             "ms_per_batch_with_kernel_events": round(s_ev / ssteps, 5),
             "speedup_vs_plain": round((1000.0 * nf / ms_batch) / res["value"], 3),
-            "dtype": "split precision: int8 MFMA slices of FP64 Legendre values with FP64 sums (oz_*), FP64 field groups (leg_*)",
-            "max_field_rel_l2_vs_fp64_path": err_fp64,
+            "dtype": "split precision allowed: int8 MFMA slices of FP64 Legendre values with FP64 sums (oz_*), "
+                     "FP64 field groups where these are the faster (leg_*)",
+            "contraction": contraction_of(sk_us),
+            "max_field_rel_l2_vs_fp64_path": err_fp64 if contraction_of(sk_us) != ["FP64"] else None,
             "max_field_rel_l2_round_trip": err_in,
             "config": {"workload": "batched split-precision scalar round trip (synthesis_batch+analysis_batch)",
                        "lmax": LMAX, "nlat": NLAT, "nlon": NLON, "fields": nf},
@@ -589,7 +611,7 @@ def main() -> int:
         }
 
     if not args.no_split and not args.no_uneven:
-        res["uneven_batch"] = measure_uneven(torch, np, shtk, dev, max(3, args.steps // 10))
+        res["uneven_batch"] = measure_uneven(torch, np, shtk, _lib, dev, max(3, args.steps // 10))
 
     if not args.no_sphtor:
         res["sphtor_batch"] = measure_sphtor(torch, np, shtk, _lib, dev, max(4, args.steps // 5), stream)

@@ -54,7 +54,9 @@ enum shtk_dtype { SHTK_F64 = 0, SHTK_F32 = 1 };
 /* Contraction precision of the batched entry points (*_ex).  Where the FP64 field
  * groups are faster than a matrix-core contraction they run in its place, with
  * results at least as close (never for FP64 arrays in SHTK_PREC_FP32, whose values
- * stay those of the FP32 contraction).
+ * stay those of the FP32 contraction: these calls can take longer than in
+ * SHTK_PREC_FP64, which they are up to 1e7 times further from 64 bits than; FP32 arrays
+ * do not have that cost).
  * SHTK_PREC_FP64: the FP64 recurrence-and-contraction kernels (the plain path).
  * SHTK_PREC_SPLIT: FP64 Legendre values and tables, contraction as an Ozaki
  *   split on int8 matrix cores (6 slices, exact int32 accumulation, FP64

@@ -389,7 +389,8 @@ __device__ __forceinline__ void stockham_gen(double2 *z, int N, int Ns, int R, c
 //
 // The pass loops hide the thread's index from the optimiser: the addresses of every pass
 // depend on it and the length alone, and kept over the loop they filled the registers and
-// 340 to 600 bytes of scratch per thread.  Whole calls: 16 fields at lmax 700, nlon 1402
+// 340 to 600 bytes of scratch per thread (12 to 56 bytes are left in the prime kernels at
+// 128 registers, 0 in the others).  Whole calls: 16 fields at lmax 700, nlon 1402
 // (Bluestein): 895 -> 421 us; 8 at 1000, nlon 2002 = 2 * 7 * 11 * 13: 672 -> 359; 32 at
 // 303, nlon 608 = 32 * 19: 173 -> 82 (nlon 640: 75); one: 29 -> 19.
 template <int SIGN, int KIND>

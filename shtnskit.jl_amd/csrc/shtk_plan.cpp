@@ -1460,8 +1460,9 @@ int env_int(const char *name, int dflt) {
 
 // ---------------------------------------------------------------------------
 // Uneven batches: several configurations (one plan each), nf[g] fields per
-// configuration.  With SHTK_PREC_SPLIT every stage is one launch for all
-// groups (the Legendre contractions as persistent work-queue kernels); with
+// configuration, run one after the other, largest first.  A direction whose groups all
+// stay on the split contraction is one launch per stage instead (the Legendre
+// contractions as persistent work-queue kernels); with
 // graphs on, the whole launch sequence of a call is captured once per
 // (direction, arrays, dtype, stream) and replayed with one hipGraphLaunch.
 // ---------------------------------------------------------------------------
