@@ -69,6 +69,10 @@ def _adapt(x, adapt: bool, op: str):
     return x
 
 
+def _as(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    return t if t.dtype is dtype else t.to(dtype)
+
+
 def _colmajor(t: torch.Tensor) -> torch.Tensor:
     """Same logical tensor with Julia column-major memory (first index fastest)."""
     if t.is_conj() or t.is_neg():  # lazy views: the memory holds other values than the tensor
@@ -128,8 +132,7 @@ def _spec_in(cfg: SHTConfig, alm, adapt: bool, op: str, batch: bool):
     if batch and alm.shape[2] < 1:
         raise ValueError(f"{op} requires at least one field")
     rdt = _real_dtype(alm)
-    alm = _colmajor(alm.to(_cplx(rdt)))
-    return alm, rdt
+    return _colmajor(_as(alm, _cplx(rdt))), rdt
 
 
 def _grid_in(cfg: SHTConfig, f, adapt: bool, op: str, batch: bool, allow_complex: bool = False):
@@ -147,9 +150,8 @@ def _grid_in(cfg: SHTConfig, f, adapt: bool, op: str, batch: bool, allow_complex
     if f.is_complex():
         if not allow_complex:
             raise ValueError(f"{op}: the fields must be real-valued")
-        return _colmajor(f.to(_cplx(rdt))), rdt
-    f = _colmajor(f.to(rdt))
-    return f, rdt
+        return _colmajor(_as(f, _cplx(rdt))), rdt
+    return _colmajor(_as(f, rdt)), rdt
 
 
 def _nf(t: torch.Tensor, batch: bool) -> int:
