@@ -534,13 +534,13 @@ def main() -> int:
             sroof = roofline_entry(dom, sk_us[dom], ops, PEAK_INT8_TOPS, "TOP/s", "mfma",
                                    f"{ops:.4e} int8 ops = 21 slice products x 2 x (nlat/2)(lmax+1)(lmax+2)/2 "
                                    f"x 2 x {nf} fields")
-        elif dom.startswith("leg"):  # FP64 field groups; no committed traffic figure for a batch
+        elif dom.startswith("leg"):  # FP64 field groups
             # a recurrence step (4 flops) serves up to 8 fields, the contraction is 4 per field
             fl = 4.0 * n_triples(LMAX, NLAT) * (nf + (nf + 7) // 8)
             sroof = roofline_entry(dom, sk_us[dom], fl, PEAK_FP64_TFLOPS, "TFLOP/s", "mfma",
                                    f"{fl:.4e} flop = 4 x (nlat/2) x (lmax+1)(lmax+2)/2 x ({nf} fields + "
                                    f"{(nf + 7) // 8} recurrences) (FP64)")
-            sroof["traffic"] = None
+            sroof["traffic"] = measured_traffic(f"{dom}_{nf}")
         else:
             by = fft_bytes(NLAT, NLON, LMAX, nf)
             sroof = roofline_entry(dom, sk_us[dom], by * 1e3, PEAK_HBM_GBS, "GB/s", "hbm", f"{by:.4e} bytes")

@@ -49,10 +49,10 @@ __device__ __forceinline__ double mfac_of(int mode, int m) {
 // accumulators, so waves share nothing and there are no barriers; every
 // coefficient is stored once.
 //
-// Bound: FP64 issue (a matrix instruction holds the FP64 pipeline 64 cycles, 52 % of
-// the kernel's cycles at lmax 1023), then LDS (operand staging) at 2 waves per
-// SIMD.  16 fields at lmax 1023: 912 us (k_anal_w) -> 410 us; 37 fields at lmax 255: 85 -> 35 us; 16 at
-// 511: 175 -> 79 us.  Tried: the pairs of a 512-pair block dealt to 4 waves with
+// Bound: FP64 issue (a matrix instruction holds the FP64 pipeline 64 cycles, 48 % of
+// the kernel's cycles for 16 fields at lmax 1023, vector instructions 16 %), then LDS
+// (operand staging) at 2 waves per SIMD.  16 fields at lmax 1023: 918 us (k_anal_w) -> 425 us;
+// 37 fields at lmax 255: 86 -> 35 us; 16 at 511: 167 -> 81 us.  Tried, at 410 us: the pairs of a 512-pair block dealt to 4 waves with
 // field operands held over 8 segments and the partial sums of every 32 degrees
 // added through LDS (445 us: barriers), 16 fields per wave (478 us), operand
 // loads straight from the Fourier columns (434 us: four times the cache lines).
@@ -267,9 +267,9 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
 // NW waves per block take equal runs of the order's live segments, each from its own
 // seeds, and add their sums through LDS.
 //
-// Bound: FP64 issue (VALU 91 % of the busy cycles for 16 fields at lmax 1023, where
-// the chip runs at 2.0 GHz).  16 fields at lmax 1023: 815 us (k_synth_d) -> 435; 3
-// fields: 192 -> 105; 16 at 511: 124 -> 63; 37 at 255: 40 -> 29; 5 at 340: 30 -> 19.
+// Bound: FP64 issue (VALU 78 % of the cycles for 16 fields at lmax 1023, at 2.1 GHz).
+// 16 fields at lmax 1023: 735 us (k_synth_d) -> 379; 3 fields: 152 -> 98; 16 at 511:
+// 114 -> 61; 37 at 255: 40 -> 30; 5 at 340: 29 -> 17; 8 at 63: 5.7 -> 4.8.
 // ---------------------------------------------------------------------------
 template <int NG, typename CT = double2>
 struct SFRec {
