@@ -136,7 +136,9 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
     double nq0 = 0.0, nq1 = 0.0, nx = 0.0, nw = 0.0;
     int nk = 0;
     auto load = [&](int ch) {
-        const int p = max(pst + 64 * ch + lane, 0);
+        // lanes before the first live pair carry weight zero over that pair's values: what the
+        // field holds at rows that count for nothing (an infinity, a NaN) stays out of the sums
+        const int p0 = pst + 64 * ch + lane, p = max(p0, pfirst);
 #pragma unroll
         for (int f = 0; f < 8; ++f) {
             const double2 *Ff = Fn + min(f, nfl - 1) * fst;
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(64, 2) void k_anal_mx(const LegArgs a) {
         nx = a.x[p];
         nw = wlat ? wlat[p] : 1.0;
         if (2 * p == nlat - 1) nw *= 0.5;  // the equator's latitude is both halves of its pair
-        if (pst + 64 * ch + lane < 0) nw = 0.0;
+        if (p0 < pfirst) nw = 0.0;
     };
     // sums and differences of the hemispheres through the tile, as [16 columns][64 pairs] per
     // half: lane (column c = lane & 15, k = lane >> 4) reads pairs 8 t + 2 k + 0, 1 of column c
