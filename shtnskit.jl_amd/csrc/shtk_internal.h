@@ -55,7 +55,7 @@ constexpr int DSEG = 64;  // segment length of the register-record Legendre kern
 // Coefficient tables, one block per stored order (offset coff[im], entries
 // l = m .. lmax+1):
 //   qc[l] = (beta_l, c_l)                  scalar and vector recurrences
-//   qd[l] = (l c_l, g_l c_{l-1})           vector kernels of their own: s dP_l/dtheta = l x P_l - g_l P_{l-1},
+//   qd[l] = (l c_l, g_l c_{l-1})           vector (other segment lengths than DSEG): s dP_l/dtheta = l x P_l - g_l P_{l-1},
 //                                          g_l = sqrt((2l+1)(l^2-m^2)/(2l-1))
 constexpr int OZ_TPAD = 64;  // entries past the end of the padded per-degree tables
 

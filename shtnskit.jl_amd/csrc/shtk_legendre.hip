@@ -1174,19 +1174,20 @@ __device__ __forceinline__ void anal_vw_run(const LegArgs &a, const Item &it, do
     // per-degree records in VGPRs, broadcast by DPP (no scalar loads in the loop):
     // lane 16 r + n holds (beta_{l+1}, l c_l, g_l c_{l-1}) of degree l0 + c16 + n
     const double *qbv = a.qb + co;                       // padded past lmax + 1
-    const double2 *qdv = a.qd + co;                      // entries l = m .. lmax + 1
-    AVRec nr;
-    auto load_rec = [&](AVRec &d, int c16) {
-        const int l = min(it.l0 + c16 + (lane & 15), a.lmax + 1);
-        d.b = qbv[l + 1];
-        const double2 dd = qdv[l];
-        d.dl = dd.x;
-        d.dg = dd.y;
+    const double *qcv = a.qcc + co, *gv = a.gtab + co;   // entries l = m .. lmax + 1
+    double nb, nc, np1, ng;  // beta_{l+1}, c_l, c_{l-1} (1 before a segment's first degree), g_l
+    int nl;
+    auto load_rec = [&](int c16) {
+        nl = min(it.l0 + c16 + (lane & 15), a.lmax + 1);
+        nb = qbv[nl + 1];
+        nc = qcv[nl];
+        np1 = nl == it.l0 ? 1.0 : qcv[nl - 1];
+        ng = gv[nl];
     };
-    load_rec(nr, 0);
+    load_rec(0);
     for (int c16 = 0; c16 < nst; c16 += 16) {
-        const AVRec r = nr;
-        if (c16 + 16 < nst) load_rec(nr, c16 + 16);
+        const AVRec r = {nb, nl * nc, ng * np1};
+        if (c16 + 16 < nst) load_rec(c16 + 16);
         avw_pairs<K, FAST, 0>(a, it, r, qcm, red, cs, ct, lane, c16, nst, x, prev, cur, kk, gt, gp, gm, mm);
     }
 }

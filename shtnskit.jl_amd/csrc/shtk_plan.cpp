@@ -1931,7 +1931,7 @@ static int plan_tables(shtk_plan *p) {
             const double gl = (l > 0 && l > m)
                                   ? std::sqrt((2.0 * l + 1.0) * ((double)l * l - (double)m * m) / (2.0 * l - 1.0))
                                   : 0.0;
-            qd.push_back(make_double2((double)l * c, gl * cprev));
+            if (S != shtk::DSEG) qd.push_back(make_double2((double)l * c, gl * cprev));
             gt.push_back(gl);
         }
     }
